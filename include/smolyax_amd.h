@@ -389,6 +389,20 @@ int sbi_contract(const void* A, int64_t lda, const void* B, int64_t ldb, const d
                  double* Y, int64_t ldy, int64_t P, int64_t n, int64_t K, int32_t dtype,
                  void* stream);
 
+/* sbi_contract with FP64 operands and a workspace: when the P x n tiles are too few to fill the GPU,
+ * the k range is spread over extra workgroups that write their partial sums to `workspace`, and a
+ * second kernel adds them in sbi_contract's order (the same bits).  sbi_contract_f64_workspace sets
+ * *bytes to what it needs for a shape (0: not used); with less (or NULL) nothing is spread.
+ * The operands are copied 16 bytes at a time when both bases are 16-byte aligned, both row strides
+ * even, and each is at least its width rounded up to two: every row, the last one included, must
+ * then be readable up to that rounded width (the extra element is never used).  Other strides and
+ * bases take 8-byte loads.  workspace: device memory, 16-byte aligned, not shared with a concurrent
+ * call.  Replaces the same dense contraction as sbi_contract (barycentric.py:69-123). */
+int sbi_contract_f64_workspace(int64_t P, int64_t n, int64_t K, int64_t* bytes);
+int sbi_contract_f64_ws(const double* A, int64_t lda, const double* B, int64_t ldb,
+                        const double* offset, double* Y, int64_t ldy, int64_t P, int64_t n,
+                        int64_t K, void* workspace, int64_t ws_bytes, void* stream);
+
 /* Mixed contraction: Y = offset + A64^T B64 (K64 rows, FP64 MFMA) + A32^T B32 (K32 rows, FP32
  * MFMA, partial sums added into FP64 every 256 terms), with the same layouts as sbi_contract.
  * The few rows that carry most of the result (the constant and low-degree terms) go in the FP64

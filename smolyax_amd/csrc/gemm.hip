@@ -6,29 +6,32 @@
 // H^T or the barycentric entry weights W^T); B is the coefficient matrix (K x n, outputs
 // contiguous: Newton surpluses or zeta-scaled node values).  Y is FP64, row stride ldy.
 //
-// Work split: a workgroup of 4 waves owns a 64-point x (32*FN)-output tile of Y; each wave a
-// 32 x 16*FN sub-tile made of 2 x FN MFMA 16x16 fragments.  Every workgroup is independent (no
-// inter-workgroup waits, no atomics), so any number of these launches may run concurrently on
-// several streams, and each Y row is a function of its own column of A only, summed in a fixed
-// order: a point's result does not depend on P, on its position in the batch or on the batch's
-// other points (bit for bit).
+// Every workgroup is independent (no inter-workgroup waits, no atomics), so any number of these
+// launches may run concurrently on several streams, and each Y row is a function of its own column
+// of A only, summed in a fixed order: a point's result does not depend on P, on its position in
+// the batch or on the batch's other points (bit for bit).
+//
+// FP64 operands: contract_f64_kernel (operands staged in LDS).  FP32: contract_kernel below.
+//
+// contract_kernel, work split: a workgroup of 4 waves owns a 64-point x (32*FN)-output tile of Y;
+// each wave a 32 x 16*FN sub-tile made of 2 x FN MFMA 16x16 fragments.
 //
 // k order: MFMA 16x16x4 takes k = lane/16 from lane group g; within a 16-wide chunk of k, step s
 // of the four MFMAs takes k = k0 + 4g + s, so each lane walks four consecutive rows of A and B.
-// A and B are read with one dword (FP32) or qword (FP64) per lane; the 16 lanes of a group read
-// 16 consecutive points (outputs) of one row: 64- (128-) byte segments.  Edges are handled by
-// clamped loads (rows beyond P or n are computed and discarded) and, in the last chunk, by zeroing
-// terms with k >= K.
+// A and B are read with one dword per lane (plain layout); the 16 lanes of a group read 16
+// consecutive points (outputs) of one row: 64-byte segments.  Edges are handled by clamped loads
+// (rows beyond P or n are computed and discarded) and, in the last chunk, by zeroing terms with
+// k >= K.
 //
-// Accumulation: FP64 operands use the FP64 MFMA (v_mfma_f64_16x16x4), FP32 operands the FP32 MFMA
-// (v_mfma_f32_16x16x4); either way the MFMA accumulators hold partial sums of kFlushK terms of k
-// that are added into FP64 accumulators (in LDS).  FP32: the accumulation error stays that of a
-// 256-term sum and the result's error is dominated by the FP32 rounding of the operands.  FP64:
-// the rounding of a K-term sum grows with kFlushK + K / kFlushK instead of K.
+// Accumulation: the FP32 MFMA accumulators (v_mfma_f32_16x16x4) hold partial sums of kFlushK terms
+// of k that are added into FP64 accumulators (in LDS), so the accumulation error stays that of a
+// 256-term sum and the result's error is dominated by the FP32 rounding of the operands.
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/smolyax_amd.h"
 #include "common.h"
@@ -38,22 +41,12 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kWaves = 4;
 constexpr int kBlockM = 64;   // points per workgroup
 constexpr int kChunk = 16;    // k per main-loop iteration
 constexpr int kFlushK = 256;  // FP32 partial sums are flushed into FP64 every kFlushK terms
-
-template <typename T>
-struct Acc;
-template <>
-struct Acc<float> {
-  using type = v4f;
-};
-template <>
-struct Acc<double> {
-  using type = v4d;
-};
 
 __device__ __forceinline__ v4f mfma(float a, float b, v4f c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -104,14 +97,12 @@ __device__ __forceinline__ void head_fp64(const double* __restrict__ A64, int64_
 // contracted first with the FP64 MFMA, straight into the FP64 accumulators.  Lane li supplies the
 // A row of point 4*(li & 3) + (li >> 2) of its 16-point block, which puts the FP64 MFMA's result
 // (row g + 4r in register r of lane group g) into the FP32 layout (row 4g + r).
-template <typename T, int FN, bool kK4 = false>
+template <int FN, bool kK4 = false>
 __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
-    const T* __restrict__ A, int64_t lda, const T* __restrict__ B, int64_t ldb,
+    const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
     const double* __restrict__ offset, double* __restrict__ Y, int64_t ldy, int64_t P, int64_t n,
     int64_t K, const double* __restrict__ A64, int64_t lda64, const double* __restrict__ B64,
     int64_t ldb64, int64_t K64) {
-  using AccT = typename Acc<T>::type;
-  constexpr bool kF32 = sizeof(T) == 4;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave & 1, wn = wave >> 1;
@@ -125,10 +116,9 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
 #pragma unroll
   for (int fn = 0; fn < FN; ++fn) jcol[fn] = min(n_base + fn * 16 + li, n - 1);
 
-  AccT acc[2][FN];
-  // FP64 sums of the partial tiles of kFlushK terms (FP32 or FP64 MFMA accumulators): in LDS (one
-  // column per thread, no sharing), which keeps the register count low enough for two waves per
-  // SIMD.  Two levels keep the FP64 rounding of a long K at that of kFlushK + K / kFlushK terms.
+  v4f acc[2][FN];
+  // FP64 sums of the partial tiles of kFlushK terms: in LDS (one column per thread, no sharing),
+  // which keeps the register count low enough for two waves per SIMD.
   __shared__ double acc64s[2 * FN * 4][64 * kWaves];
   auto acc64 = [&](int fm, int fn, int r) -> double& {
     return acc64s[(fm * FN + fn) * 4 + r][threadIdx.x];
@@ -137,42 +127,39 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
   for (int fm = 0; fm < 2; ++fm)
 #pragma unroll
     for (int fn = 0; fn < FN; ++fn) {
-      acc[fm][fn] = AccT{0, 0, 0, 0};
+      acc[fm][fn] = v4f{0, 0, 0, 0};
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc64(fm, fn, r) = 0.0;
     }
 
-  if constexpr (kF32) {
-    if (K64 > 0) {
-      int64_t ph[2];
+  if (K64 > 0) {
+    int64_t ph[2];
 #pragma unroll
-      for (int fm = 0; fm < 2; ++fm)
-        ph[fm] = min(m_base + fm * 16 + 4 * (li & 3) + (li >> 2), P - 1);
-      v4d h[2][FN];
+    for (int fm = 0; fm < 2; ++fm)
+      ph[fm] = min(m_base + fm * 16 + 4 * (li & 3) + (li >> 2), P - 1);
+    v4d h[2][FN];
 #pragma unroll
-      for (int fm = 0; fm < 2; ++fm)
+    for (int fm = 0; fm < 2; ++fm)
 #pragma unroll
-        for (int fn = 0; fn < FN; ++fn) h[fm][fn] = v4d{0, 0, 0, 0};
-      head_fp64<2, FN>(A64, lda64, B64, ldb64, K64, g, ph, jcol, h);
+      for (int fn = 0; fn < FN; ++fn) h[fm][fn] = v4d{0, 0, 0, 0};
+    head_fp64<2, FN>(A64, lda64, B64, ldb64, K64, g, ph, jcol, h);
 #pragma unroll
-      for (int fm = 0; fm < 2; ++fm)
+    for (int fm = 0; fm < 2; ++fm)
 #pragma unroll
-        for (int fn = 0; fn < FN; ++fn)
+      for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc64(fm, fn, r) = h[fm][fn][r];
-    }
+        for (int r = 0; r < 4; ++r) acc64(fm, fn, r) = h[fm][fn][r];
   }
 
   const int64_t K16 = K & ~(int64_t)(kChunk - 1);
-  T a[2][4], b[FN][4];
-  typedef T v4t __attribute__((ext_vector_type(4)));
+  float a[2][4], b[FN][4];
   auto load = [&](int64_t k0) {
     if constexpr (kK4) {
       // k-interleaved operands: the four k of a lane's steps are one 16-byte vector
       const int64_t kq = (k0 >> 2) + g;
 #pragma unroll
       for (int fm = 0; fm < 2; ++fm) {
-        const v4t v = *reinterpret_cast<const v4t*>(A + (kq * lda + pcol[fm]) * 4);
+        const v4f v = *reinterpret_cast<const v4f*>(A + (kq * lda + pcol[fm]) * 4);
         a[fm][0] = v.x;
         a[fm][1] = v.y;
         a[fm][2] = v.z;
@@ -180,7 +167,7 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
       }
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn) {
-        const v4t v = *reinterpret_cast<const v4t*>(B + (kq * ldb + jcol[fn]) * 4);
+        const v4f v = *reinterpret_cast<const v4f*>(B + (kq * ldb + jcol[fn]) * 4);
         b[fn][0] = v.x;
         b[fn][1] = v.y;
         b[fn][2] = v.z;
@@ -190,8 +177,8 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int64_t k = k0 + 4 * g + s;
-        const T* __restrict__ ar = A + k * lda;
-        const T* __restrict__ br = B + k * ldb;
+        const float* __restrict__ ar = A + k * lda;
+        const float* __restrict__ br = B + k * ldb;
 #pragma unroll
         for (int fm = 0; fm < 2; ++fm) a[fm][s] = ar[pcol[fm]];
 #pragma unroll
@@ -214,12 +201,12 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
       for (int fn = 0; fn < FN; ++fn) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc64(fm, fn, r) += (double)acc[fm][fn][r];
-        acc[fm][fn] = AccT{0, 0, 0, 0};
+        acc[fm][fn] = v4f{0, 0, 0, 0};
       }
   };
 
   auto chunk = [&](int64_t k0) {
-    T ca[2][4], cb[FN][4];
+    float ca[2][4], cb[FN][4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
 #pragma unroll
@@ -237,11 +224,11 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
   };
   if (K16 > 0) {
     load(0);
-    if constexpr (kK4 || !kF32) {
+    if constexpr (kK4) {
       // the chunks of one kFlushK run form an inner loop with the flush after it, so the MFMA
       // accumulators stay in the matrix-core registers across the run (a flush test inside the
       // chunk loop made the compiler copy them to and from ordinary registers at every chunk:
-      // 4096 x 4096 outputs, K 10 016: FP64 7.42 -> 5.58 ms, FP32 k4 3.11 -> 2.90 ms).  The
+      // 4096 x 4096 outputs, K 10 016: 3.11 -> 2.90 ms).  The
       // plain FP32 layout keeps the flat loop (3.73 ms flat, 4.53 ms nested).  Same sums.
       for (int64_t kc = 0; kc < K16; kc += kFlushK) {
         const int64_t kce = min(K16, kc + (int64_t)kFlushK);
@@ -263,13 +250,13 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
       const int64_t kc = in ? k : K - 1;
 #pragma unroll
       for (int fm = 0; fm < 2; ++fm) {
-        const T v = A[kc * lda + pcol[fm]];
-        a[fm][s] = in ? v : T(0);
+        const float v = A[kc * lda + pcol[fm]];
+        a[fm][s] = in ? v : 0.0f;
       }
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn) {
-        const T v = B[kc * ldb + jcol[fn]];
-        b[fn][s] = in ? v : T(0);
+        const float v = B[kc * ldb + jcol[fn]];
+        b[fn][s] = in ? v : 0.0f;
       }
     }
     step();
@@ -285,9 +272,8 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
       const double off = offset ? offset[col] : 0.0;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        // result layout: FP32 16x16x4 holds row 4g + r in register r of lane group g, FP64
-        // 16x16x4 holds row g + 4r (column = lane % 16 in both)
-        const int64_t row = m_base + fm * 16 + (kF32 ? 4 * g + r : g + 4 * r);
+        // result layout: row 4g + r in register r of lane group g, column lane % 16
+        const int64_t row = m_base + fm * 16 + 4 * g + r;
         const double v = acc64(fm, fn, r);
         if (row < P) Y[row * ldy + col] = off + v;
       }
@@ -311,14 +297,12 @@ inline int64_t tile_n(int64_t P, int64_t n) {
 // contract_kernel adds into its FP64 sums at that flush) is written to `part`, the head to
 // `head`, and contract_reduce_kernel adds them in contract_kernel's order: the same bits.
 // ------------------------------------------------------------------------------------------
-template <typename T, int FN, bool kK4>
+template <int FN, bool kK4>
 __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
-    const T* __restrict__ A, int64_t lda, const T* __restrict__ B, int64_t ldb, int64_t P,
+    const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb, int64_t P,
     int64_t n, int64_t K, const double* __restrict__ A64, int64_t lda64,
     const double* __restrict__ B64, int64_t ldb64, int64_t K64, int64_t cps, int nsplit,
-    T* __restrict__ part, double* __restrict__ head) {
-  using AccT = typename Acc<T>::type;  // partial tiles are stored as T (the accumulator's type)
-  constexpr bool kF32 = sizeof(T) == 4;
+    float* __restrict__ part, double* __restrict__ head) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave & 1, wn = wave >> 1;
@@ -331,35 +315,33 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
   for (int fm = 0; fm < 2; ++fm) pcol[fm] = min(m_base + fm * 16 + li, P - 1);
 #pragma unroll
   for (int fn = 0; fn < FN; ++fn) jcol[fn] = min(n_base + fn * 16 + li, n - 1);
-  // element (fm, fn, r) of this lane: row and column of Y (FP32 layout for FP32 operands)
+  // element (fm, fn, r) of this lane: row and column of Y
   auto out_at = [&](int fm, int fn, int r, int64_t& row, int64_t& col) {
-    row = m_base + fm * 16 + (kF32 ? 4 * g + r : g + 4 * r);
+    row = m_base + fm * 16 + 4 * g + r;
     col = n_base + fn * 16 + li;
   };
 
-  if ((int)blockIdx.z == nsplit) {  // the FP64 head (FP32 operands only)
-    if constexpr (kF32) {
-      int64_t ph[2];
+  if ((int)blockIdx.z == nsplit) {  // the FP64 head
+    int64_t ph[2];
 #pragma unroll
-      for (int fm = 0; fm < 2; ++fm)
-        ph[fm] = min(m_base + fm * 16 + 4 * (li & 3) + (li >> 2), P - 1);
-      v4d h[2][FN];
+    for (int fm = 0; fm < 2; ++fm)
+      ph[fm] = min(m_base + fm * 16 + 4 * (li & 3) + (li >> 2), P - 1);
+    v4d h[2][FN];
 #pragma unroll
-      for (int fm = 0; fm < 2; ++fm)
+    for (int fm = 0; fm < 2; ++fm)
 #pragma unroll
-        for (int fn = 0; fn < FN; ++fn) h[fm][fn] = v4d{0, 0, 0, 0};
-      head_fp64<2, FN>(A64, lda64, B64, ldb64, K64, g, ph, jcol, h);
+      for (int fn = 0; fn < FN; ++fn) h[fm][fn] = v4d{0, 0, 0, 0};
+    head_fp64<2, FN>(A64, lda64, B64, ldb64, K64, g, ph, jcol, h);
 #pragma unroll
-      for (int fm = 0; fm < 2; ++fm)
+    for (int fm = 0; fm < 2; ++fm)
 #pragma unroll
-        for (int fn = 0; fn < FN; ++fn)
+      for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            int64_t row, col;
-            out_at(fm, fn, r, row, col);
-            if (row < P && col < n) head[row * n + col] = h[fm][fn][r];
-          }
-    }
+        for (int r = 0; r < 4; ++r) {
+          int64_t row, col;
+          out_at(fm, fn, r, row, col);
+          if (row < P && col < n) head[row * n + col] = h[fm][fn][r];
+        }
     return;
   }
 
@@ -367,11 +349,11 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
   const int64_t c0 = (int64_t)blockIdx.z * cps, c1 = min(nch, c0 + cps);
   if (c0 >= c1) return;
   const int64_t K16 = K & ~(int64_t)(kChunk - 1);
-  AccT acc[2][FN];
+  v4f acc[2][FN];
 #pragma unroll
   for (int fm = 0; fm < 2; ++fm)
 #pragma unroll
-    for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = AccT{0, 0, 0, 0};
+    for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = v4f{0, 0, 0, 0};
   int64_t cur = c0;  // chunk whose partial tile is accumulating
   auto emit = [&]() {
 #pragma unroll
@@ -384,19 +366,18 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
           out_at(fm, fn, r, row, col);
           if (row < P && col < n) part[cur * Pn + row * n + col] = acc[fm][fn][r];
         }
-        acc[fm][fn] = AccT{0, 0, 0, 0};
+        acc[fm][fn] = v4f{0, 0, 0, 0};
       }
     ++cur;
   };
 
-  T a[2][4], b[FN][4];
-  typedef T v4t __attribute__((ext_vector_type(4)));
+  float a[2][4], b[FN][4];
   auto load = [&](int64_t k0) {
     if constexpr (kK4) {
       const int64_t kq = (k0 >> 2) + g;
 #pragma unroll
       for (int fm = 0; fm < 2; ++fm) {
-        const v4t v = *reinterpret_cast<const v4t*>(A + (kq * lda + pcol[fm]) * 4);
+        const v4f v = *reinterpret_cast<const v4f*>(A + (kq * lda + pcol[fm]) * 4);
         a[fm][0] = v.x;
         a[fm][1] = v.y;
         a[fm][2] = v.z;
@@ -404,7 +385,7 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
       }
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn) {
-        const v4t v = *reinterpret_cast<const v4t*>(B + (kq * ldb + jcol[fn]) * 4);
+        const v4f v = *reinterpret_cast<const v4f*>(B + (kq * ldb + jcol[fn]) * 4);
         b[fn][0] = v.x;
         b[fn][1] = v.y;
         b[fn][2] = v.z;
@@ -414,8 +395,8 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int64_t k = k0 + 4 * g + s;
-        const T* __restrict__ ar = A + k * lda;
-        const T* __restrict__ br = B + k * ldb;
+        const float* __restrict__ ar = A + k * lda;
+        const float* __restrict__ br = B + k * ldb;
 #pragma unroll
         for (int fm = 0; fm < 2; ++fm) a[fm][s] = ar[pcol[fm]];
 #pragma unroll
@@ -431,7 +412,7 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
     for (int64_t kc = kb; kc < ke; kc += kFlushK) {
       const int64_t kce = min(ke, kc + (int64_t)kFlushK);
       for (int64_t k0 = kc; k0 < kce; k0 += kChunk) {
-        T ca[2][4], cb[FN][4];
+        float ca[2][4], cb[FN][4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
 #pragma unroll
@@ -459,13 +440,13 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
       const int64_t kc = in ? k : K - 1;
 #pragma unroll
       for (int fm = 0; fm < 2; ++fm) {
-        const T v = A[kc * lda + pcol[fm]];
-        a[fm][s] = in ? v : T(0);
+        const float v = A[kc * lda + pcol[fm]];
+        a[fm][s] = in ? v : 0.0f;
       }
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn) {
-        const T v = B[kc * ldb + jcol[fn]];
-        b[fn][s] = in ? v : T(0);
+        const float v = B[kc * ldb + jcol[fn]];
+        b[fn][s] = in ? v : 0.0f;
       }
     }
 #pragma unroll
@@ -482,7 +463,7 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
 // kFlushK: contract_kernel's final flush then adds an empty partial tile), head = 0 without one.
 template <typename E>
 __global__ __launch_bounds__(256) void contract_reduce_kernel(const E* __restrict__ part,
-                                                              int64_t nch,
+                                                              int64_t nch, int64_t per,
                                                               const double* __restrict__ head,
                                                               const double* __restrict__ offset,
                                                               double* __restrict__ Y, int64_t ldy,
@@ -492,7 +473,17 @@ __global__ __launch_bounds__(256) void contract_reduce_kernel(const E* __restric
        i += (int64_t)gridDim.x * 256) {
     const int64_t row = i / n, col = i - row * n;
     double v = head ? head[i] : 0.0;
-    for (int64_t c = 0; c < nch; ++c) v += (double)part[c * Pn + i];
+    if (per == 1) {
+#pragma unroll 4
+      for (int64_t c = 0; c < nch; ++c) v += (double)part[c * Pn + i];
+    } else {  // FP64 chains: slice sums of `per` chains first
+      for (int64_t c = 0; c < nch; c += per) {
+        double s = 0.0;
+#pragma unroll 8
+        for (int64_t u = c; u < min(nch, c + per); ++u) s += (double)part[u * Pn + i];
+        v += s;
+      }
+    }
     if (K % kFlushK == 0) v += 0.0;
     const double off = offset ? offset[col] : 0.0;
     Y[row * ldy + col] = off + v;
@@ -504,11 +495,11 @@ __global__ __launch_bounds__(256) void contract_reduce_kernel(const E* __restric
 // kSplitTarget workgroups run (small batches: the k loop of one workgroup is the latency).
 constexpr int64_t kSplitMinGroups = 256;
 constexpr int64_t kSplitTarget = 512;
+constexpr int64_t kF64SplitGroups = 768;            // FP64: three 4-wave workgroups per CU
 constexpr int64_t kSplitMaxBytes = int64_t(256) << 20;  // workspace of one split call
 struct SplitPlan {
   int64_t nsplit = 0, cps = 0, nch = 0, part_bytes = 0, head_bytes = 0;
 };
-template <typename T>
 SplitPlan split_plan(int64_t P, int64_t n, int64_t K, int64_t K64) {
   SplitPlan sp;
   const int64_t gm = (P + kBlockM - 1) / kBlockM;
@@ -525,20 +516,18 @@ SplitPlan split_plan(int64_t P, int64_t n, int64_t K, int64_t K64) {
     sp = SplitPlan{};
     return sp;
   }
-  sp.part_bytes = ((sp.nch * P * n * (int64_t)sizeof(T)) + 255) /
-                  256 * 256;
+  sp.part_bytes = (sp.nch * P * n * (int64_t)sizeof(float) + 255) / 256 * 256;
   sp.head_bytes = K64 > 0 ? P * n * 8 : 0;
   if (sp.part_bytes + sp.head_bytes > kSplitMaxBytes || sp.nsplit >= 65535) sp = SplitPlan{};
   return sp;
 }
 
-template <typename T, bool kK4>
-int contract_split_launch(const SplitPlan& sp, const T* A, int64_t lda, const T* B, int64_t ldb,
+template <bool kK4>
+int contract_split_launch(const SplitPlan& sp, const float* A, int64_t lda, const float* B, int64_t ldb,
                           const double* offset, double* Y, int64_t ldy, int64_t P, int64_t n,
                           int64_t K, const double* A64, int64_t lda64, const double* B64,
                           int64_t ldb64, int64_t K64, void* ws, hipStream_t st) {
-  using E = T;
-  E* part = (E*)ws;
+  float* part = (float*)ws;
   double* head = K64 > 0 ? (double*)((char*)ws + sp.part_bytes) : nullptr;
   const dim3 block(64 * kWaves);
   const unsigned gm = (unsigned)((P + kBlockM - 1) / kBlockM);
@@ -546,15 +535,15 @@ int contract_split_launch(const SplitPlan& sp, const T* A, int64_t lda, const T*
   const int ns = (int)sp.nsplit;
   const int64_t tn = tile_n(P, n);
   if (tn == 32) {
-    hipLaunchKernelGGL((contract_split_kernel<T, 1, kK4>), dim3(gm, (unsigned)((n + 31) / 32), gz),
+    hipLaunchKernelGGL((contract_split_kernel<1, kK4>), dim3(gm, (unsigned)((n + 31) / 32), gz),
                        block, 0, st, A, lda, B, ldb, P, n, K, A64, lda64, B64, ldb64, K64, sp.cps,
                        ns, part, head);
   } else if (tn == 64) {
-    hipLaunchKernelGGL((contract_split_kernel<T, 2, kK4>), dim3(gm, (unsigned)((n + 63) / 64), gz),
+    hipLaunchKernelGGL((contract_split_kernel<2, kK4>), dim3(gm, (unsigned)((n + 63) / 64), gz),
                        block, 0, st, A, lda, B, ldb, P, n, K, A64, lda64, B64, ldb64, K64, sp.cps,
                        ns, part, head);
   } else {
-    hipLaunchKernelGGL((contract_split_kernel<T, 4, kK4>),
+    hipLaunchKernelGGL((contract_split_kernel<4, kK4>),
                        dim3(gm, (unsigned)((n + 127) / 128), gz), block, 0, st, A, lda, B, ldb, P,
                        n, K, A64, lda64, B64, ldb64, K64, sp.cps, ns, part, head);
   }
@@ -562,27 +551,324 @@ int contract_split_launch(const SplitPlan& sp, const T* A, int64_t lda, const T*
   const int64_t Pn = P * n;
   int64_t rg = (Pn + 255) / 256;
   if (rg > 4096) rg = 4096;
-  hipLaunchKernelGGL((contract_reduce_kernel<E>), dim3((unsigned)rg), dim3(256), 0, st, part,
-                     sp.nch, head, offset, Y, ldy, P, n, K);
+  hipLaunchKernelGGL((contract_reduce_kernel<float>), dim3((unsigned)rg), dim3(256), 0, st, part,
+                     sp.nch, int64_t(1), head, offset, Y, ldy, P, n, K);
   SBI_HIP_CHECK(hipGetLastError());
   return SBI_OK;
 }
 
-template <typename T, bool kK4 = false>
-int contract_launch(const T* A, int64_t lda, const T* B, int64_t ldb, const double* offset,
+// ------------------------------------------------------------------------------------------
+// FP64 contraction.  Bound: v_mfma_f64_16x16x4, 64 cycles of a SIMD per 2048 operations (measured
+// ceiling of a large library product on this card: 72 TFLOP/s).  The operands need only 16 bytes
+// per cycle and CU, so what matters is that several waves per SIMD always have their fragments at
+// hand: operands are staged in LDS, three buffers of 16 k, copied two chunks ahead by direct
+// global -> LDS loads (one barrier per chunk), and the register count allows three waves per SIMD.
+// 8192 points x 256 outputs, K 5000: 367 us (57 TFLOP/s) against 402-412 us with each wave loading
+// its own fragments from L2 one chunk ahead; 5000 x 160, K 10 002 (k over workgroups): 478 -> 345-390 us;
+// 5000 x 8192, K 256: 487 -> 390 us; 4096 x 4096, K 9986: 5590 -> 5500 us.  Requesting a whole
+// chunk's fragments before its first MFMA costs a wave per SIMD's worth of registers (5730 us).
+//
+// Work split: a workgroup of 4 waves owns a (32 * WM)-point x (32 * WN)-output tile, each wave 16 * WM
+// points x 16 * WN outputs; the last output tile with at most 32 outputs left is cut into four waves of
+// 16 points x 32 outputs instead, so that no wave works on outputs past the edge (160 outputs:
+// 17 % less matrix work).  WN = 1 for at most 32 outputs; WM = 1 (32 points) where k is not spread
+// and 64-point tiles would be fewer than one per CU (500 x 64, K 9986, no workspace: 472 -> 342
+// us).  The output tiles of one point tile run
+// on one XCD (its L2 serves their A rows).
+//
+// LDS image of a chunk: rows of the tile's width; the 16-byte slot q of row r holds the elements
+// of slot q ^ (8 * (r & 1)), so the two rows that half a wave reads together lie in different
+// halves of the banks.  kDirect = false: row strides, widths or bases that are not multiples of
+// 16 bytes go through registers (8-byte loads one chunk ahead); the same image, the same bits.
+//
+// Sums: the MFMA accumulators hold a chain of kFlushK terms, the chains are added into a slice sum
+// of kF64Slice terms, the slice sums in order, so the rounding grows with kFlushK + kF64Slice /
+// kFlushK + K / kF64Slice terms.  Small grids spread k over workgroups (nz > 1) in units of a
+// slice, very small ones in units of a chain; each writes the sums of its units to `part` and
+// contract_reduce_kernel adds them in the same order: the same bits for any P, alone or in a batch.
+// ------------------------------------------------------------------------------------------
+constexpr int kF64Slice = 2048;
+constexpr int kF64Buf = 3;
+enum { kWhole = 0, kBySlice = 1, kByChain = 2 };  // how k is spread over workgroups (kSplit)
+
+template <int WM, int WN, bool kDirect, int kSplit>
+__global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64_kernel(
+    const double* __restrict__ A, int64_t lda, const double* __restrict__ B, int64_t ldb,
+    const double* __restrict__ offset, double* __restrict__ Y, int64_t ldy, int64_t P, int64_t n,
+    int64_t K, int ntm, int ntn, int nz, int64_t kpz, double* __restrict__ part) {
+  constexpr int TM = 32 * WM, TN = 32 * WN;
+  constexpr int kA = kChunk * TM * 8, kStep = kA + kChunk * TN * 8;  // bytes of a chunk: A, then B
+  constexpr int nA = kA / 1024, kPer = kStep / 4096;                 // 1 KB copies: of A, per wave
+  static_assert(kStep % 4096 == 0, "whole copies per wave");
+  __shared__ __attribute__((aligned(16))) char smem[kF64Buf * kStep];
+  const int L = blockIdx.x;
+  const int idx = L >> 3;
+  const int tn = idx % ntn;
+  const int pair = (idx / ntn) * 8 + (L & 7);
+  if (pair >= ntm * nz) return;
+  const int tm = pair % ntm, z = pair / ntm;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, g = lane >> 4;
+  const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
+  const bool thin = WM == 2 && WN == 2 && n - n0 <= 32;  // 4 x 1 waves of 16 x 32 instead of 2 x 2 of 32 x 32
+  const int mw = thin ? wave * 16 : (wave & 1) * (16 * WM);
+  const int nw = thin ? 0 : (wave >> 1) * (16 * WN);
+  const int64_t kb = (int64_t)z * kpz;  // kpz: k per workgroup, whole units
+  const int64_t ke = kSplit ? min(K, kb + kpz) : K;
+
+  // copy i of this wave: 128 consecutive elements of the LDS image, two per lane (columns past
+  // the edge re-read the last pair or element, rows past K row K - 1: never used)
+  const double* src[kPer];  // this lane's pair in the next chunk
+  auto krow = [&](int i) {
+    const int c = wave + 4 * i;
+    return c < nA ? (c * 128 + lane * 2) / TM : ((c - nA) * 128 + lane * 2) / TN;
+  };
+  uint32_t odd = 0;  // bit i: the pair's second element is past the edge (kDirect = false)
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int c = wave + 4 * i;
+    const bool isA = c < nA;
+    const int T = isA ? TM : TN;
+    const int pos = (isA ? c : c - nA) * 128 + lane * 2;
+    const int64_t col = (((pos % T) / 2) ^ (8 * (krow(i) & 1))) * 2;
+    const int64_t at = (isA ? m0 : n0) + col, end = isA ? P : n;
+    const int64_t ld = isA ? lda : ldb;
+    const double* base = (isA ? A : B) + min(at, kDirect ? (end - 1) & ~(int64_t)1 : end - 1);
+    if (!kDirect && at + 1 >= end) odd |= 1u << i;
+    src[i] = base + (kb + krow(i)) * ld;
+  }
+  int64_t ki = kb;  // first row of the next chunk to be copied
+  double pend[kDirect ? 1 : 2 * kPer];
+  auto advance = [&](auto&& put) {
+    if (ki + kChunk <= K) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        put(i, src[i]);
+        src[i] += kChunk * (wave + 4 * i < nA ? lda : ldb);
+      }
+    } else {  // the last chunk of K
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        put(i, src[i] - max((int64_t)0, ki + krow(i) - (K - 1)) * (wave + 4 * i < nA ? lda : ldb));
+    }
+    ki += kChunk;
+  };
+  auto fetch = [&] {  // kDirect = false: the next chunk into registers
+    if (ki < ke)
+      advance([&](int i, const double* p) {
+        pend[2 * i] = p[0];
+        pend[2 * i + 1] = p[(odd >> i) & 1 ? 0 : 1];
+      });
+  };
+  auto issue = [&](int b) {  // the next chunk into buffer b
+    char* dst = smem + b * kStep + wave * 1024;
+    if constexpr (kDirect) {
+      if (ki < ke)
+        advance([&](int i, const double* p) {
+          __builtin_amdgcn_global_load_lds((const void*)p, (lds_void*)(dst + i * 4096), 16, 0, 0);
+        });
+    } else {
+      typedef double v2d __attribute__((ext_vector_type(2)));
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        *(v2d*)(dst + i * 4096 + lane * 16) = v2d{pend[2 * i], pend[2 * i + 1]};
+      fetch();
+    }
+  };
+  // the chunk at k0 has landed in every wave (the copies of the next one may be in flight)
+  auto wait = [&](int64_t k0) {
+    if constexpr (kDirect) {
+      if (k0 + kChunk < ke) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_barrier" ::: "memory");
+    } else {
+      __syncthreads();
+    }
+  };
+
+  v4d total[WM][WN], sum[WM][WN], acc[WM][WN];
+  auto each = [&](auto&& f) {  // the fragments of this wave
+#pragma unroll
+    for (int fm = 0; fm < WM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < WN; ++fn) f(fm, fn);
+  };
+  each([&](int fm, int fn) { total[fm][fn] = v4d{0, 0, 0, 0}; });
+
+  int bi = 0;  // buffer of the chunk being computed
+  const int sw = 16 * (g & 1);
+  auto compute = [&](int64_t k0, bool tail) {
+    const double* la = (const double*)(smem + bi * kStep);
+    const double* lb = (const double*)(smem + bi * kStep + kA);
+#pragma unroll
+    for (int s = 0; s < kChunk / 4; ++s) {
+      double a[WM], b[WN];
+      const int r = 4 * s + g;
+#pragma unroll
+      for (int fm = 0; fm < WM; ++fm) a[fm] = la[r * TM + ((mw + fm * 16 + li) ^ sw)];
+#pragma unroll
+      for (int fn = 0; fn < WN; ++fn) b[fn] = lb[r * TN + ((nw + fn * 16 + li) ^ sw)];
+      if (tail && k0 + r >= K) {
+#pragma unroll
+        for (int fm = 0; fm < WM; ++fm) a[fm] = 0.0;
+#pragma unroll
+        for (int fn = 0; fn < WN; ++fn) b[fn] = 0.0;
+      }
+#pragma unroll
+      for (int fm = 0; fm < WM; ++fm) {
+        if (fm && thin) break;
+#pragma unroll
+        for (int fn = 0; fn < WN; ++fn) acc[fm][fn] = mfma(a[fm], b[fn], acc[fm][fn]);
+      }
+    }
+  };
+  auto chain = [&](int64_t kc, int64_t kce) {  // acc += rows [kc, kce)
+    const int64_t kf = kc + ((kce - kc) & ~(int64_t)(kChunk - 1));
+    for (int64_t k0 = kc; k0 < kf; k0 += kChunk) {
+      wait(k0);
+      issue(kDirect ? (bi == 0 ? kF64Buf - 1 : bi - 1) : (bi + 1 == kF64Buf ? 0 : bi + 1));
+      compute(k0, false);
+      bi = bi + 1 == kF64Buf ? 0 : bi + 1;
+    }
+    if (kf < kce) {
+      wait(kf);
+      compute(kf, true);
+    }
+  };
+  if (kb < ke) {
+    if constexpr (kDirect) {
+      issue(0);
+      issue(1);
+    } else {
+      fetch();
+      issue(0);
+    }
+  }
+  auto row_of = [&](int fm, int r) { return m0 + mw + fm * 16 + g + 4 * r; };
+  auto col_of = [&](int fn) { return n0 + nw + fn * 16 + li; };
+  auto emit = [&](int64_t unit, v4d(&v)[WM][WN]) {
+    double* __restrict__ out = part + unit * P * n;
+    each([&](int fm, int fn) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t row = row_of(fm, r), col = col_of(fn);
+        if (row < P && col < n && !(thin && fm)) out[row * n + col] = v[fm][fn][r];
+      }
+    });
+  };
+  for (int64_t ks = kb; ks < ke; ks += kF64Slice) {
+    const int64_t kse = min(ke, ks + (int64_t)kF64Slice);
+    each([&](int fm, int fn) { sum[fm][fn] = v4d{0, 0, 0, 0}; });
+    for (int64_t kc = ks; kc < kse; kc += kFlushK) {
+      each([&](int fm, int fn) { acc[fm][fn] = v4d{0, 0, 0, 0}; });
+      chain(kc, min(kse, kc + (int64_t)kFlushK));
+      if constexpr (kSplit == kByChain) emit(kc / kFlushK, acc);
+      else each([&](int fm, int fn) { sum[fm][fn] += acc[fm][fn]; });
+    }
+    if constexpr (kSplit == kWhole) each([&](int fm, int fn) { total[fm][fn] += sum[fm][fn]; });
+    else if constexpr (kSplit == kBySlice) emit(ks / kF64Slice, sum);
+  }
+  if constexpr (kSplit != kWhole) return;
+  each([&](int fm, int fn) {
+    const int64_t col = col_of(fn);
+    const double off = offset ? offset[min(col, n - 1)] : 0.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t row = row_of(fm, r);
+      if (row < P && col < n && !(thin && fm)) Y[row * ldy + col] = off + total[fm][fn][r];
+    }
+  });
+}
+
+// How contract_f64_kernel spreads k over workgroups (nz = 1: not at all, no workspace): when the
+// tiles alone are fewer than kF64SplitGroups, in units of a slice if that gives enough
+// workgroups (little workspace traffic: 5000 x 160 outputs, K 10 002, 480 -> 345-390 us), else in
+// units of a chain (500 x 64, K 9986: 472 us unsplit, 104 us by slices, 31 us by chains).
+struct F64Plan {
+  int64_t nz = 1, kpz = 0, units = 0, bytes = 0;
+  int split = kWhole;
+};
+inline int64_t f64_tile_n(int64_t n) { return n <= 32 ? 32 : 64; }
+F64Plan f64_plan(int64_t P, int64_t n, int64_t K) {
+  F64Plan pl;
+  if (P <= 0 || n <= 0) return pl;
+  const int64_t groups = ((P + kBlockM - 1) / kBlockM) * ((n + f64_tile_n(n) - 1) / f64_tile_n(n));
+  const int64_t want = (kF64SplitGroups + groups - 1) / groups;
+  const bool fine = want > (K + kF64Slice - 1) / kF64Slice;
+  const int64_t unit = fine ? kFlushK : kF64Slice;
+  const int64_t units = (K + unit - 1) / unit;
+  if (want < 2 || units < 2) return pl;
+  const int64_t upz = (units + want - 1) / want, nz = (units + upz - 1) / upz;
+  const int64_t bytes = units * P * n * 8;
+  if (nz < 2 || bytes > kSplitMaxBytes) return pl;
+  pl.nz = nz;
+  pl.kpz = upz * unit;
+  pl.units = units;
+  pl.bytes = bytes;
+  pl.split = fine ? kByChain : kBySlice;
+  return pl;
+}
+
+typedef void (*f64_kernel_t)(const double*, int64_t, const double*, int64_t, const double*, double*,
+                             int64_t, int64_t, int64_t, int64_t, int, int, int, int64_t, double*);
+template <int WN, bool kDirect>
+f64_kernel_t f64_kernel(int wm, int split) {
+  if (split == kBySlice) return contract_f64_kernel<2, WN, kDirect, kBySlice>;
+  if (split == kByChain) return contract_f64_kernel<2, WN, kDirect, kByChain>;
+  return wm == 1 ? contract_f64_kernel<1, WN, kDirect, kWhole>
+                 : contract_f64_kernel<2, WN, kDirect, kWhole>;
+}
+
+// padded: every row of A (B) is readable up to P (n) rounded up to a multiple of two.
+int contract_f64(const double* A, int64_t lda, const double* B, int64_t ldb, const double* offset,
+                 double* Y, int64_t ldy, int64_t P, int64_t n, int64_t K, bool padded, void* ws,
+                 int64_t ws_bytes, hipStream_t st) {
+  F64Plan pl = f64_plan(P, n, K);
+  if (!ws || ws_bytes < pl.bytes) pl = F64Plan{};
+  const bool direct = K == 0 || (((uintptr_t)A | (uintptr_t)B) % 16 == 0 && lda % 2 == 0 &&
+                                 ldb % 2 == 0 && (padded || (P % 2 == 0 && n % 2 == 0)));
+  const int64_t tn = f64_tile_n(n), ntn = (n + tn - 1) / tn;
+  const int wm = pl.nz == 1 && (P + 63) / 64 * ntn < 192 ? 1 : 2;
+  const int64_t ntm = (P + 32 * wm - 1) / (32 * wm);
+  const int64_t grid = ((ntm * pl.nz + 7) / 8) * 8 * ntn;
+  if (grid > 0x7fffffff) {
+    sbi::set_error("sbi_contract: launch too large");
+    return SBI_ERR_INVALID;
+  }
+  const f64_kernel_t kernel = tn == 32 ? (direct ? f64_kernel<1, true>(wm, pl.split)
+                                                 : f64_kernel<1, false>(wm, pl.split))
+                                       : (direct ? f64_kernel<2, true>(wm, pl.split)
+                                                 : f64_kernel<2, false>(wm, pl.split));
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * kWaves), 0, st, A, lda, B, ldb, offset,
+                     Y, ldy, P, n, K, (int)ntm, (int)ntn, (int)pl.nz, pl.kpz, (double*)ws);
+  SBI_HIP_CHECK(hipGetLastError());
+  if (pl.nz > 1) {
+    const int64_t rg = std::min<int64_t>((P * n + 255) / 256, 4096);
+    const int64_t per = pl.split == kByChain ? kF64Slice / kFlushK : 1;
+    hipLaunchKernelGGL((contract_reduce_kernel<double>), dim3((unsigned)rg), dim3(256), 0, st,
+                       (const double*)ws, pl.units, per, nullptr, offset, Y, ldy, P, n, K);
+    SBI_HIP_CHECK(hipGetLastError());
+  }
+  return SBI_OK;
+}
+
+template <bool kK4 = false>
+int contract_launch(const float* A, int64_t lda, const float* B, int64_t ldb, const double* offset,
                     double* Y, int64_t ldy, int64_t P, int64_t n, int64_t K, const double* A64,
                     int64_t lda64, const double* B64, int64_t ldb64, int64_t K64, hipStream_t st) {
   const dim3 block(64 * kWaves);
   const unsigned gm = (unsigned)((P + kBlockM - 1) / kBlockM);
   const int64_t tn = tile_n(P, n);
   if (tn == 32) {
-    hipLaunchKernelGGL((contract_kernel<T, 1, kK4>), dim3(gm, (unsigned)((n + 31) / 32)), block, 0, st,
+    hipLaunchKernelGGL((contract_kernel<1, kK4>), dim3(gm, (unsigned)((n + 31) / 32)), block, 0, st,
                        A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64);
   } else if (tn == 64) {
-    hipLaunchKernelGGL((contract_kernel<T, 2, kK4>), dim3(gm, (unsigned)((n + 63) / 64)), block, 0, st,
+    hipLaunchKernelGGL((contract_kernel<2, kK4>), dim3(gm, (unsigned)((n + 63) / 64)), block, 0, st,
                        A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64);
   } else {
-    hipLaunchKernelGGL((contract_kernel<T, 4, kK4>), dim3(gm, (unsigned)((n + 127) / 128)), block, 0,
+    hipLaunchKernelGGL((contract_kernel<4, kK4>), dim3(gm, (unsigned)((n + 127) / 128)), block, 0,
                        st, A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64);
   }
   SBI_HIP_CHECK(hipGetLastError());
@@ -614,7 +900,6 @@ int contract_launch(const T* A, int64_t lda, const T* B, int64_t ldb, const doub
 // ------------------------------------------------------------------------------------------
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) v8bf lds_v8bf;
-typedef __attribute__((address_space(3))) void lds_void;
 constexpr int kBfFlush = 1024;  // k per FP32 partial sum
 constexpr int kBfBuf = 4;       // LDS buffers of one 32-k step each
 
@@ -986,13 +1271,38 @@ extern "C" int sbi_contract(const void* A, int64_t lda, const void* B, int64_t l
   if (P == 0 || n == 0) return SBI_OK;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == 0)
-    return contract_launch<double>((const double*)A, lda, (const double*)B, ldb, offset, Y, ldy,
-                                   P, n, K, nullptr, 0, nullptr, 0, 0, st);
+    return contract_f64((const double*)A, lda, (const double*)B, ldb, offset, Y, ldy, P, n, K,
+                        false, nullptr, 0, st);
   if (dtype == 1)
-    return contract_launch<float>((const float*)A, lda, (const float*)B, ldb, offset, Y, ldy, P,
+    return contract_launch<false>((const float*)A, lda, (const float*)B, ldb, offset, Y, ldy, P,
                                   n, K, nullptr, 0, nullptr, 0, 0, st);
   sbi::set_error("sbi_contract: dtype must be 0 (f64) or 1 (f32)");
   return SBI_ERR_INVALID;
+}
+
+extern "C" int sbi_contract_f64_workspace(int64_t P, int64_t n, int64_t K, int64_t* bytes) {
+  if (P < 0 || n < 0 || K < 0 || !bytes) {
+    sbi::set_error("sbi_contract_f64_workspace: invalid argument");
+    return SBI_ERR_INVALID;
+  }
+  *bytes = f64_plan(P, n, K).bytes;
+  return SBI_OK;
+}
+
+extern "C" int sbi_contract_f64_ws(const double* A, int64_t lda, const double* B, int64_t ldb,
+                                   const double* offset, double* Y, int64_t ldy, int64_t P,
+                                   int64_t n, int64_t K, void* workspace, int64_t ws_bytes,
+                                   void* stream) {
+  if (P < 0 || n < 0 || K < 0 || ws_bytes < 0 || (P > 0 && n > 0 && (!Y || ldy < n)) ||
+      (P > 0 && n > 0 && K > 0 && (!A || !B || lda < P || ldb < n)) ||
+      ((uintptr_t)workspace & 15) || P > (int64_t)65535 * kBlockM || n > (int64_t)65535 * 32) {
+    sbi::set_error("sbi_contract_f64_ws: invalid argument");
+    return SBI_ERR_INVALID;
+  }
+  if (P == 0 || n == 0) return SBI_OK;
+  const bool padded = lda >= P + (P & 1) && ldb >= n + (n & 1);
+  return contract_f64(A, lda, B, ldb, offset, Y, ldy, P, n, K, padded, workspace, ws_bytes,
+                      (hipStream_t)stream);
 }
 
 extern "C" int sbi_contract_split_k4(const double* A64, int64_t lda64, const double* B64,
@@ -1011,7 +1321,7 @@ extern "C" int sbi_contract_split_k4(const double* A64, int64_t lda64, const dou
     return SBI_ERR_INVALID;
   }
   if (P == 0 || n == 0) return SBI_OK;
-  return contract_launch<float, true>(A32, lda32, B32, ldb32, offset, Y, ldy, P, n, K32, A64,
+  return contract_launch<true>(A32, lda32, B32, ldb32, offset, Y, ldy, P, n, K32, A64,
                                       lda64, B64, ldb64, K64, (hipStream_t)stream);
 }
 
@@ -1021,7 +1331,7 @@ extern "C" int64_t sbi_contract_split_k4_workspace(int64_t P, int64_t n, int64_t
     sbi::set_error("sbi_contract_split_k4_workspace: invalid argument");
     return -1;
   }
-  const SplitPlan sp = split_plan<float>(P, n, K32, K64);
+  const SplitPlan sp = split_plan(P, n, K32, K64);
   return sp.nsplit ? sp.part_bytes + sp.head_bytes : 0;
 }
 
@@ -1042,11 +1352,11 @@ extern "C" int sbi_contract_split_k4_ws(const double* A64, int64_t lda64, const 
     return SBI_ERR_INVALID;
   }
   if (P == 0 || n == 0) return SBI_OK;
-  const SplitPlan sp = split_plan<float>(P, n, K32, K64);
+  const SplitPlan sp = split_plan(P, n, K32, K64);
   if (sp.nsplit == 0 || !workspace || ws_bytes < sp.part_bytes + sp.head_bytes)
-    return contract_launch<float, true>(A32, lda32, B32, ldb32, offset, Y, ldy, P, n, K32, A64,
+    return contract_launch<true>(A32, lda32, B32, ldb32, offset, Y, ldy, P, n, K32, A64,
                                         lda64, B64, ldb64, K64, (hipStream_t)stream);
-  return contract_split_launch<float, true>(sp, A32, lda32, B32, ldb32, offset, Y, ldy, P, n,
+  return contract_split_launch<true>(sp, A32, lda32, B32, ldb32, offset, Y, ldy, P, n,
                                             K32, A64, lda64, B64, ldb64, K64, workspace,
                                             (hipStream_t)stream);
 }
@@ -1064,7 +1374,7 @@ extern "C" int sbi_contract_split(const double* A64, int64_t lda64, const double
     return SBI_ERR_INVALID;
   }
   if (P == 0 || n == 0) return SBI_OK;
-  return contract_launch<float>(A32, lda32, B32, ldb32, offset, Y, ldy, P, n, K32, A64, lda64,
+  return contract_launch<false>(A32, lda32, B32, ldb32, offset, Y, ldy, P, n, K32, A64, lda64,
                                 B64, ldb64, K64, (hipStream_t)stream);
 }
 

@@ -418,7 +418,9 @@ class SmolyakBarycentricInterpolator:
         # surpluses in nf.nus order (adjoint), and in the basis-row order of the GEMM paths (the
         # FP64 head rows first)
         self._S = {"f64": _dev_tensor(self._nform.s, f64, dev)}
-        self._Sg = {"f64": _dev_tensor(self._nform.s[NL.basis_order], f64, dev)}
+        Sg = self._rows_buffer(len(NL.basis_order), self._d_out, f64, dev)
+        Sg.copy_(_dev_tensor(self._nform.s[NL.basis_order], f64, dev))
+        self._Sg = {"f64": Sg}
         self._head_fac = _dev_tensor(NL.head_fac, i32, dev)
         # the mixed GEMM path's operands, for sbi_newton_eval_mixed_gemm
         nh = NL.n_head
@@ -566,15 +568,31 @@ class SmolyakBarycentricInterpolator:
         """Row stride of a row-major matrix (a single row may carry any stride in torch)."""
         return t.stride(0) if t.shape[0] > 1 else max(t.shape[1], 1)
 
+    @staticmethod
+    def _rows_buffer(rows, cols, dtype, device):
+        """An uninitialised (rows, cols) matrix; FP64 rows start on 16 bytes (an odd width gets one
+        spare element), which the FP64 contraction's wide copies need."""
+        ld = cols + (cols & 1) if dtype == torch.float64 else cols
+        return torch.empty((rows, ld), dtype=dtype, device=device)[:, :cols]
+
     def _contract(self, A, B, offset, y):
-        """y[P, n] = offset + A^T B on the matrix cores (sbi_contract: FP64 or FP32 MFMA with
-        FP64 accumulation; rows independent of the batch)."""
-        code = {torch.float64: 0, torch.float32: 1}[A.dtype]
+        """y[P, n] = offset + A^T B on the matrix cores (sbi_contract_f64_ws; sbi_contract for FP32
+        operands with FP64 accumulation; rows independent of the batch)."""
         ld = self._ld
-        N.check(N.fn["sbi_contract"](A.data_ptr(), ld(A), B.data_ptr(), ld(B),
-                                     None if offset is None else offset.data_ptr(), y.data_ptr(),
-                                     ld(y), y.shape[0], y.shape[1], A.shape[0], code,
-                                     self._stream()), "contract")
+        off = None if offset is None else offset.data_ptr()
+        (P, n), K = y.shape, A.shape[0]
+        if A.dtype == torch.float64:
+            nb = N.c_i64()
+            N.check(N.fn["sbi_contract_f64_workspace"](P, n, K, ctypes.byref(nb)), "contract")
+            ws = nb.value
+            W = torch.empty(ws, dtype=torch.uint8, device=y.device) if ws else None
+            N.check(N.fn["sbi_contract_f64_ws"](A.data_ptr(), ld(A), B.data_ptr(), ld(B), off,
+                                                y.data_ptr(), ld(y), P, n, K,
+                                                W.data_ptr() if ws else None, ws, self._stream()),
+                    "contract")
+            return
+        N.check(N.fn["sbi_contract"](A.data_ptr(), ld(A), B.data_ptr(), ld(B), off, y.data_ptr(),
+                                     ld(y), P, n, K, 1, self._stream()), "contract")
 
     def _eval_bary_gemm(self, x, fp32=False, out=None):
         """y = offset + W F: barycentric entry weights (HIP kernel), then the contraction with the
@@ -595,9 +613,9 @@ class SmolyakBarycentricInterpolator:
         for a in range(0, P, pc):
             b = min(P, a + pc)
             xc = x[a:b]
-            WT = torch.empty((K, b - a), dtype=dt, device=self._device)
-            N.check(N.fn[fn](self._plan, xc.data_ptr(), b - a, xc.stride(0), WT.data_ptr(), b - a,
-                             self._stream()), "bary_basis")
+            WT = self._rows_buffer(K, b - a, dt, self._device)
+            N.check(N.fn[fn](self._plan, xc.data_ptr(), b - a, xc.stride(0), WT.data_ptr(),
+                             WT.stride(0), self._stream()), "bary_basis")
             self._contract(WT, F, self._dev["offset"], y[a:b])
         return y
 
@@ -618,7 +636,9 @@ class SmolyakBarycentricInterpolator:
         key = kind + "T"
         ST = self._S.get(key)
         if ST is None:
-            ST = self._surpluses(kind).t().contiguous()
+            S = self._surpluses(kind)
+            ST = self._rows_buffer(S.shape[1], S.shape[0], S.dtype, S.device)
+            ST.copy_(S.t())
             self._S[key] = ST
         return ST
 
@@ -666,10 +686,10 @@ class SmolyakBarycentricInterpolator:
             for a in range(0, P, pc):
                 b = min(P, a + pc)
                 xc = x[a:b]
-                HT = torch.empty((Nn, b - a), dtype=torch.float64, device=self._device)
+                HT = self._rows_buffer(Nn, b - a, torch.float64, self._device)
                 N.check(N.fn["sbi_newton_basis_rows"](self._nplan, xc.data_ptr(), b - a,
-                                                      xc.stride(0), 0, Nn, HT.data_ptr(), b - a, 0,
-                                                      st), "basis")
+                                                      xc.stride(0), 0, Nn, HT.data_ptr(),
+                                                      HT.stride(0), 0, st), "basis")
                 self._contract(HT, S, None, y[a:b])
             return y
         if kind == "f32":  # one call per chunk: head rows, FP32 rows, contraction
@@ -747,9 +767,10 @@ class SmolyakBarycentricInterpolator:
         for p0 in range(0, P, chunk):
             p1 = min(P, p0 + chunk)
             xc = x[p0:p1]
-            # G^T[nu, p] = sum_m S[nu, m] v[p, m] on the matrix cores (sbi_contract with
-            # A = S^T and B = v^T; FP64, or FP32 operands with FP64 accumulation)
-            VT = v[p0:p1].t().to(dt).contiguous()
+            # G^T[nu, p] = sum_m S[nu, m] v[p, m] on the matrix cores (A = S^T and B = v^T; FP64,
+            # or FP32 operands with FP64 accumulation)
+            VT = self._rows_buffer(self._d_out, p1 - p0, dt, self._device)
+            VT.copy_(v[p0:p1].detach().t())
             GT = torch.empty((n_nodes, p1 - p0), dtype=torch.float64, device=self._device)
             self._contract(ST, VT, None, GT)
             nb = int(N.fn["sbi_newton_vjp_workspace"](self._nplan, p1 - p0))

@@ -274,3 +274,29 @@ def test_contract_bf16_tile_shapes_same_bits(gpu):
         Ys = [_bf16_contract(A64, B64, K64, A8, B8, K16, off, P, n, 4096, n) for P in (4096, 2048, 512)]
         assert torch.equal(Ys[0][:2048], Ys[1]), K64
         assert torch.equal(Ys[0][:512], Ys[2]), K64
+
+
+@pytest.mark.parametrize("P,n,K", [(1, 1, 1), (63, 33, 15), (65, 96, 257), (500, 64, 2049),
+                                   (130, 7, 4096), (777, 40, 5003), (5000, 160, 4100)])
+def test_contract_f64_ws_same_bits_for_every_split_and_alignment(gpu, P, n, K):
+    """sbi_contract_f64_ws: k spread over workgroups (by 256-term chains or 2048-term slices, as the
+    shape asks) and 16-byte copies with a spare element per odd row, against sbi_contract (no
+    workspace, 8-byte loads where a width is odd): the same bits; and against the FP64 product.
+    Bound: (K + 8) * 2^-53 of sum |A| |B| per element (one rounding per term, any order)."""
+    g = torch.Generator(device="cuda").manual_seed(P + 3 * n + 7 * K)
+    A = torch.randn((K, P + P % 2), dtype=torch.float64, device="cuda", generator=g)
+    B = torch.randn((K, n + n % 2), dtype=torch.float64, device="cuda", generator=g)
+    off = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
+    A[:, P:], B[:, n:] = float("nan"), float("nan")  # the spare elements are never used
+    nb = N.c_i64()
+    N.check(N.fn["sbi_contract_f64_workspace"](P, n, K, ctypes.byref(nb)), "workspace")
+    W = torch.full((max(nb.value, 8) // 8,), float("nan"), dtype=torch.float64, device="cuda")
+    Y = torch.full((P, n), float("nan"), dtype=torch.float64, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    N.check(N.fn["sbi_contract_f64_ws"](A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0),
+                                        off.data_ptr(), Y.data_ptr(), n, P, n, K, W.data_ptr(),
+                                        nb.value, st), "contract")
+    Ac, Bc = A[:, :P].contiguous(), B[:, :n].contiguous()
+    assert torch.equal(Y, contract(Ac, Bc, off))
+    ref, scale = _ref(Ac, Bc, off)
+    assert ((Y - ref).abs() <= (K + 8) * 2.0 ** -53 * (scale + off.abs())).all()
