@@ -286,6 +286,20 @@ typedef struct sbi_newton_desc {
   /* FP64 matrix-core kernel of sbi_newton_eval_f64 (optional: NULL selects the streaming one):
    * the A steps of mt_a in FP64 ([64 * mt_steps], read from global memory) */
   const double* mt_a64;
+  /* dense Jacobian of more than 8 outputs: the adjoint entries in rows, dim by dim, each dim
+   * padded to a multiple of four rows (padding rows repeat the dim's last entry and are not used) */
+  int32_t n_jac_jobs;
+  int32_t n_jac_slots;
+  int32_t n_jac_group_red;
+  int32_t _pad7;
+  const int32_t* jac_row;     /* [2 * jac_row_off[d_in]] {adjoint entry, its node} */
+  const int32_t* jac_row_off; /* [d_in + 1] first row of each input dim */
+  const int32_t* jac_row_end; /* [d_in] one past its last row that is not padding */
+  const int32_t* jac_job;     /* [4 * n_jac_jobs] {first row, end row, first dim, partial slot}: the
+                                 rows of whole groups of 8 dims (slot -1), or a part of one group's
+                                 rows (slot 0 .. n_jac_slots - 1) */
+  const int32_t* jac_group_red; /* [3 * n_jac_group_red] {first dim, first slot, slots} of the
+                                 groups in several parts */
 } sbi_newton_desc;
 
 typedef struct sbi_newton_plan sbi_newton_plan;

@@ -68,6 +68,9 @@ class NewtonDesc(ctypes.Structure):
         ("mt_a", c_vp), ("mt_grp", c_vp), ("mi_rec", c_vp), ("mwave_item", c_vp),
         ("gemm_head", c_i32), ("gemm_kq", c_i32), ("head_fac", c_vp), ("gemm_s64", c_vp),
         ("ld_s64", c_i64), ("gemm_sq", c_vp), ("mt_a64", c_vp),
+        ("n_jac_jobs", c_i32), ("n_jac_slots", c_i32), ("n_jac_group_red", c_i32), ("_pad7", c_i32),
+        ("jac_row", c_vp), ("jac_row_off", c_vp), ("jac_row_end", c_vp), ("jac_job", c_vp),
+        ("jac_group_red", c_vp),
     ]
 
 

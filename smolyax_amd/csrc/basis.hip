@@ -1033,6 +1033,8 @@ static bool jac_global_table(const sbi_newton_desc& d) {
   return (size_t)d.n_tab_rows * kTile * sizeof(double) > kJacLdsMax;
 }
 
+static int64_t jac_ld(int64_t P) { return P + (P & 1); }  // row stride of D^T
+
 extern "C" int64_t sbi_newton_jacobian_workspace(const sbi_newton_plan* plan, int64_t P,
                                                  int64_t n) {
   const sbi_newton_desc* dp = nullptr;
@@ -1043,7 +1045,9 @@ extern "C" int64_t sbi_newton_jacobian_workspace(const sbi_newton_plan* plan, in
   int64_t bytes = 0;
   const int64_t P64 = (P + kTile - 1) / kTile * kTile;
   if (jac_global_table(*dp)) bytes += (int64_t)dp->n_tab_rows * P64 * (int64_t)sizeof(double);
-  if (n > kJacDirectMax) bytes += (int64_t)dp->n_vjp_ent * P * (int64_t)sizeof(double);
+  if (n > kJacDirectMax)  // D^T (row stride even), then the jobs' parts
+    bytes += (int64_t)dp->n_vjp_ent * jac_ld(P) * (int64_t)sizeof(double) +
+             (int64_t)dp->n_jac_slots * P * n * sbi::kJacGroup * (int64_t)sizeof(double);
   else bytes += (int64_t)dp->n_jac_partials * P * n * (int64_t)sizeof(double);
   return bytes;
 }
@@ -1075,7 +1079,7 @@ static void jac_basis_launch(const sbi_newton_desc& d, const double* x, int64_t 
       1, std::min<int64_t>((ngrp + kDTWaves - 1) / kDTWaves, (1024 + tiles - 1) / tiles));
   hipLaunchKernelGGL(newton_jac_basis_kernel<kG>, dim3((unsigned)tiles, (unsigned)ny),
                      dim3(kTile * kDTWaves), lds_bytes, st, d, x, P, ldx, gtab, (int64_t)d.n_tab_rows,
-                     DT, P);
+                     DT, jac_ld(P));
 }
 
 extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double* x, int64_t P,
@@ -1090,7 +1094,9 @@ extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double
   }
   const sbi_newton_desc& d = *dp;
   if (!d.vjp_ent || !d.vjp_slot_off || !d.tab_dim || !d.vjp_dim_off || !d.sing_off ||
-      !d.sing_x || !d.jac_unit || !d.jac_red || !d.vjp_ent_row || !d.row_tdim || ldx < d.d_in) {
+      !d.sing_x || !d.jac_unit || !d.jac_red || !d.vjp_ent_row || !d.row_tdim || ldx < d.d_in ||
+      (n > kJacDirectMax && (!d.jac_row || !d.jac_row_off || !d.jac_row_end || !d.jac_job ||
+                              !d.jac_group_red || d.n_jac_jobs < 1))) {
     sbi::set_error("sbi_newton_jacobian_f64: plan has no Jacobian tables");
     return SBI_ERR_INVALID;
   }
@@ -1151,10 +1157,11 @@ extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double
       else jac_basis_launch<false>(d, x, P, ldx, gtab, DT, st);
       SBI_HIP_CHECK(hipGetLastError());
     }
-    // one group of D^T rows per input dim (dims without entries get zeros); the surplus row of
-    // an entry is its node, the first int32 of its 16-byte record
-    const int rc = sbi::contract_jacobian_f64(DT, P, S, lds, (const int32_t*)d.vjp_ent, 4,
-                                              d.vjp_dim_off, (int)d.d_in, J, P, n, st);
+    // the rows of D^T by input dim (dims without entries get zeros)
+    const sbi::JacRows rows{d.jac_row, d.jac_row_off, d.jac_row_end, d.jac_job, d.jac_group_red,
+                            d.n_jac_jobs, d.n_jac_group_red};
+    const int rc = sbi::contract_jacobian_f64(DT, jac_ld(P), S, lds, rows, (int)d.d_in, J, P, n,
+                                              DT + (int64_t)d.n_vjp_ent * jac_ld(P), st);
     if (rc != SBI_OK) return rc;
   }
   const int64_t tot = P * d.d_in;

@@ -1059,170 +1059,232 @@ contract_bf16_wide_kernel(SBI_BF16_ARGS) {
 #undef SBI_BF16_ARGS
 
 // ------------------------------------------------------------------------------------------
-// Jacobian contraction: for each input dim z, J[p, c, z] = sum_{k in [zoff[z], zoff[z+1])}
-// A[k, p] B[brow[k * brs], c] (B rows gathered per row of A).  A workgroup owns a
-// 64-point x (32 * FN)-output tile for JG consecutive dims, streams their rows
-// [zoff[z0], zoff[z0 + JG]) as one pipelined sequence of 16-row chunks and keeps JG accumulator
-// tiles in registers: a chunk that spans a dim boundary is applied once per dim it touches, with
-// the other rows masked to zero.  Each lane finally writes JG consecutive doubles
-// J[p, c, z0 .. z0 + JG) (one 8 * JG-byte run) instead of JG scattered words.
-// Workgroup order: the n-tiles of one (point tile, dim group) go to the same XCD (consecutive
-// workgroups of one XCD), so its L2 serves their shared A rows; consecutive (point tile, dim
-// group) pairs go to different XCDs, which spreads the heavy low dims.
+// Jacobian contraction: for each input dim z, J[p, c, z] = sum over the rows q of dim z of
+// A[e_q, p] S[v_q, c].  Rows are listed dim by dim, each dim padded to a multiple of four, so every
+// 4-row MFMA step belongs to one dim (steps spanning dims would run once per dim: 2-4 x the
+// matrix work of the many dims with a handful of rows).
+//
+// A workgroup of 4 waves takes one job for 64 points x 32 outputs: the rows of a group of kJacDims
+// consecutive dims (one accumulator tile per dim in registers), or one part of a group with many
+// rows: the first dims of an index set hold most of them (the first 8 of 200: 5594 of 11 506), so
+// the host cuts such a group into parts, which jac_group_reduce_kernel adds in order.  Bound: the
+// FP64 matrix cores (75 us at 999 points x 256 outputs x 200 dims) and, for the many short groups,
+// the latency of a job's start; measured there 277 us + 28 us for the parts (466 us with masked
+// chunks across dims, each wave loading from L2 and every lane writing its own 64 bytes; without
+// the writes of J 223 us).  (Groups with few rows joined into longer jobs were slower, 542 us: a wave's stores of a finished group hold
+// up its next loads, which complete in order behind them.)
+//
+// Operands are staged in LDS in chunks of 32 rows, three buffers, copied two chunks ahead by direct
+// global -> LDS loads (16-byte slots of odd rows rotated by 8, as in contract_f64_kernel); the row
+// table is copied the same way three chunks ahead of that, into each wave's own ring, and read
+// into registers a chunk before it is needed.  Every wave issues the same number of copies per
+// chunk, past the last one too (rows clamped), so the waits are counts.  kWide = false: S rows that do not start on 16 bytes are copied in 4-byte pieces.
+//
+// The tile is written through LDS, one accumulator register of every dim at a time, so that eight
+// consecutive lanes write the kJacDims consecutive doubles of one (point, output): a lane writing
+// them itself makes eight requests of 8 bytes where one of 64 does.
 // ------------------------------------------------------------------------------------------
-// Tile shapes (dims per workgroup JG, 16-output fragments per wave FN): 8 x 1 for up to 512
-// outputs (d_out 256: 1.31 ms against 1.43-1.48 ms for 4 x 2, 2 x 4, 8 x 2), 2 x 4 above (d_out
-// 4096: 3.48 ms against 4.10 ms for 8 x 1, 3.72 ms for 4 x 2, 3.58 ms for 2 x 2).
+constexpr int kJacDims = sbi::kJacGroup;  // dims per job
+constexpr int kJacN = 32;                 // outputs per job
+constexpr int kJacChunk = 32;             // rows per chunk
+constexpr int kJacRing = 8;               // row-table chunks on chip (six in use)
+constexpr int kJacT = 68;  // doubles between dims of a tile being written (the 8 dims of 4 outputs
+                           // fall into all banks)
 
-template <int JG, int FN>
-__global__ __launch_bounds__(64 * kWaves) void jac_contract_kernel(
-    const double* __restrict__ A, int64_t lda, const double* __restrict__ B, int64_t ldb,
-    const int32_t* __restrict__ brow, int64_t brs, const int32_t* __restrict__ zoff, int nz,
-    double* __restrict__ J, int64_t P, int64_t n, int nt, int ntp, int npairs) {
-  const int L = blockIdx.x;
-  const int xcd = L & 7, idx = L >> 3;
-  const int tn = idx % nt;
-  const int pair = (idx / nt) * 8 + xcd;
-  if (pair >= npairs) return;
-  const int tp = pair % ntp, zg = pair / ntp;
+template <bool kWide>
+__global__ __launch_bounds__(64 * kWaves, 2) void jac_contract_kernel(
+    const double* __restrict__ A, uint32_t lda, const double* __restrict__ S, int64_t lds,
+    sbi::JacRows t, int nz, double* __restrict__ J, int64_t P, int64_t n, int ntp, int ntn,
+    double* __restrict__ part) {
+  constexpr int C = kJacChunk;
+  constexpr int kA = C * kBlockM * 8, kB = C * kJacN * 8, kRec = C * 8;  // bytes of a chunk
+  constexpr int kNA = kA / 4096, kNB = kB / 4096 * (kWide ? 1 : 4);      // copies per wave
+  constexpr int kPer = kNA + kNB + 1;
+  static_assert(kRec == 64 * 4, "one copy per row-table chunk");
+  __shared__ __attribute__((aligned(16))) char smem[3 * (kA + kB) + kWaves * kJacRing * kRec];
+  static_assert(kWaves * kJacDims * kJacT * 8 <= 3 * (kA + kB), "the tile being written");
+  const int L = blockIdx.x, idx = L >> 3;
+  const int tn = idx % ntn;
+  const int pair = (idx / ntn) * 8 + (L & 7);
+  if (pair >= ntp * t.n_jobs) return;
+  const int tp = pair % ntp;
+  const int32_t* __restrict__ job = t.job + 4 * (pair / ntp);
+  const int r0 = job[0], r1 = job[1], slot = job[3];
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, g = lane >> 4;
-  const int64_t m_base = (int64_t)tp * kBlockM + wm * 32;
-  const int64_t n_base = (int64_t)tn * (32 * FN) + wn * (16 * FN);
-  int64_t pcol[2], jcol[FN];
-#pragma unroll
-  for (int fm = 0; fm < 2; ++fm) pcol[fm] = min(m_base + fm * 16 + li, P - 1);
-#pragma unroll
-  for (int fn = 0; fn < FN; ++fn) jcol[fn] = min(n_base + fn * 16 + li, n - 1);
+  const int mw = (wave & 1) * 32, nw = (wave >> 1) * 16;
+  const int64_t m0 = (int64_t)tp * kBlockM, n0 = (int64_t)tn * kJacN;
+  char* const ring = smem + 3 * (kA + kB) + wave * kJacRing * kRec;
 
-  const int z0 = zg * JG;
-  int zb[JG + 1];  // row boundaries of the group's dims (uniform)
-#pragma unroll
-  for (int jj = 0; jj <= JG; ++jj) zb[jj] = zoff[min(z0 + jj, nz)];
-  const int64_t R0 = zb[0], R1 = zb[JG];
-
-  v4d acc[JG][2][FN];
-#pragma unroll
-  for (int jj = 0; jj < JG; ++jj)
-#pragma unroll
-    for (int fm = 0; fm < 2; ++fm)
-#pragma unroll
-      for (int fn = 0; fn < FN; ++fn) acc[jj][fm][fn] = v4d{0, 0, 0, 0};
-
-  // rows k0 + 4g + s of a chunk, clamped into the stream (the extra rows are masked); the B row
-  // indices are read one chunk ahead of the B rows themselves
-  double a[2][4], b[FN][4];
-  int bi[4];
-  auto load_idx = [&](int64_t k0) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) bi[s] = brow[min(k0 + 4 * g + s, R1 - 1) * brs];
+  // copies of this wave: LDS rows 2 i, 2 i + 1 of A for i = wave + 4 u (lane: row 2 i + lane / 32, pair
+  // lane % 32); S rows 4 i .. 4 i + 3 for i = wave + 4 u, four at a time (lane: row lane / 16, pair
+  // lane % 16) or one at a time in words (lane: word lane of the row's 64)
+  const int ar = lane >> 5;
+  const double* __restrict__ ap =
+      A + min(m0 + (((lane & 31) ^ (8 * ar)) * 2), (P - 1) & ~(int64_t)1);
+  const int br = kWide ? lane >> 4 : 0;
+  const int64_t bcol = n0 + (((lane & 15) ^ (8 * (br & 1))) * 2);
+  const double* __restrict__ bp = S + min(bcol, (n - 1) & ~(int64_t)1);
+  int ra[kNA], rs[kNB];  // rows of A and S of the next chunk to be copied
+  auto copy_rec = [&](int c) {  // row-table chunk c
+    const int64_t w = (int64_t)min(r0 + c * C + (lane >> 1), r1 - 1) * 2 + (lane & 1);
+    __builtin_amdgcn_global_load_lds((const void*)(t.row + w),
+                                     (lds_void*)(ring + (c % kJacRing) * kRec), 4, 0, 0);
   };
-  auto load = [&](int64_t k0) {
+  auto read_rec = [&](int c) {  // (row-table chunk c has landed)
+    const int2* rec = (const int2*)(ring + (c % kJacRing) * kRec);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int64_t k = min(k0 + 4 * g + s, R1 - 1);
-      const double* __restrict__ ar = A + k * lda;
+    for (int u = 0; u < kNA; ++u) ra[u] = rec[2 * (wave + 4 * u) + ar].x;
 #pragma unroll
-      for (int fm = 0; fm < 2; ++fm) a[fm][s] = ar[pcol[fm]];
-      const double* __restrict__ br = B + (int64_t)bi[s] * ldb;
-#pragma unroll
-      for (int fn = 0; fn < FN; ++fn) b[fn][s] = br[jcol[fn]];
-    }
+    for (int u = 0; u < kNB; ++u)
+      rs[u] = kWide ? rec[4 * (wave + 4 * u) + br].y : rec[4 * (wave + 4 * (u / 4)) + u % 4].y;
   };
-  if (R1 > R0) {
-    load_idx(R0);
-    load(R0);
-    if (R0 + kChunk < R1) load_idx(R0 + kChunk);
-  }
-  double ca[2][4], cb[FN][4];
-  auto advance = [&](int64_t k0) {  // this chunk's operands; the next chunk's loads in flight
+  auto copy = [&](int b) {  // the next chunk of A and S into buffer b
+    char* da = smem + b * kA + wave * 1024;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      ca[0][s] = a[0][s];
-      ca[1][s] = a[1][s];
+    for (int u = 0; u < kNA; ++u)
+      __builtin_amdgcn_global_load_lds((const void*)(ap + (uint64_t)(uint32_t)ra[u] * lda),
+                                       (lds_void*)(da + u * 4096), 16, 0, 0);
+    char* ds = smem + 3 * kA + b * kB + wave * 1024;
 #pragma unroll
-      for (int fn = 0; fn < FN; ++fn) cb[fn][s] = b[fn][s];
-    }
-    if (k0 + kChunk < R1) {
-      load(k0 + kChunk);
-      if (k0 + 2 * kChunk < R1) load_idx(k0 + 2 * kChunk);
-    }
-  };
-  auto apply = [&](int64_t k0) {  // a chunk applied to every dim it touches
-    const int64_t klast = min(k0 + kChunk, R1) - 1;
-    // dims touched by this chunk: [first row's dim, last row's dim] (uniform)
-#pragma unroll
-    for (int jj = 0; jj < JG; ++jj) {
-      if (zb[jj + 1] <= k0 || zb[jj] > klast || zb[jj] == zb[jj + 1]) continue;
-      if (zb[jj] <= k0 && zb[jj + 1] >= k0 + kChunk) {  // all 16 rows belong to this dim
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int fm = 0; fm < 2; ++fm)
-#pragma unroll
-            for (int fn = 0; fn < FN; ++fn)
-              acc[jj][fm][fn] = mfma(ca[fm][s], cb[fn][s], acc[jj][fm][fn]);
+    for (int u = 0; u < kNB; ++u) {
+      if constexpr (kWide) {
+        __builtin_amdgcn_global_load_lds((const void*)(bp + (int64_t)rs[u] * lds),
+                                         (lds_void*)(ds + u * 4096), 16, 0, 0);
       } else {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int64_t k = k0 + 4 * g + s;
-          const bool in = k >= zb[jj] && k < zb[jj + 1];
-#pragma unroll
-          for (int fn = 0; fn < FN; ++fn) {
-            const double bv = in ? cb[fn][s] : 0.0;
-#pragma unroll
-            for (int fm = 0; fm < 2; ++fm) acc[jj][fm][fn] = mfma(ca[fm][s], bv, acc[jj][fm][fn]);
-          }
-        }
+        const int64_t col = n0 + ((lane >> 1) ^ (16 * (u & 1)));
+        const double* row = S + (int64_t)rs[u] * lds + min(col, n - 1);
+        __builtin_amdgcn_global_load_lds((const void*)((const int*)row + (lane & 1)),
+                                         (lds_void*)(ds + u / 4 * 4096 + u % 4 * 256), 4, 0, 0);
       }
     }
   };
-  // The chunks in stream order: those wholly inside dim jj in a branch-free loop on acc[jj], then
-  // the chunk that ends dim jj inside it (or the stream's last, partial chunk) through apply.  At
-  // dim jj the next chunk starts at or after the dim's first row, so every chunk is applied once
-  // and each dim's sum sees the same MFMAs in the same order as a single chunk loop with a per-dim
-  // test (same bits; 320 points x 4096 outputs x 100 dims: 3.14-3.23 ms against 3.45-3.51 ms,
-  // 2560 x 256 x 200: 1.15-1.23 ms against 1.20-1.26 ms).
-  int64_t k0 = R0;
-#pragma unroll
-  for (int jj = 0; jj < JG; ++jj) {
-    while (k0 < R1 && zb[jj] <= k0 && k0 + kChunk <= zb[jj + 1]) {
-      advance(k0);
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int fm = 0; fm < 2; ++fm)
-#pragma unroll
-          for (int fn = 0; fn < FN; ++fn)
-            acc[jj][fm][fn] = mfma(ca[fm][s], cb[fn][s], acc[jj][fm][fn]);
-      k0 += kChunk;
+  const int sw = 16 * (g & 1);
+  v4d cur[2];
+  // one 4-row step at row 4 s of the chunk in buffer b; rows at and past `end` (relative to the
+  // chunk) count as zero
+  auto step = [&](int b, int s, int end) {
+    const int r = 4 * s + g;
+    const double* sa = (const double*)(smem + b * kA) + r * kBlockM;
+    double a0 = sa[(mw + li) ^ sw], a1 = sa[(mw + 16 + li) ^ sw];
+    double bv = ((const double*)(smem + 3 * kA + b * kB))[r * kJacN + ((nw + li) ^ sw)];
+    if (4 * s + 4 > end && r >= end) a0 = a1 = bv = 0.0;
+    cur[0] = mfma(a0, bv, cur[0]);
+    cur[1] = mfma(a1, bv, cur[1]);
+  };
+
+  v4d acc[kJacDims][2];
+  int z0 = job[2];
+  if (r0 < r1) {
+    copy_rec(0);
+    copy_rec(1);
+    copy_rec(2);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    read_rec(0);
+    copy(0);
+    copy_rec(3);
+    read_rec(1);
+    copy(1);
+    copy_rec(4);
+    read_rec(2);
+  }
+  // lane l: first row of the group's dim l, end of its real rows
+  const int offv = t.off[min(z0 + min(lane, kJacDims), nz)];
+  const int endv = t.end[min(z0 + min(lane, kJacDims - 1), nz - 1)];
+  int q = r0, c = 0, q0 = r0, b = 0;  // next row; its chunk, the chunk's first row and buffer
+  auto begin = [&] {  // chunk c has landed in every wave (and row-table chunk c + 3); c + 2 is copied
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
+    asm volatile("s_barrier" ::: "memory");
+    copy(b == 0 ? 2 : b - 1);
+    copy_rec(c + 5);
+    read_rec(c + 3);
+  };
+  auto advance = [&](int rows) {
+    q += rows;
+    if (q == q0 + C) {
+      ++c;
+      q0 = q;
+      b = b == 2 ? 0 : b + 1;
     }
-    if (k0 < R1 && k0 < zb[jj + 1]) {
-      advance(k0);
-      apply(k0);
-      k0 += kChunk;
+  };
+  for (int jj = 0; jj < kJacDims; ++jj) {
+    const int end = min(__builtin_amdgcn_readlane(offv, jj + 1), r1);
+    const int real = __builtin_amdgcn_readlane(endv, jj);
+    const int whole = min(end, real);
+    cur[0] = cur[1] = v4d{0, 0, 0, 0};
+    while (q < end) {
+      // (whole chunks in a loop of their own: the accumulators stay in place)
+      while (q == q0 && q + C <= whole) {
+        begin();
+#pragma unroll
+        for (int s = 0; s < C / 4; ++s) step(b, s, C);
+        advance(C);
+      }
+      if (q >= end) break;
+      if (q == q0) begin();
+      const int stop = min(end, q0 + C);
+      for (; q < stop; q += 4) step(b, (q - q0) >> 2, real - q0);
+      advance(0);
+    }
+    switch (jj) {  // (register arrays take constant indices)
+#define SBI_KEEP(i)      \
+  case i:                \
+    acc[i][0] = cur[0];  \
+    acc[i][1] = cur[1];  \
+    break;
+      SBI_KEEP(0) SBI_KEEP(1) SBI_KEEP(2) SBI_KEEP(3) SBI_KEEP(4) SBI_KEEP(5) SBI_KEEP(6) SBI_KEEP(7)
+#undef SBI_KEEP
     }
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies past the last chunk
+  __syncthreads();
 
   // FP64 16x16x4 result: row (point) g + 4r in register r, column (output) = lane % 16
-#pragma unroll
-  for (int fn = 0; fn < FN; ++fn) {
-    const int64_t col = n_base + fn * 16 + li;
-    if (col >= n) continue;
+  double* __restrict__ tr = (double*)smem + wave * kJacDims * kJacT;
+  const int jj = lane & 7;
+  for (;; z0 += kJacDims) {  // (groups without rows follow the job of the group before them)
+    double* __restrict__ out = slot >= 0 ? part + (int64_t)slot * P * n * kJacDims + jj : J + z0 + jj;
+    const int64_t ldo = slot >= 0 ? kJacDims : nz;
+    const bool mine = slot >= 0 || z0 + jj < nz;
 #pragma unroll
     for (int fm = 0; fm < 2; ++fm)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t row = m_base + fm * 16 + g + 4 * r;
-        if (row >= P) continue;
-        double* __restrict__ out = J + (row * n + col) * nz + z0;
 #pragma unroll
-        for (int jj = 0; jj < JG; ++jj)
-          if (z0 + jj < nz) out[jj] = acc[jj][fm][fn][r];
+        for (int u = 0; u < kJacDims; ++u) tr[u * kJacT + lane] = acc[u][fm][r];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {  // the elements of lanes 8 i .. 8 i + 7
+          const int l = 8 * i + (lane >> 3);
+          const int64_t row = m0 + mw + fm * 16 + (l >> 4) + 4 * r, col = n0 + nw + (l & 15);
+          const double v = tr[jj * kJacT + l];
+          if (row < P && col < n && mine) out[(row * n + col) * ldo] = v;
+        }
       }
+    if (slot >= 0 || z0 + kJacDims >= nz ||
+        t.off[min(z0 + 2 * kJacDims, nz)] > t.off[z0 + kJacDims])
+      return;
+#pragma unroll
+    for (int u = 0; u < kJacDims; ++u) acc[u][0] = acc[u][1] = v4d{0, 0, 0, 0};
+  }
+}
+
+// J of the dim groups that several jobs share: the sum of their parts in order (blockIdx.y: the
+// shared group).
+__global__ __launch_bounds__(256) void jac_group_reduce_kernel(const double* __restrict__ part,
+                                                              const int32_t* __restrict__ red,
+                                                              int nz, double* __restrict__ J,
+                                                              int64_t Pn) {
+  const int z0 = red[3 * blockIdx.y], slot = red[3 * blockIdx.y + 1], count = red[3 * blockIdx.y + 2];
+  const int nd = min(kJacDims, nz - z0);
+  for (int64_t i8 = (int64_t)blockIdx.x * 256 + threadIdx.x; i8 < Pn * kJacDims;
+       i8 += (int64_t)gridDim.x * 256) {
+    const int jj = (int)(i8 % kJacDims);
+    double v = 0.0;
+#pragma unroll 4
+    for (int u = 0; u < count; ++u) v += part[((int64_t)slot + u) * Pn * kJacDims + i8];
+    if (jj < nd) J[i8 / kJacDims * nz + z0 + jj] = v;
   }
 }
 
@@ -1230,31 +1292,28 @@ __global__ __launch_bounds__(64 * kWaves) void jac_contract_kernel(
 
 namespace sbi {
 
-template <int JG, int FN>
-static int jac_contract_launch(const double* A, int64_t lda, const double* B, int64_t ldb,
-                               const int32_t* brow, int64_t brs, const int32_t* zoff, int nz,
-                               double* J, int64_t P, int64_t n, hipStream_t st) {
-  const int64_t nt = (n + 32 * FN - 1) / (32 * FN), ntp = (P + kBlockM - 1) / kBlockM,
-                nzg = (nz + JG - 1) / JG;
-  const int64_t npairs = ntp * nzg;
-  const int64_t grid = nt * ((npairs + 7) / 8) * 8;
-  if (grid > 0x7fffffff || npairs > 0x7fffffff) {
+int contract_jacobian_f64(const double* A, int64_t lda, const double* S, int64_t lds,
+                          const JacRows& t, int nz, double* J, int64_t P, int64_t n, double* part,
+                          hipStream_t st) {
+  if (P <= 0 || n <= 0 || nz <= 0) return SBI_OK;
+  const int64_t ntp = (P + kBlockM - 1) / kBlockM, ntn = (n + kJacN - 1) / kJacN;
+  const int64_t grid = ntn * ((ntp * t.n_jobs + 7) / 8) * 8;
+  if (grid > 0x7fffffff || t.n_red > 65535) {
     set_error("contract_jacobian_f64: launch too large");
     return SBI_ERR_INVALID;
   }
-  hipLaunchKernelGGL((jac_contract_kernel<JG, FN>), dim3((unsigned)grid), dim3(64 * kWaves), 0,
-                     st, A, lda, B, ldb, brow, brs, zoff, nz, J, P, n, (int)nt, (int)ntp,
-                     (int)npairs);
+  const bool wide = ((uintptr_t)S & 15) == 0 && lds % 2 == 0 && lds >= n + (n & 1);
+  hipLaunchKernelGGL(wide ? jac_contract_kernel<true> : jac_contract_kernel<false>,
+                     dim3((unsigned)grid), dim3(64 * kWaves), 0, st, A, (uint32_t)lda, S, lds, t, nz,
+                     J, P, n, (int)ntp, (int)ntn, part);
   SBI_HIP_CHECK(hipGetLastError());
+  if (t.n_red > 0) {
+    const int64_t rg = std::min<int64_t>((P * n * kJacDims + 255) / 256, 4096);
+    hipLaunchKernelGGL(jac_group_reduce_kernel, dim3((unsigned)rg, (unsigned)t.n_red), dim3(256), 0,
+                       st, part, t.red, nz, J, P * n);
+    SBI_HIP_CHECK(hipGetLastError());
+  }
   return SBI_OK;
-}
-
-int contract_jacobian_f64(const double* A, int64_t lda, const double* B, int64_t ldb,
-                          const int32_t* brow, int64_t brs, const int32_t* zoff, int nz, double* J,
-                          int64_t P, int64_t n, hipStream_t st) {
-  if (P <= 0 || n <= 0 || nz <= 0) return SBI_OK;
-  if (n > 512) return jac_contract_launch<2, 4>(A, lda, B, ldb, brow, brs, zoff, nz, J, P, n, st);
-  return jac_contract_launch<8, 1>(A, lda, B, ldb, brow, brs, zoff, nz, J, P, n, st);
 }
 
 }  // namespace sbi

@@ -397,6 +397,8 @@ class SmolyakBarycentricInterpolator:
             "jac_red": _dev_tensor(NL.jac_red, i32, dev),
             "vjp_ent_row": _dev_tensor(NL.vjp_ent_row, i32, dev),
             "row_tdim": _dev_tensor(NL.row_tdim, i32, dev),
+            **{f: _dev_tensor(getattr(NL, f), i32, dev)
+               for f in ("jac_row", "jac_row_off", "jac_row_end", "jac_job", "jac_group_red")},
         }
         sing_off, sing_x = self._singular_coordinates()
         # the Jacobian kernels mark NaNs while writing the dims that have factors: every dim with
@@ -417,7 +419,9 @@ class SmolyakBarycentricInterpolator:
             t["mwave_item"] = _dev_tensor(NL.mwave_item, i32, dev)
         # surpluses in nf.nus order (adjoint), and in the basis-row order of the GEMM paths (the
         # FP64 head rows first)
-        self._S = {"f64": _dev_tensor(self._nform.s, f64, dev)}
+        S = self._rows_buffer(self._nform.s.shape[0], self._d_out, f64, dev)
+        S.copy_(_dev_tensor(self._nform.s, f64, dev))
+        self._S = {"f64": S}
         Sg = self._rows_buffer(len(NL.basis_order), self._d_out, f64, dev)
         Sg.copy_(_dev_tensor(self._nform.s[NL.basis_order], f64, dev))
         self._Sg = {"f64": Sg}
@@ -436,6 +440,7 @@ class SmolyakBarycentricInterpolator:
         d.basis_n, d.n_tab_dims, d.n_tab_rows = NL.basis_n, NL.n_tab_dims, NL.n_tab_rows
         d.n_vjp_ent = NL.n_vjp_ent
         d.n_jac_units, d.n_jac_partials, d.n_jac_red = NL.n_jac_units, NL.n_jac_partials, NL.n_jac_red
+        d.n_jac_jobs, d.n_jac_slots, d.n_jac_group_red = NL.n_jac_jobs, NL.n_jac_slots, NL.n_jac_group_red
         d.gemm_head, d.gemm_kq = nh, t["gemm_sq"].shape[0] * 4
         d.ld_s64 = max(t["gemm_s64"].stride(0), self._d_out)
         if "mt_a" in t:

@@ -525,6 +525,7 @@ def head_order(nf: NewtonForm, L: NewtonLayout, n_head: int = HEAD_ROWS):
 
 
 JAC_UNIT = 128  # adjoint entries per work unit of the Jacobian's register pass
+JAC_GROUP = 8   # dims per accumulator set of the Jacobian contraction (d_out > 8)
 
 
 def build_basis_tables(nf: NewtonForm, L: NewtonLayout) -> None:
@@ -593,7 +594,45 @@ def build_basis_tables(nf: NewtonForm, L: NewtonLayout) -> None:
     L.n_jac_units, L.n_jac_partials, L.n_jac_red = len(units), n_part, len(red)
     L.jac_unit = np.array(units or [(0, 0, 0, -1)], dtype=np.int32).reshape(-1)
     L.jac_red = np.array(red or [(0, 0, 0)], dtype=np.int32).reshape(-1)
+    node = np.array([e[0:2].view(np.int32)[0] for e in ent] or [0], dtype=np.int32)
+    build_jacobian_rows(L, node, nf.d_out)
     L.vjp_ent = (np.stack(ent) if ent else np.full((1, 8), 0xFFFF, dtype=np.uint16)).reshape(-1).view(np.uint8)
+
+
+def build_jacobian_rows(L: NewtonLayout, node, d_out: int) -> None:
+    """Rows and jobs of the Jacobian's contraction (d_out > 8): the adjoint entries dim by dim, each
+    dim padded to a multiple of four rows by repeats of its last entry.  Jobs by groups of 8 dims:
+    a group of more than 8 d_out rows (at least 256, whole chunks of 16) is cut into parts of that
+    many, whose sums are added afterwards; groups without rows go with the job before them.  (At
+    256 outputs a part is 20 us of one SIMD's matrix work.)  The cuts depend on the plan alone: a
+    point's sums are the same in every batch."""
+    d_in = len(L.vjp_dim_off) - 1
+    cnt = np.diff(L.vjp_dim_off.astype(np.int64))
+    off = np.zeros(d_in + 1, dtype=np.int64)
+    off[1:] = np.cumsum((cnt + 3) // 4 * 4)
+    dim = np.repeat(np.arange(d_in), np.diff(off))
+    ei = L.vjp_dim_off[dim] + np.minimum(np.arange(len(dim)) - off[dim], cnt[dim] - 1)
+    L.jac_row = np.stack([ei, node[ei]], axis=1).astype(np.int32) if len(dim) else \
+        np.zeros((1, 2), dtype=np.int32)
+    L.jac_row_off = off.astype(np.int32)
+    L.jac_row_end = (off[:-1] + cnt).astype(np.int32)
+    most = max(256, (8 * d_out + 15) // 16 * 16)
+    jobs, red, slots = [], [], 0
+    for z0 in range(0, d_in, JAC_GROUP):
+        a, b = int(off[z0]), int(off[min(z0 + JAC_GROUP, d_in)])
+        if b - a > most:
+            cuts = list(range(a, b, most)) + [b]
+            red.append((z0, slots, len(cuts) - 1))
+            for c0, c1 in zip(cuts[:-1], cuts[1:]):
+                jobs.append((c0, c1, z0, slots))
+                slots += 1
+        elif jobs and jobs[-1][3] < 0 and a == b:
+            continue
+        else:
+            jobs.append((a, b, z0, -1))
+    L.n_jac_jobs, L.n_jac_slots, L.n_jac_group_red = len(jobs), slots, len(red)
+    L.jac_job = np.array(jobs, dtype=np.int32)
+    L.jac_group_red = np.array(red or [(0, 0, 0)], dtype=np.int32)
 
 
 def eval_newton_layout(L: NewtonLayout, x, fp32=False):

@@ -254,3 +254,23 @@ def test_mixed_gemm_one_call_equals_steps(gpu, d, d_out, m, P):
                                           y0.data_ptr(), d_out, P, d_out, st), "contract")
     torch.cuda.synchronize()
     assert torch.equal(y0, y1)
+
+
+@pytest.mark.parametrize("d,d_out,m,P", [(3, 9, 12, 1), (10, 33, 400, 65), (17, 64, 900, 130),
+                                         (30, 9, 1500, 63)])
+def test_jacobian_rows_of_every_dim(gpu, d, d_out, m, P):
+    """Dense Jacobian of more than 8 outputs at ragged edges (points, outputs, a last group of
+    fewer than 8 dims, dims with fewer rows than a matrix step) and with dim groups shared by
+    several jobs (more than 256 rows of 9 to 33 outputs): against the exact Jacobian, and the same
+    bits for a point alone and in the batch."""
+    ref, ip, rng = make(d, d_out, m, seed=d)
+    L = ip._nlayout
+    rows = L.jac_row_off.astype(int)
+    print("rows per group of 8 dims", [int(rows[min(j + 8, d)] - rows[j]) for j in range(0, d, 8)],
+          flush=True)
+    x = rng.uniform(-1, 1, (P, d))
+    J = ip.gradient(x).cpu().numpy()
+    Je = exact_grad(ref, x)
+    assert J.shape == Je.shape and rel(J, Je) <= GRAD_TOL
+    p = P // 2
+    assert np.array_equal(ip.gradient(x[p:p + 1]).cpu().numpy()[0], J[p])
