@@ -137,6 +137,18 @@ typedef struct sbi_bary_desc {
   const double* pF;              /* F values of the records, 2 * DL per record */
   int32_t n_pseg;
   int32_t ones_row;              /* first of two table rows of 1.0 after the prefix rows */
+  /* shares for 2 to 16 outputs (sbi_bary_eval_few_f64; optional: n_share = 0): runs of entries
+   * (block, index of every factor) that need at most share_rows - 1 rows of 1D basis values */
+  int32_t n_share;
+  int32_t share_rows;            /* basis rows + 1 of the largest share (at most 320) */
+  const int32_t* share;          /* [16 * n_share] {first slot record, slot records, basis rows,
+                                    first entry, first u16 of the records, steps of four entries
+                                    with 1, 2, .. 8 factors, 0, 0, 0} */
+  const int32_t* share_slot;     /* {slot, its first row} */
+  const void* share_rec;         /* u16 basis rows of every entry's factors, share by share in step
+                                    order: 2 per entry for up to 2 factors, 4 for up to 4, else 8;
+                                    the share's row of ones fills them up and pads a step */
+  const double* share_F;         /* [entries * d_out] values in the same order (0 where padded) */
 } sbi_bary_desc;
 
 typedef struct sbi_plan sbi_plan;
@@ -152,6 +164,15 @@ int sbi_plan_destroy(sbi_plan* plan);
  * (sbi_bary_basis_f64 + a dense GEMM) evaluates such plans. */
 int sbi_bary_eval_f64(const sbi_plan* plan, const double* x, int64_t P, int64_t ldx, double* y,
                       void* stream);
+
+/* The same sum for plans with shares (2 to 16 outputs) on the FP64 matrix cores; each point's bits do
+ * not depend on the batch.  workspace: sbi_bary_eval_few_workspace bytes (0: not used; -1: invalid)
+ * of device memory, 8-byte aligned, not shared with a concurrent call; with less (or NULL) a small
+ * batch runs on fewer workgroups.  SBI_ERR_CAPACITY: the plan has no shares. */
+int64_t sbi_bary_eval_few_workspace(const sbi_plan* plan, int64_t P);
+int sbi_bary_eval_few_f64(const sbi_plan* plan, const double* x, int64_t P, int64_t ldx, double* y,
+                          void* workspace, int64_t ws_bytes, void* stream);
+
 
 /* interpolation.py:306-345 gradient with barycentric.py:126-229: dense Jacobian
  * J[P, d_out, d_in] (FP64), NaN where x_j equals a node of a slot of dim j (reference

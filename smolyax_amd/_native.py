@@ -42,6 +42,8 @@ class BaryDesc(ctypes.Structure):
         ("pseg_off", c_vp), ("pseg", c_vp), ("pbasis", c_vp), ("prow", c_vp), ("pF", c_vp),
         ("n_pseg", c_i32),
         ("ones_row", c_i32),
+        ("n_share", c_i32), ("share_rows", c_i32), ("share", c_vp), ("share_slot", c_vp),
+        ("share_rec", c_vp), ("share_F", c_vp),
     ]
 
 
@@ -95,6 +97,8 @@ SIGNATURES = {
     "sbi_bary_plan_create": (c_i32, [ctypes.POINTER(BaryDesc), ctypes.POINTER(c_vp)]),
     "sbi_plan_destroy": (c_i32, [c_vp]),
     "sbi_bary_eval_f64": (c_i32, [c_vp, c_vp, c_i64, c_i64, c_vp, c_vp]),
+    "sbi_bary_eval_few_workspace": (c_i64, [c_vp, c_i64]),
+    "sbi_bary_eval_few_f64": (c_i32, [c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_i64, c_vp]),
     "sbi_bary_jacobian_f64": (c_i32, [c_vp, c_vp, c_i64, c_i64, c_vp, c_vp]),
     "sbi_bary_integral_workspace": (c_i64, [c_vp]),
     "sbi_bary_integral_f64": (c_i32, [c_vp, c_vp, c_vp, c_vp]),

@@ -897,6 +897,12 @@ int sbi_bary_plan_create(const sbi_bary_desc* desc, sbi_plan** out) {
       return SBI_ERR_CAPACITY;
     }
   }
+  if (d.n_share < 0 || (d.n_share > 0 && (d.d_out > 16 || d.share_rows < 1 || d.share_rows > 320 ||
+                                          !d.share || !d.share_slot || !d.share_rec ||
+                                          !d.share_F || !d.slot_dim))) {
+    sbi::set_error("sbi_bary_plan_create: invalid shares (at most 16 outputs and 320 basis rows)");
+    return SBI_ERR_INVALID;
+  }
   sbi_plan* p = new sbi_plan();
   p->kind = 1;
   p->bary = d;

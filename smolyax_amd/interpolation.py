@@ -134,8 +134,7 @@ class SmolyakBarycentricInterpolator:
         self._newton_fp64_ok = self._is_nested
         self._fp64_newton = False
         self._proxy_err = None
-        self._upload()
-        self._values = None
+        self._upload(shares=not self._is_nested)
         try:
             if self._is_nested:
                 nf = newton.NewtonForm(self._k, self._t, self._node_gen, self._d_out)
@@ -150,6 +149,9 @@ class SmolyakBarycentricInterpolator:
             self._nform = self._nlayout = None
             self._newton_off = str(e)
         self._fp64_newton = self._is_nested and self._nplan is not None and self._finite_s
+        if self._is_nested and not self._fp64_newton and 2 <= self._d_out <= packing.SHARE_MAX_OUT:
+            self._upload(shares=True)
+        self._values = None
         if not self._is_nested and self._nplan is not None:
             self._check_proxy()
         self._calibrate_mixed()
@@ -282,7 +284,7 @@ class SmolyakBarycentricInterpolator:
             self._nplan = None
             self._nform = self._nlayout = None
 
-    def _upload(self):
+    def _upload(self, shares=False):
         if not torch.cuda.is_available():
             raise RuntimeError("smolyax_amd needs a HIP device (MI355X); none is visible")
         if self._device is None:
@@ -340,6 +342,19 @@ class SmolyakBarycentricInterpolator:
             N.check(N.fn["sbi_pack_rows_f64"](V.data_ptr(), len(vt.V), 1, pn.data_ptr(),
                                               ps.data_ptr(), len(prog.f_index), t["pF"].data_ptr(),
                                               ctypes.c_void_p(st.cuda_stream)), "pack_rows")
+        # entry list of the kernel for few outputs: for plans that the Newton form does not serve
+        sh = packing.build_shares(L) if 2 <= self._d_out <= packing.SHARE_MAX_OUT and shares else None
+        if sh is not None:
+            t["share"] = _dev_tensor(sh.hdr, i32, dev)
+            t["share_slot"] = _dev_tensor(sh.slot if len(sh.slot) else [0], i32, dev)
+            t["share_rec"] = torch.as_tensor(sh.rec.view(np.uint8).copy()).to(dev)
+            pn, ps = packing.program_rows(sh, vt.row_node, vt.row_scale)
+            pn, ps = _dev_tensor(pn, i32, dev), _dev_tensor(ps, f64, dev)
+            t["share_F"] = torch.empty((len(sh.f_index), self._d_out), dtype=f64, device=dev)
+            N.check(N.fn["sbi_pack_rows_f64"](V.data_ptr(), len(vt.V), self._d_out, pn.data_ptr(),
+                                              ps.data_ptr(), len(sh.f_index),
+                                              t["share_F"].data_ptr(),
+                                              ctypes.c_void_p(st.cuda_stream)), "pack_rows")
         st.synchronize()  # F is read on other streams (serving) once set_f returns
         self._dev = t
         d = N.BaryDesc()
@@ -356,6 +371,8 @@ class SmolyakBarycentricInterpolator:
             setattr(d, name, ten.data_ptr())
         d.n_split = packing.N_WAVES
         d.n_seg = int(L.seg_off[-1])
+        if sh is not None:
+            d.n_share, d.share_rows = sh.n, sh.rows
         if prog is not None:
             d.n_pseg = int(prog.seg_off[-1])
             d.ones_row = prog.ones_row
@@ -558,7 +575,13 @@ class SmolyakBarycentricInterpolator:
                 or (precision != "fp64" and self._d_out > 1))
         if not gemm:
             y = torch.empty((P, self._d_out), dtype=torch.float64, device=self._device)
-            if precision == "fp64":
+            if precision == "fp64" and self._desc.n_share:
+                ws = N.fn["sbi_bary_eval_few_workspace"](self._plan, P)
+                W = torch.empty(ws, dtype=torch.uint8, device=self._device) if ws else None
+                N.check(N.fn["sbi_bary_eval_few_f64"](self._plan, x.data_ptr(), P, x.stride(0),
+                                                      y.data_ptr(), W.data_ptr() if ws else None,
+                                                      ws, self._stream()), "eval")
+            elif precision == "fp64":
                 rc = N.fn["sbi_bary_eval_f64"](self._plan, x.data_ptr(), P, x.stride(0),
                                                y.data_ptr(), self._stream())
                 if rc == N.SBI_ERR_CAPACITY:  # prefix table too large for LDS: GEMM form

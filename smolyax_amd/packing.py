@@ -38,6 +38,14 @@ PROG_GROUP = 4           # segments per group of the eval kernel (kXGroup in bar
 PROG_MAX_GEN = 255       # per-block (generic) blocks per program segment
 PROG_MAX_COUNT = 65535   # records of one type per program segment
 PROG_MAX_ROWS = 320      # prefix table rows + 2 rows of ones, 64 points x 8 B each, in 160 KiB
+# Shares of the kernel for 2 to 16 outputs (few.hip): entries per share (about 10 us of a CU's matrix
+# work; 64 shares of 96 000 entries), basis rows per share (64 points x 8 B each in 160 KiB, with the
+# row of ones), factors per entry, header size in int32
+SHARE_ENTRIES = 1536
+SHARE_ROWS = 318
+SHARE_MAX_K = 8
+SHARE_HDR = 16
+SHARE_MAX_OUT = 16
 PROG_SGPR = 48           # SGPRs per record chunk (kProgSgpr in bary.hip)
 # Wave split of the program: per-wave cost in cycles as measured on MI355X at d_in = 1000 (one
 # scalar memory round trip per record chunk): a full chunk, a partial chunk, a segment start
@@ -666,6 +674,102 @@ def build_eval_program(L: Layout):
                        basis=np.array(basis).reshape(-1) if basis else np.zeros(PROG_BASIS),
                        rows=np.array(rows or [0], dtype=np.int32),
                        f_index=np.array(fidx or [0], dtype=np.int64), n_records=nrec, ones_row=ones)
+
+
+@dataclass
+class Shares:
+    """Entry list of the kernel for 2 to 16 outputs (see build_shares)."""
+    hdr: np.ndarray       # [n * SHARE_HDR] int32 share headers
+    slot: np.ndarray      # [2 * records] int32 {slot, first row of the share's table}
+    rec: np.ndarray       # uint16 basis rows of the entries' factors
+    f_index: np.ndarray   # int64: position of every entry in the flat device F (-1: padding)
+    n: int
+    rows: int             # table rows of the largest share, its row of ones included
+
+
+def share_stride(k: int) -> int:
+    """Basis rows stored per entry of k factors."""
+    return 2 if k <= 2 else 4 if k <= 4 else 8
+
+
+def build_shares(L: Layout):
+    """The entries (block, index of every factor) of all blocks in shares: runs of blocks in device
+    order of about SHARE_ENTRIES entries (a larger block is a share of its own) whose slots need at
+    most SHARE_ROWS basis rows; in a share the entries by factor count, padded to steps of four
+    with rows of ones and zero values.  None if a block does not fit (factors, rows) or there are
+    none."""
+    nb = len(L.blk_n)
+    fac, fo = L.fac_slot, L.blk_fac
+    size = (L.slot_deg + 1).tolist()
+    foff = L.blk_foff
+    slots_of = []
+    for b in range(nb):
+        sl = fac[fo[b]: fo[b + 1]].tolist()
+        if L.blk_last_slot[b] >= 0:
+            sl.append(int(L.blk_last_slot[b]))
+        if len(sl) > SHARE_MAX_K or sum(size[s] for s in set(sl)) > SHARE_ROWS:
+            return None
+        slots_of.append(sl)
+    cuts, used, rows, ents = [0], set(), 0, 0
+    for b in range(nb):
+        n = int(foff[b + 1] - foff[b])
+        new = set(slots_of[b]) - used
+        add = sum(size[s] for s in new)
+        if b > cuts[-1] and (ents + n > SHARE_ENTRIES or rows + add > SHARE_ROWS):
+            cuts.append(b)
+            used, rows, ents = set(), 0, 0
+            new = set(slots_of[b])
+            add = sum(size[s] for s in new)
+        used |= new
+        rows += add
+        ents += n
+    if nb:
+        cuts.append(nb)
+    hdr, slot, rec, f_index = [], [], [], []
+    n_slot = n_rec = n_ent = most = 0
+    row_of = np.zeros(max(len(size), 1), dtype=np.int64)
+    size = np.asarray(size or [1], dtype=np.int64)
+    for b0, b1 in zip(cuts[:-1], cuts[1:]):
+        own = np.array(sorted({s for sl in slots_of[b0:b1] for s in sl}), dtype=np.int64)
+        first = np.concatenate([[0], np.cumsum(size[own])]) if len(own) else np.zeros(1, np.int64)
+        ones = int(first[-1])
+        row_of[own] = first[:-1]
+        h = [n_slot, len(own), ones, n_ent, n_rec]
+        slot.append(np.stack([own, first[:-1]], axis=1))
+        n_slot += len(own)
+        most = max(most, ones + 1)
+        by_k = {}
+        for b in range(b0, b1):
+            by_k.setdefault(max(len(slots_of[b]), 1), []).append(b)
+        for k in range(1, SHARE_MAX_K + 1):
+            bl = by_k.get(k, [])
+            if not bl:
+                h.append(0)
+                continue
+            sl = np.array([slots_of[b] for b in bl], dtype=np.int64).reshape(len(bl), -1)
+            cnt = foff[np.array(bl) + 1] - foff[np.array(bl)]
+            rep = np.repeat(np.arange(len(bl)), cnt)
+            e = np.arange(len(rep)) - np.repeat(np.cumsum(cnt) - cnt, cnt)
+            n4 = (len(rep) + 3) // 4 * 4
+            r = np.full((n4, share_stride(k)), ones, dtype=np.uint16)
+            rem = e.copy()
+            for i in range(sl.shape[1] - 1, -1, -1):  # C order: the last factor fastest
+                m = size[sl[rep, i]]
+                r[: len(rep), i] = row_of[sl[rep, i]] + rem % m
+                rem //= m
+            fi = np.full(n4, -1, dtype=np.int64)
+            fi[: len(rep)] = foff[np.array(bl)][rep] + e
+            h.append(n4 // 4)
+            rec.append(r.reshape(-1))
+            f_index.append(fi)
+            n_rec += r.size
+            n_ent += n4
+        hdr.append(h + [0] * (SHARE_HDR - len(h)))
+    if not hdr or n_rec >= 2**31:
+        return None
+    return Shares(hdr=np.array(hdr, dtype=np.int32).reshape(-1),
+                  slot=np.concatenate(slot).astype(np.int32).reshape(-1),
+                  rec=np.concatenate(rec), f_index=np.concatenate(f_index), n=len(hdr), rows=most)
 
 
 def program_values(prog: EvalProgram, F: np.ndarray) -> np.ndarray:

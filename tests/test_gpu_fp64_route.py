@@ -47,6 +47,14 @@ def technique(ip, x):
     if ip.d_out >= 16:
         return ip._eval_bary_gemm(xt)
     y = torch.empty((xt.shape[0], ip.d_out), dtype=torch.float64, device="cuda")
+    if ip._desc.n_share:  # 2 to 16 outputs on a plan without a Newton form in FP64
+        nb = N.fn["sbi_bary_eval_few_workspace"](ip._plan, xt.shape[0])
+        W = torch.empty(max(nb, 8), dtype=torch.uint8, device="cuda")
+        N.check(N.fn["sbi_bary_eval_few_f64"](ip._plan, xt.data_ptr(), xt.shape[0], xt.stride(0),
+                                              y.data_ptr(), W.data_ptr(), nb,
+                                              ctypes.c_void_p(None)), "eval")
+        torch.cuda.synchronize()
+        return y
     N.check(N.fn["sbi_bary_eval_f64"](ip._plan, xt.data_ptr(), xt.shape[0], xt.stride(0),
                                       y.data_ptr(), ctypes.c_void_p(None)), "eval")
     torch.cuda.synchronize()

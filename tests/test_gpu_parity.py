@@ -376,3 +376,58 @@ def test_eval_record_program(gpu, d, m, kind, kscale):
     e_blk = rel(y0.cpu().numpy(), y_ex)
     print(f"  per-block kernel {e_blk:.2e}", flush=True)
     assert e_blk <= max(4.0 * e_ora, 1e-14)
+
+
+@pytest.mark.parametrize("d,m,kind,kscale,d_out,P", [(1, 22, "gh", 1.0, 2, 1), (5, 300, "gh", 1.0, 3, 65),
+                                                     (8, 3000, "leja", 0.3, 15, 70),
+                                                     (40, 3000, "gh", 1.0, 10, 500),
+                                                     (300, 2000, "gh", 1.0, 5, 130)])
+def test_eval_few_outputs(gpu, d, m, kind, kscale, d_out, P):
+    """2 to 16 outputs on plans without a Newton form in FP64: the share kernel through the C ABI
+    against the exact interpolant of the FP64 data (within 4x the FP64 oracle's own distance, the
+    bound of every combination-technique kernel), with and without its workspace (the same bits),
+    a point alone and in the batch (the same bits), points on nodes, a partial last tile."""
+    import ctypes
+
+    import torch
+
+    from smolyax_amd import _native as N
+    from smolyax_amd import nodes as SN
+    from smolyax_amd.interpolation import SmolyakBarycentricInterpolator
+
+    k = kscale * np.log((2 + np.arange(d)) / np.log(2))
+    ong, sng = (ON.leja(dim=d), SN.Leja(dim=d)) if kind == "leja" else \
+        (ON.gauss_hermite(dim=d), SN.GaussHermite(dim=d))
+    t = OI.find_approximate_threshold(k, m, ong.is_nested)
+    A = np.random.default_rng(d + m).standard_normal((d_out, d)) / (np.arange(d) + 1.0)
+    f = lambda x: np.cos(A @ x + 0.2)
+    ref = OS.Interpolant(d_out=d_out, node_gen=ong, k=k, t=t, f=f)
+    ip = SmolyakBarycentricInterpolator(d_out=d_out, node_gen=sng, k=k, t=t, f=f)
+    if not ip._desc.n_share:  # (served by the Newton form: build the share list all the same)
+        from smolyax_amd import packing
+
+        L = ip._layout
+        vt = packing.gather_values(L, packing.nonzero_blocks(k, t), sng, f, {}, False)
+        ip._values = vt
+        ip._upload(shares=True)
+    print(f"{kind} d={d}: {ip._desc.n_share} shares of at most {ip._desc.share_rows} rows", flush=True)
+    x = sample(ong, P, seed=m)
+    x[0, 0] = ong[0](2)[1]
+    xt = torch.as_tensor(x, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def run(xx, ws=True):
+        y = torch.full((len(xx), d_out), float("nan"), dtype=torch.float64, device="cuda")
+        nb = N.fn["sbi_bary_eval_few_workspace"](ip._plan, len(xx)) if ws else 0
+        W = torch.empty(max(nb, 8), dtype=torch.uint8, device="cuda")
+        N.check(N.fn["sbi_bary_eval_few_f64"](ip._plan, xx.data_ptr(), len(xx), xx.stride(0),
+                                              y.data_ptr(), W.data_ptr(), nb, st), "few")
+        return y
+
+    y = run(xt)
+    assert torch.equal(y, run(xt, ws=False))
+    p = P // 2
+    assert torch.equal(run(xt[p:p + 1])[0], y[p])
+    nx = min(P, 64)
+    ye = ref(x[:nx], dtype=np.longdouble).astype(np.float64)
+    assert rel(y[:nx].cpu().numpy(), ye) <= max(4.0 * rel(ref(x[:nx]), ye), 1e-14)

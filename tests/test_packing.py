@@ -160,3 +160,51 @@ def test_eval_program_matches_layout(kind, d, m, kscale):
     npre = np.diff(L.blk_fac)
     print(f"{kind} d={d}: {prog.n_records} records, {n_gen} per-block blocks "
           f"(of {len(L.blk_n)}; max prefix factors {npre.max()})")
+
+
+@pytest.mark.parametrize("kind,d,m,kscale,entries", [("gh", 1, 22, 1.0, 1536), ("gh", 6, 300, 1.0, 64),
+                                                     ("leja", 8, 900, 0.3, 200), ("gh", 40, 600, 1.0, 500),
+                                                     ("leja", 3, 2, 1.0, 1536)])
+def test_shares_hold_every_entry_once(monkeypatch, kind, d, m, kscale, entries):
+    """The share list (few-output kernel) on the CPU: every F row is used once, each entry's factor
+    rows give the layout's weight, padding has value zero and rows of ones, and table rows and
+    steps stay within the limits that the kernel assumes."""
+    from smolyax_amd import nodes as SN
+    from smolyax_amd import packing
+
+    monkeypatch.setattr(packing, "SHARE_ENTRIES", entries)
+    k = kscale * np.log((2 + np.arange(d)) / np.log(2))
+    gen = SN.Leja(dim=d) if kind == "leja" else SN.GaussHermite(dim=d)
+    t = OI.find_approximate_threshold(k, m, gen.is_nested)
+    L = packing.build_layout(packing.nonzero_blocks(k, t), gen, d, 3)
+    S = packing.build_shares(L)
+    assert S is not None and S.rows <= 320 and S.rec.max() < S.rows
+    rng = np.random.default_rng(d)
+    x = rng.uniform(-0.9, 0.9, (7, d))
+    F = rng.standard_normal((L.k_raw, 3))
+    used = np.zeros(L.k_raw, dtype=int)
+    y = np.zeros((7, 3))
+    hdr = S.hdr.reshape(S.n, packing.SHARE_HDR)
+    slot = S.slot.reshape(-1, 2)
+    for h in hdr:
+        tab = np.full((h[2] + 1, 7), np.nan)
+        tab[h[2]] = 1.0
+        for s, r in slot[h[0]: h[0] + h[1]]:
+            g = L.slot_deg[s]
+            tab[r: r + g + 1] = layout_eval.first_form_basis(
+                x[:, L.slot_dim[s]], L.slot_nodes[s, : g + 1], L.slot_w[s, : g + 1]).T
+        assert not np.isnan(tab).any()
+        rec, ent = int(h[4]), int(h[3])
+        assert rec % 8 == 0
+        for kk in range(1, packing.SHARE_MAX_K + 1):
+            n, st = int(h[4 + kk]) * 4, packing.share_stride(kk)
+            rows = S.rec[rec: rec + n * st].reshape(n, st)
+            assert (rows[:, kk:] == h[2]).all()
+            fi = S.f_index[ent: ent + n]
+            used += np.bincount(fi[fi >= 0], minlength=L.k_raw)
+            w = tab[rows[:, :kk]].prod(axis=1)
+            y += w.T @ np.where(fi[:, None] >= 0, F[np.maximum(fi, 0)], 0.0)
+            rec, ent = rec + n * st, ent + n
+    assert (used == 1).all()
+    ref = layout_eval.eval_layout(L, F, np.zeros(3), x)
+    assert np.max(np.abs(y - ref)) <= 1e-12 * max(1.0, np.abs(F).sum())
