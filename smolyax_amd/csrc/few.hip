@@ -7,15 +7,16 @@
 // entries, made here and never stored) with F on v_mfma_f64_16x16x4: 64 cycles of a SIMD per 4
 // entries x 16 points x 16 outputs, beside 1 to 8 LDS reads and products per 64 weights.
 //
-// The host cuts the list into shares of about 1500 entries whose factors need at most kFewRows rows
-// of 1D basis values; a workgroup of 16 waves takes 64 points and one or more shares, one after
+// The host cuts the list into shares of about 1500 entries whose factors need at most 318 rows
+// of 1D basis values; a workgroup of 8 waves (two per CU) takes 64 points and one or more shares, one after
 // another: the share's basis rows for the 64 points in LDS, the entries in steps of four (one per
 // lane group) dealt over the waves, the waves' sums added in wave order.  When the 64-point tiles
 // are few, the shares are spread over workgroups that write their sums to a workspace, and a second
 // kernel adds them in share order: the same bits for any batch.
 //
 // 500 points x 40 inputs x 10 outputs, 95 956 entries: 1830 us for one workgroup per 64 points and 4
-// outputs walking the blocks through scalar loads, FEWUS us here (matrix cores alone: 20 us).
+// outputs walking the blocks through scalar loads, 55 us here (matrix cores alone: 20 us); with 8-byte
+// reads of the basis rows 73 us (LDS-bound), one workgroup of 16 waves 60 us, four of 4 waves 65 us.
 
 #include <hip/hip_runtime.h>
 
@@ -29,7 +30,7 @@
 namespace {
 
 constexpr int kTile = 64;    // points per workgroup
-constexpr int kWaves = 16;
+constexpr int kWaves = 8;
 constexpr int kOut = 16;     // outputs of a matrix fragment
 constexpr int kHdr = 16;     // int32 per share header
 constexpr int kSlotBatch = 4;  // slots per wave whose coordinates are requested together
@@ -69,16 +70,17 @@ __device__ __forceinline__ void basis_rows(double x, cptr<double> xi, cptr<doubl
 constexpr int rec_stride(int K) { return K <= 2 ? 2 : K <= 4 ? 4 : 8; }
 
 // The steps of a share whose entries have K factors: step s holds entries 4 s + g for lane group g.
-// Lane (li, g) computes the weights of its entry at points 16 f + li of the four fragments f.  Odd
-// lane groups read the fragments of a pair in swapped order, so that the two groups that half a
-// wave reads together lie in different halves of the LDS banks (every row starts at bank 0).
+// Lane (li, g) computes the weights of its entry at the points 32 h + 2 li + c of the four fragments
+// f = 2 h + c, two neighbouring points per 16-byte LDS read (a lane group reads 256 contiguous
+// bytes of a row: no bank conflicts whatever the rows).
 template <int K>
 __device__ __forceinline__ void run_steps(int n, const uint16_t* __restrict__ rec,
                                           const double* __restrict__ F, int64_t d_out, int wave,
                                           int lane, const lds_f64* tab, v4d (&acc)[4]) {
   constexpr int R = rec_stride(K);
   const int li = lane & 15, g = lane >> 4;
-  const bool odd = g & 1;
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(3))) v2d lds_v2d;
   const double* __restrict__ Fl = F + (int64_t)g * d_out + min((int64_t)li, d_out - 1);
   uint32_t rw[R / 2];
   double b = 0.0;
@@ -94,26 +96,26 @@ __device__ __forceinline__ void run_steps(int n, const uint16_t* __restrict__ re
 #pragma unroll
     for (int i = 0; i < K; ++i) {
       const uint32_t r = i & 1 ? rw[i >> 1] >> 16 : rw[i >> 1] & 0xffff;
-      off[i] = (int)r * kTile + (odd ? 16 : 0) + li;
+      off[i] = (int)r * kTile + 2 * li;
     }
     const double bs = b;
     if (s + kWaves < n) fetch(s + kWaves);
 #pragma unroll
-    for (int pr = 0; pr < 2; ++pr) {
-      double u = tab[off[0] + 32 * pr], v = tab[(off[0] ^ 16) + 32 * pr];
+    for (int h = 0; h < 2; ++h) {
+      v2d u = *(const lds_v2d*)(tab + off[0] + 32 * h);
 #pragma unroll
       for (int i = 1; i < K; ++i) {
-        u *= tab[off[i] + 32 * pr];
-        v *= tab[(off[i] ^ 16) + 32 * pr];
+        const v2d t = *(const lds_v2d*)(tab + off[i] + 32 * h);
+        u.x *= t.x;
+        u.y *= t.y;
       }
-      acc[2 * pr] = __builtin_amdgcn_mfma_f64_16x16x4f64(odd ? v : u, bs, acc[2 * pr], 0, 0, 0);
-      acc[2 * pr + 1] =
-          __builtin_amdgcn_mfma_f64_16x16x4f64(odd ? u : v, bs, acc[2 * pr + 1], 0, 0, 0);
+      acc[2 * h] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.x, bs, acc[2 * h], 0, 0, 0);
+      acc[2 * h + 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.y, bs, acc[2 * h + 1], 0, 0, 0);
     }
   }
 }
 
-__global__ __launch_bounds__(kTile* kWaves) void bary_few_kernel(sbi_bary_desc d,
+__global__ __launch_bounds__(kTile* kWaves, 4) void bary_few_kernel(sbi_bary_desc d,
                                                                 const double* __restrict__ x,
                                                                 int64_t P, int64_t ldx,
                                                                 double* __restrict__ y,
@@ -130,8 +132,10 @@ __global__ __launch_bounds__(kTile* kWaves) void bary_few_kernel(sbi_bary_desc d
   // this thread's element of the tile after the waves' sums are added: point tid / 16, output tid % 16
   const int64_t prow = (int64_t)blockIdx.x * kTile + (threadIdx.x >> 4);
   const int pcol = threadIdx.x & 15;
-  const bool mine = prow < P && pcol < n;
-  double total = 0.0;
+  constexpr int kE = 16 / kWaves;  // elements per thread: points prow + 4 kWaves i
+  double total[kE];
+#pragma unroll
+  for (int i = 0; i < kE; ++i) total[i] = 0.0;
 
   for (int sh = sh0; sh < sh1; ++sh) {
     cptr<int32_t> h = C(d.share) + (int64_t)sh * kHdr;
@@ -175,24 +179,30 @@ __global__ __launch_bounds__(kTile* kWaves) void bary_few_kernel(sbi_bary_desc d
     SBI_STEPS(5) SBI_STEPS(6) SBI_STEPS(7) SBI_STEPS(8)
 #undef SBI_STEPS
     __syncthreads();  // the table is done with
-    // result layout: register r of lane group g holds point g + 4 r of the fragment, output li
+    // result layout: register r of lane group g holds row g + 4 r of the fragment, output li
     const int li = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int f = 0; f < 4; ++f)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        tab[(wave * kTile + 16 * f + g + 4 * r) * kOut + li] = acc[f][r];
+        tab[(wave * kTile + 32 * (f >> 1) + 2 * (g + 4 * r) + (f & 1)) * kOut + li] = acc[f][r];
     __syncthreads();
-    double s = 0.0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) s += tab[w * kTile * kOut + threadIdx.x];
-    if (part) {
-      if (mine) part[((int64_t)sh * P + prow) * n + pcol] = s;
-    } else {
-      total += s;
+    for (int i = 0; i < kE; ++i) {
+      const int64_t row = prow + 4 * kWaves * i;
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w)
+        s += tab[w * kTile * kOut + kTile * kWaves * i + threadIdx.x];
+      if (!part) total[i] += s;
+      else if (row < P && pcol < n) part[((int64_t)sh * P + row) * n + pcol] = s;
     }
   }
-  if (!part && mine) y[prow * n + pcol] = d.offset[pcol] + total;
+#pragma unroll
+  for (int i = 0; i < kE; ++i) {
+    const int64_t row = prow + 4 * kWaves * i;
+    if (!part && row < P && pcol < n) y[row * n + pcol] = d.offset[pcol] + total[i];
+  }
 }
 
 // y = offset + the shares' sums in share order.
