@@ -321,6 +321,21 @@ typedef struct sbi_newton_desc {
                                  rows (slot 0 .. n_jac_slots - 1) */
   const int32_t* jac_group_red; /* [3 * n_jac_group_red] {first dim, first slot, slots} of the
                                  groups in several parts */
+  /* register pass of the Jacobian (d_out <= 8) and the adjoint with the factor table in LDS
+   * (optional: n_jt_blocks = 0 selects the pass over jac_unit).  A unit is a run of at most 64
+   * entries of one factor row; 16 units of about one length, the longest first, are a block, whose
+   * records lie step by step; a dim of several units adds their sums in slot order */
+  int32_t n_jt_blocks;
+  int32_t n_jt_slots;
+  int32_t n_jt_red;
+  int32_t _pad8;
+  const void* jt_ent;         /* [steps of all blocks + 8][16 units] 16 bytes {node | factors of the
+                                 step << 24, six 16-bit factor rows, n_tab_rows where there is none} */
+  const int32_t* jt_unit;     /* [4 * 16 * n_jt_blocks] {dim | degree << 16, first step of the block,
+                                 entries, slot or ~i (the unit is all of table dim i)} */
+  const int32_t* jt_dim;      /* [4 * n_tab_dims] {dim, first row, largest degree | count << 16, first
+                                 singular coordinate (sing_x)} */
+  const int32_t* jt_red;      /* [3 * n_jt_red] {dim, first slot, slot count} */
 } sbi_newton_desc;
 
 typedef struct sbi_newton_plan sbi_newton_plan;

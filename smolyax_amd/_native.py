@@ -73,6 +73,8 @@ class NewtonDesc(ctypes.Structure):
         ("n_jac_jobs", c_i32), ("n_jac_slots", c_i32), ("n_jac_group_red", c_i32), ("_pad7", c_i32),
         ("jac_row", c_vp), ("jac_row_off", c_vp), ("jac_row_end", c_vp), ("jac_job", c_vp),
         ("jac_group_red", c_vp),
+        ("n_jt_blocks", c_i32), ("n_jt_slots", c_i32), ("n_jt_red", c_i32), ("_pad8", c_i32),
+        ("jt_ent", c_vp), ("jt_unit", c_vp), ("jt_dim", c_vp), ("jt_red", c_vp),
     ]
 
 

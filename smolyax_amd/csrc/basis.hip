@@ -539,21 +539,248 @@ __global__ __launch_bounds__(kTile* kBWaves) void newton_jac_kernel(
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// The Jacobian's register pass with the factor table of 16 points in LDS.  A unit is a run of at
+// most 64 entries of one factor row (j, k), so h'_k(x_j) multiplies its sum once; a wave takes 16
+// units of about one length side by side: 4 lanes per unit, four points per lane, one entry of each
+// unit per step, nothing reduced across lanes.  Decoding an entry costs 20-odd instructions and
+// serves 16 points; the pass above decodes per 64 points in scalar registers, but reads every
+// factor from L2.  Records lie step by step (one 256-byte read per step, no address arithmetic); a
+// step's coefficients are requested one step (of U entries) ahead, its records two.  Bound by LDS
+// reads and VALU issue.
+// 4096 points x 1000 inputs, 22 097 entries: 66 us and 7 us for the reduction, against 118 + 26 us
+// for the factor table in global memory and 9.5 us.  (8 lanes per unit: 103 us; units one after
+// another, 8 lanes by entry: 251 us, a chain of loads per unit.)  The adjoint keeps the pass above:
+// its 2.3 reads of G per node bound it (220 us here against 199 + 16 us; 8192 points x 200 inputs).
+// ------------------------------------------------------------------------------------------
+constexpr int kJTile = 16;  // points per workgroup
+
+inline size_t jac_tile_lds(const sbi_newton_desc& d) {
+  return (size_t)(d.n_tab_rows + 1) * kJTile * sizeof(double) + ((size_t)d.n_tab_dims * 2 + 15) / 16 * 16;
+}
+
+constexpr int jac_tile_max_waves(int no) { return no <= 2 ? 16 : 8; }
+
+template <int NO>
+__global__ __launch_bounds__(64 * jac_tile_max_waves(NO)) void newton_jac_tile_kernel(
+    sbi_newton_desc d, const double* __restrict__ x, int64_t P, int64_t ldx,
+    const double* __restrict__ S, int64_t lds, int n, double* __restrict__ J,
+    double* __restrict__ part) {
+  extern __shared__ double lds_raw[];
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  typedef typename lds_t<double>::type LT;
+  typedef __attribute__((address_space(3))) v2d LV;
+  typedef __attribute__((address_space(3))) uint16_t LM;
+  constexpr int U = NO <= 2 ? 2 : 1;  // entries of a unit whose loads go out together
+  LT* tab = (LT*)lds_raw;
+  LM* on_node_mask = (LM*)(tab + (d.n_tab_rows + 1) * kJTile);  // [table dim], bit = point
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int waves = blockDim.x >> 6;
+  const int64_t tile0 = (int64_t)blockIdx.x * kJTile;
+
+  // 1. factor table [row][point], four dims x 16 points per wave step; the row of ones after it
+  {
+    const int pp = lane & 15;
+    const double* __restrict__ xp = x + min(tile0 + pp, P - 1) * ldx;
+    const int4* __restrict__ dim = reinterpret_cast<const int4*>(d.jt_dim);
+    constexpr int kB = 4;  // steps whose loads are requested together
+    const int last = d.n_tab_dims - 1, step = waves * 4;
+    for (int i0 = wave * 4 + (lane >> 4); i0 - (lane >> 4) <= last; i0 += step * kB) {
+      int4 r[kB];  // {dim, first row, largest degree | singular coordinates << 16, the first of them}
+      double xv[kB], x0[kB], c1[kB], s0[kB], s1[kB];
+#pragma unroll
+      for (int u = 0; u < kB; ++u) r[u] = dim[min(i0 + u * step, last)];
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        xv[u] = xp[r[u].x];
+        x0[u] = d.dim_xi[(int64_t)r[u].x * d.kmax1];
+        c1[u] = d.dim_c[(int64_t)r[u].x * d.kmax1 + 1];
+        s0[u] = d.sing_x[r[u].w];
+        s1[u] = d.sing_x[r[u].w + ((uint32_t)r[u].z >> 17 ? 1 : 0)];
+      }
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        const int i = i0 + u * step, row = r[u].y, km = r[u].z & 0xffff;
+        const int ns = (int)((uint32_t)r[u].z >> 16);
+        const bool live = i <= last;
+        if (live) {
+          double pr = xv[u] - x0[u];
+          tab[row * kJTile + pp] = pr * c1[u];
+          const double* __restrict__ xi = d.dim_xi + (int64_t)r[u].x * d.kmax1;
+          const double* __restrict__ c = d.dim_c + (int64_t)r[u].x * d.kmax1;
+          for (int k = 2; k <= km; ++k) {
+            pr *= xv[u] - xi[k - 1];
+            tab[(row + k - 1) * kJTile + pp] = pr * c[k];
+          }
+        }
+        const double d0 = xv[u] - s0[u], d1 = xv[u] - s1[u];
+        bool on = ns > 0 && (d0 * d0 == 0.0 || d1 * d1 == 0.0);
+        for (int q = 2; q < ns; ++q) {
+          const double dq = xv[u] - d.sing_x[r[u].w + q];
+          on |= dq * dq == 0.0;
+        }
+        const uint64_t m = __ballot(on);
+        if (live && pp == 0) on_node_mask[i] = (uint16_t)(m >> (lane & 48));
+      }
+    }
+    if (threadIdx.x < kJTile) tab[d.n_tab_rows * kJTile + threadIdx.x] = 1.0;
+  }
+  __syncthreads();
+
+  // 2. units, 16 side by side: 4 lanes each, two pairs of points per lane.  Neighbouring units read
+  // opposite halves of their rows first, so that the 8 lanes of one LDS pass hit different banks.
+  const int pl = lane & 3, sub = lane >> 2;
+  const int q0 = 2 * pl + ((sub & 1) ? 8 : 0), q1 = q0 ^ 8;  // first points of the pairs
+  int64_t pt[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) pt[q] = min(tile0 + (q < 2 ? q0 : q1) + (q & 1), P - 1);
+  const LT* ta = tab + q0;
+  const LT* tb = tab + q1;
+  const uint4* __restrict__ ent = reinterpret_cast<const uint4*>(d.jt_ent) + sub;
+  const int4* __restrict__ unit = reinterpret_cast<const int4*>(d.jt_unit) + sub;
+  const int nb = d.n_jt_blocks, stride = (int)gridDim.y * waves;
+  // records [step][16 units] (16 bytes: node | factors of the step << 24, rows of the factors);
+  // reading ahead of the last block ends in the table's padding
+  auto records = [&](uint4(&r)[U], int step) {
+#pragma unroll
+    for (int i = 0; i < U; ++i) r[i] = ent[(int64_t)(step + i) * 16];
+  };
+  double ca[U * NO];
+  auto coefficients = [&](const uint4(&r)[U]) {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const double* __restrict__ Sn = S + (uint64_t)(r[i].x & 0xffffff) * (uint32_t)lds;
+#pragma unroll
+      for (int o = 0; o < NO; ++o) ca[i * NO + o] = o < n ? Sn[o] : 0.0;
+    }
+  };
+  int b = (int)blockIdx.y * waves + wave;
+  if (b >= nb) return;
+  // {dim | degree << 16, first step of the block, entries, slot or ~table dim}; the unit two blocks
+  // ahead and the first records of the next block are requested before the entries of this one
+  int4 un = unit[b * 16], un1 = unit[min(b + stride, nb - 1) * 16];
+  uint4 rf[U];
+  records(rf, __builtin_amdgcn_readfirstlane(un.y));
+  for (; b < nb; b += stride) {
+    const int first = __builtin_amdgcn_readfirstlane(un.y);
+    const int steps = __builtin_amdgcn_readfirstlane(un.z);  // the first unit is the longest
+    uint4 rc[U], rn[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) rc[i] = rf[i];
+    coefficients(rc);
+    records(rn, first + U);
+    records(rf, __builtin_amdgcn_readfirstlane(un1.y));
+    const int4 un2 = unit[min(b + 2 * stride, nb - 1) * 16];
+    const int j = un.x & 0xffff, k = (int)((uint32_t)un.x >> 16), len = un.z;
+    const double c = d.dim_c[(int64_t)j * d.kmax1 + k];
+    double g[4 * NO];
+#pragma unroll
+    for (int o = 0; o < 4 * NO; ++o) g[o] = 0.0;
+    for (int t = 0; t < steps; t += U) {
+      uint4 e[U];
+      double f[U * NO];
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        e[i] = rc[i];
+        rc[i] = rn[i];
+      }
+#pragma unroll
+      for (int i = 0; i < U * NO; ++i) f[i] = ca[i];
+      coefficients(rc);
+      records(rn, first + t + 2 * U);
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        // the other factors (the row of ones where a unit has fewer than the step)
+        const uint32_t nf = (uint32_t)__builtin_amdgcn_readfirstlane((int)e[i].x) >> 24;
+        const int r0 = (int)(e[i].y & 0xffff) * kJTile;
+        v2d va = *(const LV*)(ta + r0), vb = *(const LV*)(tb + r0);
+#pragma unroll
+        for (uint32_t h = 1; h < 6; ++h) {
+          if (nf <= h) break;
+          const uint32_t w = h < 2 ? e[i].y : h < 4 ? e[i].z : e[i].w;
+          const int r = (int)(h & 1 ? w >> 16 : w & 0xffff) * kJTile;
+          va *= *(const LV*)(ta + r);
+          vb *= *(const LV*)(tb + r);
+        }
+        if (t + i < len) {
+          const double v[4] = {va.x, va.y, vb.x, vb.y};
+#pragma unroll
+          for (int o = 0; o < NO; ++o)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              g[4 * o + q] = fma(v[q], f[i * NO + o], g[4 * o + q]);
+        }
+      }
+    }
+    // times h'_k(x_j), a constant for k = 1; Jacobian: NaN at node coordinates
+    double dv[4] = {c, c, c, c};
+    if (__any(k > 1)) {
+      const double* __restrict__ xi = d.dim_xi + (int64_t)j * d.kmax1;
+      double xq[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) xq[q] = x[pt[q] * ldx + j];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        double pr = 1.0, dp = 0.0;
+        for (int r = 0; r < k; ++r) {
+          const double tv = xq[q] - xi[r];
+          dp = dp * tv + pr;
+          pr *= tv;
+        }
+        dv[q] = dp * c;
+      }
+    }
+    uint32_t on = 0;
+    if (un.w < 0) on = (uint32_t)on_node_mask[~un.w];
+    if (len > 0) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int pq = (q < 2 ? q0 : q1) + (q & 1);
+        const int64_t p = tile0 + pq;
+        if (p < P) {
+#pragma unroll
+          for (int o = 0; o < NO; ++o) {
+            double v = g[4 * o + q] * dv[q];
+            if ((on >> pq) & 1) v = NAN;
+            if (o < n) {
+              if (un.w < 0) J[(p * n + o) * d.d_in + j] = v;
+              else part[((int64_t)un.w * P + p) * n + o] = v;
+            }
+          }
+        }
+      }
+    }
+    un = un1;
+    un1 = un2;
+  }
+}
+
 // J[p, o, j] = sum of the partial sums of dim j's units, in unit order (with x: the Jacobian,
 // NaN at node coordinates; without: the adjoint).
-__global__ __launch_bounds__(256) void jac_reduce_kernel(sbi_newton_desc d, int64_t P, int64_t n,
+__global__ __launch_bounds__(256) void jac_reduce_kernel(sbi_newton_desc d,
+                                                        const int32_t* __restrict__ redv,
+                                                        int64_t P, int64_t n,
                                                         const double* __restrict__ part,
                                                         double* __restrict__ J,
                                                         const double* __restrict__ x, int64_t ldx) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (p >= P) return;
-  cptr<int32_t> red = C(d.jac_red);
+  cptr<int32_t> red = C(redv);
   const int r = blockIdx.y;
   const int j = red[3 * r], s0 = red[3 * r + 1], ns = red[3 * r + 2];
   const bool nan_here = x && on_node(d, x[p * ldx + j], j);
   for (int64_t o = 0; o < n; ++o) {
     double acc = 0.0;
-    for (int u = 0; u < ns; ++u) acc += part[((int64_t)(s0 + u) * P + p) * n + o];
+    int u = 0;
+    for (; u + 8 <= ns; u += 8) {  // eight loads in flight, added in slot order
+      double v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = part[((int64_t)(s0 + u + i) * P + p) * n + o];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc += v[i];
+    }
+    for (; u < ns; ++u) acc += part[((int64_t)(s0 + u) * P + p) * n + o];
     J[(p * n + o) * d.d_in + j] = nan_here ? NAN : acc;
   }
 }
@@ -895,6 +1122,42 @@ extern "C" int sbi_newton_eval_mixed_gemm(const sbi_newton_plan* plan, const dou
 
 static bool jac_global_table(const sbi_newton_desc& d);
 
+constexpr int kJacDirectMax = 8;  // outputs handled in one register pass
+
+// Waves per workgroup of newton_jac_tile_kernel (0: its table does not fit LDS, or the plan has no
+// units for it): 16 where one workgroup fits a CU, fewer where several do (16 waves per CU).  The
+// kernel multiplies row numbers by 32-bit strides: from 16 rows on, a longer stride exceeds the
+// card's 288 GB.  5..8 outputs take 240 registers, so that small tables gain nothing from LDS:
+// 4096 points x 200 inputs x 8 outputs (249 rows) 179 us against 153 us by the other pass, 1000
+// inputs (1058 rows) 409 us against 573 us; 4 outputs: 98 against 104 us, 198 against 284 us.
+static int jac_tile_waves(const sbi_newton_desc& d, int64_t n) {
+  if (!d.jt_unit || d.n_jt_blocks <= 0 || d.basis_n < 16 || n > kJacDirectMax) return 0;
+  for (int waves : {4, 8, 16})
+    if (jac_tile_lds(d) <= (size_t)kMaxLds * waves / 16) return n > 4 && waves < 16 ? 0 : waves;
+  return 0;
+}
+
+template <int NO>
+static int jac_tile_launch(const sbi_newton_desc& d, const double* x, int64_t P, int64_t ldx,
+                           const double* S, int64_t lds, int n, double* J, double* part,
+                           hipStream_t st) {
+  sbi::allow_lds((const void*)newton_jac_tile_kernel<NO>);
+  const int waves = std::min(jac_tile_waves(d, n), jac_tile_max_waves(NO));
+  const int64_t tiles = (P + kJTile - 1) / kJTile;
+  // workgroups per tile: enough for every CU's 16 waves, at most a block of units per wave
+  const int64_t ny = std::max<int64_t>(
+      1, std::min<int64_t>((d.n_jt_blocks + waves - 1) / waves, 256 * (16 / waves) / tiles));
+  hipLaunchKernelGGL((newton_jac_tile_kernel<NO>), dim3((unsigned)tiles, (unsigned)ny),
+                     dim3(64 * waves), jac_tile_lds(d), st, d, x, P, ldx, S, lds, n, J, part);
+  SBI_HIP_CHECK(hipGetLastError());
+  if (d.n_jt_red > 0) {
+    hipLaunchKernelGGL(jac_reduce_kernel, dim3((unsigned)((P + 255) / 256), (unsigned)d.n_jt_red),
+                       dim3(256), 0, st, d, d.jt_red, P, (int64_t)n, part, J, x, ldx);
+    SBI_HIP_CHECK(hipGetLastError());
+  }
+  return SBI_OK;
+}
+
 extern "C" int64_t sbi_newton_vjp_workspace(const sbi_newton_plan* plan, int64_t P) {
   const sbi_newton_desc* dp = nullptr;
   if (sbi_newton_plan_desc(plan, &dp) != SBI_OK || P < 0) {
@@ -947,7 +1210,7 @@ static int vjp_launch(const sbi_newton_desc& d, const double* x, int64_t P, int6
   }
   if (d.n_jac_red > 0) {
     hipLaunchKernelGGL(jac_reduce_kernel, dim3((unsigned)((P + 255) / 256), (unsigned)d.n_jac_red),
-                       dim3(256), 0, st, d, P, (int64_t)1, part, gx, (const double*)nullptr,
+                       dim3(256), 0, st, d, d.jac_red, P, (int64_t)1, part, gx, (const double*)nullptr,
                        (int64_t)0);
     SBI_HIP_CHECK(hipGetLastError());
   }
@@ -1023,7 +1286,6 @@ extern "C" int sbi_bary_basis_f32(const sbi_plan* plan, const double* x, int64_t
 // ------------------------------------------------------------------------------------------
 // Dense Jacobian of the Newton form
 // ------------------------------------------------------------------------------------------
-constexpr int kJacDirectMax = 8;  // outputs handled in one register pass
 
 // The Jacobian and adjoint passes are bound by latency per entry, so they need many waves per
 // CU: a factor table above kJacLdsMax (which would leave room for too few workgroups per CU) goes
@@ -1044,11 +1306,14 @@ extern "C" int64_t sbi_newton_jacobian_workspace(const sbi_newton_plan* plan, in
   }
   int64_t bytes = 0;
   const int64_t P64 = (P + kTile - 1) / kTile * kTile;
-  if (jac_global_table(*dp)) bytes += (int64_t)dp->n_tab_rows * P64 * (int64_t)sizeof(double);
+  if (jac_global_table(*dp) && !jac_tile_waves(*dp, n))
+    bytes += (int64_t)dp->n_tab_rows * P64 * (int64_t)sizeof(double);
   if (n > kJacDirectMax)  // D^T (row stride even), then the jobs' parts
     bytes += (int64_t)dp->n_vjp_ent * jac_ld(P) * (int64_t)sizeof(double) +
              (int64_t)dp->n_jac_slots * P * n * sbi::kJacGroup * (int64_t)sizeof(double);
-  else bytes += (int64_t)dp->n_jac_partials * P * n * (int64_t)sizeof(double);
+  else
+    bytes += (int64_t)(jac_tile_waves(*dp, n) ? dp->n_jt_slots : dp->n_jac_partials) * P * n *
+             (int64_t)sizeof(double);
   return bytes;
 }
 
@@ -1112,7 +1377,8 @@ extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double
     return SBI_ERR_INVALID;
   }
   hipStream_t st = (hipStream_t)stream;
-  const bool g = jac_global_table(d);
+  const int waves = jac_tile_waves(d, n);
+  const bool g = !waves && jac_global_table(d);
   double* gtab = g ? (double*)workspace : nullptr;
   const int64_t P64 = (P + kTile - 1) / kTile * kTile;
   double* DT = (double*)workspace + (g ? (int64_t)d.n_tab_rows * P64 : 0);
@@ -1131,6 +1397,12 @@ extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double
     }
     const int ni = (int)n;
     double* part = DT;  // partial sums of split dims: [n_jac_partials][P][n]
+    if (waves) {
+      if (n == 1) return jac_tile_launch<1>(d, x, P, ldx, S, lds, ni, J, part, st);
+      if (n == 2) return jac_tile_launch<2>(d, x, P, ldx, S, lds, ni, J, part, st);
+      if (n <= 4) return jac_tile_launch<4>(d, x, P, ldx, S, lds, ni, J, part, st);
+      return jac_tile_launch<8>(d, x, P, ldx, S, lds, ni, J, part, st);
+    }
     if (d.n_jac_units > 0) {
       if (g) {
         if (n == 1) jac_direct_launch<1, true>(d, x, P, ldx, S, lds, ni, gtab, J, part, st);
@@ -1147,7 +1419,7 @@ extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double
     }
     if (d.n_jac_red > 0) {
       hipLaunchKernelGGL(jac_reduce_kernel, dim3((unsigned)((P + 255) / 256), (unsigned)d.n_jac_red),
-                         dim3(256), 0, st, d, P, n, part, J, x, ldx);
+                         dim3(256), 0, st, d, d.jac_red, P, n, part, J, x, ldx);
       SBI_HIP_CHECK(hipGetLastError());
     }
     return SBI_OK;  // the register pass and the reduction wrote the NaNs at node coordinates

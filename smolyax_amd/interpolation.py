@@ -431,6 +431,17 @@ class SmolyakBarycentricInterpolator:
         if not np.isin(sing_dims, NL.tab_dim[: NL.n_tab_dims]).all():
             raise RuntimeError("singular coordinates in a dim without factors")
         t["sing_off"], t["sing_x"] = _dev_tensor(sing_off, i32, dev), _dev_tensor(sing_x, f64, dev)
+        if NL.n_jt_blocks:
+            nt = NL.n_tab_dims
+            first, ns = sing_off[NL.tab_dim[:nt]], np.diff(sing_off)[NL.tab_dim[:nt]]
+            if int(ns.max()) > 0x7FFF:
+                raise RuntimeError("more singular coordinates in a dim than the plan's records hold")
+            jt_dim = np.stack([NL.tab_dim[:nt], NL.tab_row[:nt],
+                               NL.tab_kmax[:nt].astype(np.int64) | ns.astype(np.int64) << 16,
+                               np.where(ns > 0, first, 0)], axis=1)
+            t["jt_dim"] = _dev_tensor(jt_dim.astype(np.int32).reshape(-1), i32, dev)
+            t["jt_ent"] = torch.as_tensor(NL.jt_ent.copy()).to(dev)
+            t["jt_unit"], t["jt_red"] = _dev_tensor(NL.jt_unit, i32, dev), _dev_tensor(NL.jt_red, i32, dev)
         if NL.node_sq is not None:  # staged kernel tables (else the unstaged kernel runs)
             t["node_sq"] = _dev_tensor(NL.node_sq, i32, dev)
         if getattr(NL, "mt_a", None) is not None:  # matrix-core kernel tables
@@ -465,6 +476,7 @@ class SmolyakBarycentricInterpolator:
         d.n_vjp_ent = NL.n_vjp_ent
         d.n_jac_units, d.n_jac_partials, d.n_jac_red = NL.n_jac_units, NL.n_jac_partials, NL.n_jac_red
         d.n_jac_jobs, d.n_jac_slots, d.n_jac_group_red = NL.n_jac_jobs, NL.n_jac_slots, NL.n_jac_group_red
+        d.n_jt_blocks, d.n_jt_slots, d.n_jt_red = NL.n_jt_blocks, NL.n_jt_slots, NL.n_jt_red
         d.gemm_head, d.gemm_kq = nh, t["gemm_sq"].shape[0] * 4
         d.ld_s64 = max(t["gemm_s64"].stride(0), self._d_out)
         if "mt_a" in t:

@@ -525,6 +525,8 @@ def head_order(nf: NewtonForm, L: NewtonLayout, n_head: int = HEAD_ROWS):
 
 
 JAC_UNIT = 128  # adjoint entries per work unit of the Jacobian's register pass
+JAC_TILE_UNIT = 64  # entries per unit of the Jacobian's register pass with its table in LDS
+JAC_TILE_BLOCK = 16  # units a wave of it takes side by side
 JAC_GROUP = 8   # dims per accumulator set of the Jacobian contraction (d_out > 8)
 
 
@@ -596,7 +598,61 @@ def build_basis_tables(nf: NewtonForm, L: NewtonLayout) -> None:
     L.jac_red = np.array(red or [(0, 0, 0)], dtype=np.int32).reshape(-1)
     node = np.array([e[0:2].view(np.int32)[0] for e in ent] or [0], dtype=np.int32)
     build_jacobian_rows(L, node, nf.d_out)
+    build_jacobian_units(L, tab_dims, row0, per_row)
     L.vjp_ent = (np.stack(ent) if ent else np.full((1, 8), 0xFFFF, dtype=np.uint16)).reshape(-1).view(np.uint8)
+
+
+def build_jacobian_units(L: NewtonLayout, tab_dims, row0, per_row) -> None:
+    """Units of the register pass with the factor table in LDS: the entries of one factor row (j, k)
+    by number of other factors, in runs of at most JAC_TILE_UNIT; a dim of several units adds their
+    sums in the order of (k, run).  Blocks of JAC_TILE_BLOCK units of about one length (longest
+    first, then by dim), records step by step, so that a wave reads 16 units' records in one run.
+    None when the table does not fit LDS or a field its record."""
+    L.n_jt_blocks = L.n_jt_slots = L.n_jt_red = 0
+    L.jt_ent = L.jt_unit = L.jt_red = None
+    n_rows, B = L.n_tab_rows, JAC_TILE_BLOCK
+    if (n_rows + 1) * 128 + 2 * len(tab_dims) > 160 * 1024 or tab_dims[-1:] > [0xFFFF]:
+        return
+    units, red, slots = [], [], 0  # units: (dim | degree << 16, slot, entries)
+    for i, j in enumerate(tab_dims):
+        km = int(L.tab_kmax[i])
+        mine = []
+        for k in range(1, km + 1):
+            run = sorted(per_row[row0[j] + k - 1], key=lambda e: len(e[1]))
+            mine += [(j | k << 16, run[a: a + JAC_TILE_UNIT]) for a in range(0, len(run), JAC_TILE_UNIT)]
+        if len(mine) > 1:
+            red.append((j, slots, len(mine)))
+            units += [(key, slots + q, run) for q, (key, run) in enumerate(mine)]
+            slots += len(mine)
+        else:
+            units += [(key, ~i, run) for key, run in mine]
+    if not units or max(e[0] for u in units for e in u[2]) >= 1 << 24 or L.kmax1 > 0x8000:
+        return
+    units.sort(key=lambda u: (-len(u[2]), u[0] >> 16 > 1))
+    heads, recs, step = [], [], 0
+    for a in range(0, len(units), B):
+        blk = units[a: a + B]
+        n = len(blk[0][2])
+        rec = np.full((n, B, 8), n_rows, dtype=np.uint16)
+        rec[:, :, :2] = 0
+        for t in range(n):
+            nf = max(len(u[2][t][1]) for u in blk if t < len(u[2]))
+            rec[t, :, 1] = nf << 8
+        for q, (key, slot, run) in enumerate(blk):
+            heads.append((key, step, len(run), slot))
+            for t, (node, others) in enumerate(run):
+                rec[t, q, 0] = node & 0xFFFF
+                rec[t, q, 1] |= node >> 16
+                rec[t, q, 2: 2 + len(others)] = others
+        heads += [(1 << 16 | tab_dims[0], step, 0, 0)] * (B - len(blk))
+        recs.append(rec)
+        step += n
+    pad = np.full((8, B, 8), n_rows, dtype=np.uint16)  # steps read ahead of the last block
+    pad[:, :, :2] = 0
+    L.jt_ent = np.concatenate(recs + [pad]).reshape(-1).view(np.uint8)
+    L.jt_unit = np.array(heads, dtype=np.int64).astype(np.int32).reshape(-1)
+    L.jt_red = np.array(red or [(0, 0, 0)], dtype=np.int32).reshape(-1)
+    L.n_jt_blocks, L.n_jt_slots, L.n_jt_red = len(recs), slots, len(red)
 
 
 def build_jacobian_rows(L: NewtonLayout, node, d_out: int) -> None:

@@ -274,3 +274,34 @@ def test_jacobian_rows_of_every_dim(gpu, d, d_out, m, P):
     assert J.shape == Je.shape and rel(J, Je) <= GRAD_TOL
     p = P // 2
     assert np.array_equal(ip.gradient(x[p:p + 1]).cpu().numpy()[0], J[p])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,d_out,m,P", [(1, 1, 20, 16), (2, 1, 40, 1), (10, 1, 1000, 17), (40, 2, 200, 33),
+                                         (300, 1, 1500, 48), (60, 3, 700, 31), (10, 4, 1000, 47),
+                                         (1000, 8, 3000, 18)])
+def test_jacobian_few_outputs_units(gpu, d, d_out, m, P):
+    """Jacobian of 1..8 outputs over units of entries: one unit, less than a block of 16, several
+    blocks per wave, dims of several units, ragged tiles of 16 points; NaN exactly at the node
+    coordinates of a dim; against the exact Jacobian, and the same bits for a point alone."""
+    ref, ip, rng = make(d, d_out, m, seed=d + d_out)
+    L = ip._nlayout
+    print("units", L.n_jt_blocks, L.n_jt_slots, "rows", L.n_tab_rows, flush=True)
+    assert L.n_jt_blocks > 0
+    x = rng.uniform(-1, 1, (P, d))
+    J = ip.gradient(x).cpu().numpy().reshape(P, d_out, d)
+    Je = exact_grad(ref, x).reshape(P, d_out, d)
+    assert rel(J, Je) <= GRAD_TOL
+    p = P - 1
+    assert np.array_equal(ip.gradient(x[p:p + 1]).cpu().numpy().reshape(d_out, d), J[p])
+    off, nodes = ip._singular_coordinates()
+    dims = [0, d // 2, d - 1]
+    y = x.copy()
+    for i, j in enumerate(dims):
+        if off[j + 1] > off[j]:
+            y[(5 * i) % P, j] = nodes[off[j + 1] - 1]  # the largest node of the dim
+    Jn = ip.gradient(y).cpu().numpy().reshape(P, d_out, d)
+    hit = np.zeros((P, d), dtype=bool)
+    for j in range(d):
+        hit[:, j] = np.isin(y[:, j], nodes[off[j]:off[j + 1]])
+    assert np.array_equal(np.isnan(Jn), np.broadcast_to(hit[:, None, :], Jn.shape))
