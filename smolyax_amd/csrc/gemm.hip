@@ -495,7 +495,6 @@ __global__ __launch_bounds__(256) void contract_reduce_kernel(const E* __restric
 // kSplitTarget workgroups run (small batches: the k loop of one workgroup is the latency).
 constexpr int64_t kSplitMinGroups = 256;
 constexpr int64_t kSplitTarget = 512;
-constexpr int64_t kF64SplitGroups = 768;            // FP64: three 4-wave workgroups per CU
 constexpr int64_t kSplitMaxBytes = int64_t(256) << 20;  // workspace of one split call
 struct SplitPlan {
   int64_t nsplit = 0, cps = 0, nch = 0, part_bytes = 0, head_bytes = 0;
@@ -563,17 +562,16 @@ int contract_split_launch(const SplitPlan& sp, const float* A, int64_t lda, cons
 // per cycle and CU, so what matters is that several waves per SIMD always have their fragments at
 // hand: operands are staged in LDS, three buffers of 16 k, copied two chunks ahead by direct
 // global -> LDS loads (one barrier per chunk), and the register count allows three waves per SIMD.
-// 8192 points x 256 outputs, K 5000: 367 us (57 TFLOP/s) against 402-412 us with each wave loading
-// its own fragments from L2 one chunk ahead; 5000 x 160, K 10 002 (k over workgroups): 478 -> 345-390 us;
-// 5000 x 8192, K 256: 487 -> 390 us; 4096 x 4096, K 9986: 5590 -> 5500 us.  Requesting a whole
+// 8192 points x 256 outputs, K 5000: 340-376 us (matrix cores busy 85 % of the time, 2.15 GHz) against
+// 402-412 us with each wave loading its own fragments from L2 one chunk ahead; 5000 x 160, K 10 002 (k
+// over workgroups): 478 -> 305 us; 5000 x 8192, K 256: 487 -> 380-430 us.  Requesting a whole
 // chunk's fragments before its first MFMA costs a wave per SIMD's worth of registers (5730 us).
 //
 // Work split: a workgroup of 4 waves owns a (32 * WM)-point x (32 * WN)-output tile, each wave 16 * WM
 // points x 16 * WN outputs; the last output tile with at most 32 outputs left is cut into four waves of
 // 16 points x 32 outputs instead, so that no wave works on outputs past the edge (160 outputs:
-// 17 % less matrix work).  WN = 1 for at most 32 outputs; WM = 1 (32 points) where k is not spread
-// and 64-point tiles would be fewer than one per CU (500 x 64, K 9986, no workspace: 472 -> 342
-// us).  The output tiles of one point tile run
+// 17 % less matrix work).  WN = 1 for at most 32 outputs; WM = 1 (32 points) where that fills the CUs
+// better (f64_plan).  The output tiles of one point tile run
 // on one XCD (its L2 serves their A rows).
 //
 // LDS image of a chunk: rows of the tile's width; the 16-byte slot q of row r holds the elements
@@ -581,21 +579,27 @@ int contract_split_launch(const SplitPlan& sp, const float* A, int64_t lda, cons
 // halves of the banks.  kDirect = false: row strides, widths or bases that are not multiples of
 // 16 bytes go through registers (8-byte loads one chunk ahead); the same image, the same bits.
 //
-// Sums: the MFMA accumulators hold a chain of kFlushK terms, the chains are added into a slice sum
-// of kF64Slice terms, the slice sums in order, so the rounding grows with kFlushK + kF64Slice /
-// kFlushK + K / kF64Slice terms.  Small grids spread k over workgroups (nz > 1) in units of a
-// slice, very small ones in units of a chain; each writes the sums of its units to `part` and
+// Sums: the MFMA accumulators hold a chain of kFlushK terms, the chains are added into the sum of a
+// slice (a third of K), the three slice sums in order, so the rounding grows with kFlushK + K / (3
+// kFlushK) + 3 terms.  Grids that would leave CUs idle spread k over workgroups (f64_plan), a
+// slice or some chains each; they write the sums of these units to `part` and
 // contract_reduce_kernel adds them in the same order: the same bits for any P, alone or in a batch.
 // ------------------------------------------------------------------------------------------
-constexpr int kF64Slice = 2048;
+constexpr int kF64Slices = 3;
 constexpr int kF64Buf = 3;
+// k per slice (the last one may be shorter): whole chunks, one slice up to three chains
+inline int64_t f64_slice(int64_t K) {
+  if (K <= kF64Slices * kFlushK) return std::max<int64_t>(K, 1);
+  const int64_t third = (K + kF64Slices - 1) / kF64Slices;
+  return (third + kChunk - 1) / kChunk * kChunk;
+}
 enum { kWhole = 0, kBySlice = 1, kByChain = 2 };  // how k is spread over workgroups (kSplit)
 
 template <int WM, int WN, bool kDirect, int kSplit>
 __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64_kernel(
     const double* __restrict__ A, int64_t lda, const double* __restrict__ B, int64_t ldb,
     const double* __restrict__ offset, double* __restrict__ Y, int64_t ldy, int64_t P, int64_t n,
-    int64_t K, int ntm, int ntn, int nz, int64_t kpz, double* __restrict__ part) {
+    int64_t K, int ntm, int ntn, int nz, int64_t slice, int upz, double* __restrict__ part) {
   constexpr int TM = 32 * WM, TN = 32 * WN;
   constexpr int kA = kChunk * TM * 8, kStep = kA + kChunk * TN * 8;  // bytes of a chunk: A, then B
   constexpr int nA = kA / 1024, kPer = kStep / 4096;                 // 1 KB copies: of A, per wave
@@ -615,48 +619,58 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64
   const bool thin = WM == 2 && WN == 2 && n - n0 <= 32;  // 4 x 1 waves of 16 x 32 instead of 2 x 2 of 32 x 32
   const int mw = thin ? wave * 16 : (wave & 1) * (16 * WM);
   const int nw = thin ? 0 : (wave >> 1) * (16 * WN);
-  const int64_t kb = (int64_t)z * kpz;  // kpz: k per workgroup, whole units
-  const int64_t ke = kSplit ? min(K, kb + kpz) : K;
+  // k in chunks: KC of them, sc per slice; chain u (kByChain: upz of them per workgroup, in slices
+  // of `per`) starts at chunk c_of(u); this workgroup takes [cb, ce)
+  const int KC = (int)((K + kChunk - 1) / kChunk), KF = (int)(K / kChunk);
+  const int sc = (int)((slice + kChunk - 1) / kChunk), cpc = kFlushK / kChunk;
+  const int per = (sc + cpc - 1) / cpc;
+  auto c_of = [&](int u) { return min(KC, (u / per) * sc + (u % per) * cpc); };
+  const int cb = kSplit == kWhole ? 0 : kSplit == kBySlice ? z * sc : c_of(z * upz);
+  const int ce = kSplit == kWhole ? KC : kSplit == kBySlice ? min(KC, cb + sc) : c_of((z + 1) * upz);
 
   // copy i of this wave: 128 consecutive elements of the LDS image, two per lane (columns past
-  // the edge re-read the last pair or element, rows past K row K - 1: never used)
-  const double* src[kPer];  // this lane's pair in the next chunk
+  // the edge re-read the last pair or element, rows past K row K - 1: never used).  The address is
+  // a scalar base that advances by a chunk plus this lane's fixed offset: every vector instruction
+  // in the loop takes time from the matrix cores (23 per chunk: 437 us, 4 per chunk: 400 us, 8192 x
+  // 256, K 5000).
+  typedef typename std::conditional<kDirect, uint32_t, uint64_t>::type off_t;
+  const char* baseA = (const char*)(A + m0 + (int64_t)cb * kChunk * lda);  // of the next chunk
+  const char* baseB = (const char*)(B + n0 + (int64_t)cb * kChunk * ldb);
   auto krow = [&](int i) {
     const int c = wave + 4 * i;
-    return c < nA ? (c * 128 + lane * 2) / TM : ((c - nA) * 128 + lane * 2) / TN;
+    return 4 * i < nA ? (c * 128 + lane * 2) / TM : ((c - nA) * 128 + lane * 2) / TN;
   };
+  off_t col[kPer], voff[kPer];  // bytes from the base to this lane's pair: in its row, in all
   uint32_t odd = 0;  // bit i: the pair's second element is past the edge (kDirect = false)
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int c = wave + 4 * i;
-    const bool isA = c < nA;
+    const bool isA = 4 * i < nA;
     const int T = isA ? TM : TN;
     const int pos = (isA ? c : c - nA) * 128 + lane * 2;
-    const int64_t col = (((pos % T) / 2) ^ (8 * (krow(i) & 1))) * 2;
-    const int64_t at = (isA ? m0 : n0) + col, end = isA ? P : n;
-    const int64_t ld = isA ? lda : ldb;
-    const double* base = (isA ? A : B) + min(at, kDirect ? (end - 1) & ~(int64_t)1 : end - 1);
+    const int64_t org = isA ? m0 : n0;
+    const int64_t at = org + (((pos % T) / 2) ^ (8 * (krow(i) & 1))) * 2, end = isA ? P : n;
     if (!kDirect && at + 1 >= end) odd |= 1u << i;
-    src[i] = base + (kb + krow(i)) * ld;
+    col[i] = (off_t)((min(at, kDirect ? (end - 1) & ~(int64_t)1 : end - 1) - org) * 8);
+    voff[i] = col[i] + (off_t)krow(i) * (off_t)((isA ? lda : ldb) * 8);
   }
-  int64_t ki = kb;  // first row of the next chunk to be copied
+  int ci = cb;  // the next chunk to be copied
   double pend[kDirect ? 1 : 2 * kPer];
   auto advance = [&](auto&& put) {
-    if (ki + kChunk <= K) {
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) {
-        put(i, src[i]);
-        src[i] += kChunk * (wave + 4 * i < nA ? lda : ldb);
-      }
-    } else {  // the last chunk of K
+    if (ci >= KF) {  // the last rows of K
 #pragma unroll
       for (int i = 0; i < kPer; ++i)
-        put(i, src[i] - max((int64_t)0, ki + krow(i) - (K - 1)) * (wave + 4 * i < nA ? lda : ldb));
+        voff[i] = col[i] + (off_t)min(krow(i), (int)(K - 1 - (int64_t)ci * kChunk)) *
+                               (off_t)((4 * i < nA ? lda : ldb) * 8);
     }
-    ki += kChunk;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) put(i, (const double*)((4 * i < nA ? baseA : baseB) + voff[i]));
+    baseA += kChunk * 8 * lda;
+    baseB += kChunk * 8 * ldb;
+    ++ci;
   };
   auto fetch = [&] {  // kDirect = false: the next chunk into registers
-    if (ki < ke)
+    if (ci < ce)
       advance([&](int i, const double* p) {
         pend[2 * i] = p[0];
         pend[2 * i + 1] = p[(odd >> i) & 1 ? 0 : 1];
@@ -665,7 +679,7 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64
   auto issue = [&](int b) {  // the next chunk into buffer b
     char* dst = smem + b * kStep + wave * 1024;
     if constexpr (kDirect) {
-      if (ki < ke)
+      if (ci < ce)
         advance([&](int i, const double* p) {
           __builtin_amdgcn_global_load_lds((const void*)p, (lds_void*)(dst + i * 4096), 16, 0, 0);
         });
@@ -677,10 +691,10 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64
       fetch();
     }
   };
-  // the chunk at k0 has landed in every wave (the copies of the next one may be in flight)
-  auto wait = [&](int64_t k0) {
+  // chunk c has landed in every wave (the copies of the next one may be in flight)
+  auto wait = [&](int c) {
     if constexpr (kDirect) {
-      if (k0 + kChunk < ke) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
+      if (c + 1 < ce) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       asm volatile("s_barrier" ::: "memory");
     } else {
@@ -688,56 +702,9 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64
     }
   };
 
-  v4d total[WM][WN], sum[WM][WN], acc[WM][WN];
-  auto each = [&](auto&& f) {  // the fragments of this wave
-#pragma unroll
-    for (int fm = 0; fm < WM; ++fm)
-#pragma unroll
-      for (int fn = 0; fn < WN; ++fn) f(fm, fn);
-  };
-  each([&](int fm, int fn) { total[fm][fn] = v4d{0, 0, 0, 0}; });
-
   int bi = 0;  // buffer of the chunk being computed
   const int sw = 16 * (g & 1);
-  auto compute = [&](int64_t k0, bool tail) {
-    const double* la = (const double*)(smem + bi * kStep);
-    const double* lb = (const double*)(smem + bi * kStep + kA);
-#pragma unroll
-    for (int s = 0; s < kChunk / 4; ++s) {
-      double a[WM], b[WN];
-      const int r = 4 * s + g;
-#pragma unroll
-      for (int fm = 0; fm < WM; ++fm) a[fm] = la[r * TM + ((mw + fm * 16 + li) ^ sw)];
-#pragma unroll
-      for (int fn = 0; fn < WN; ++fn) b[fn] = lb[r * TN + ((nw + fn * 16 + li) ^ sw)];
-      if (tail && k0 + r >= K) {
-#pragma unroll
-        for (int fm = 0; fm < WM; ++fm) a[fm] = 0.0;
-#pragma unroll
-        for (int fn = 0; fn < WN; ++fn) b[fn] = 0.0;
-      }
-#pragma unroll
-      for (int fm = 0; fm < WM; ++fm) {
-        if (fm && thin) break;
-#pragma unroll
-        for (int fn = 0; fn < WN; ++fn) acc[fm][fn] = mfma(a[fm], b[fn], acc[fm][fn]);
-      }
-    }
-  };
-  auto chain = [&](int64_t kc, int64_t kce) {  // acc += rows [kc, kce)
-    const int64_t kf = kc + ((kce - kc) & ~(int64_t)(kChunk - 1));
-    for (int64_t k0 = kc; k0 < kf; k0 += kChunk) {
-      wait(k0);
-      issue(kDirect ? (bi == 0 ? kF64Buf - 1 : bi - 1) : (bi + 1 == kF64Buf ? 0 : bi + 1));
-      compute(k0, false);
-      bi = bi + 1 == kF64Buf ? 0 : bi + 1;
-    }
-    if (kf < kce) {
-      wait(kf);
-      compute(kf, true);
-    }
-  };
-  if (kb < ke) {
+  if (cb < ce) {
     if constexpr (kDirect) {
       issue(0);
       issue(1);
@@ -746,73 +713,168 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64
       issue(0);
     }
   }
-  auto row_of = [&](int fm, int r) { return m0 + mw + fm * 16 + g + 4 * r; };
-  auto col_of = [&](int fn) { return n0 + nw + fn * 16 + li; };
-  auto emit = [&](int64_t unit, v4d(&v)[WM][WN]) {
-    double* __restrict__ out = part + unit * P * n;
+  // the walk over k, once for whole tiles and once for thin ones: a test inside a chunk would cut its
+  // matrix instructions into pairs that each wait for their LDS reads
+  auto walk = [&](auto thin_tile) {
+    constexpr bool kThin = decltype(thin_tile)::value;
+    constexpr int M = kThin ? 1 : WM;
+    v4d total[M][WN], sum[M][WN], acc[M][WN];
+    auto each = [&](auto&& f) {  // the fragments of this wave
+#pragma unroll
+      for (int fm = 0; fm < M; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < WN; ++fn) f(fm, fn);
+    };
+    each([&](int fm, int fn) { total[fm][fn] = v4d{0, 0, 0, 0}; });
+    uint32_t pa[M], pb[WN];  // byte offsets of this lane's elements in a buffer
+#pragma unroll
+    for (int fm = 0; fm < M; ++fm) pa[fm] = (uint32_t)(g * TM + ((mw + fm * 16 + li) ^ sw)) * 8;
+#pragma unroll
+    for (int fn = 0; fn < WN; ++fn) pb[fn] = (uint32_t)(kA + (g * TN + ((nw + fn * 16 + li) ^ sw)) * 8);
+    auto compute = [&](int c, bool tail) {
+      const char* buf = smem + bi * kStep;
+#pragma unroll
+      for (int s = 0; s < kChunk / 4; ++s) {
+        double a[M], b[WN];
+#pragma unroll
+        for (int fm = 0; fm < M; ++fm) a[fm] = *(const double*)(buf + pa[fm] + s * 32 * TM);
+#pragma unroll
+        for (int fn = 0; fn < WN; ++fn) b[fn] = *(const double*)(buf + pb[fn] + s * 32 * TN);
+        if (tail && (int64_t)c * kChunk + 4 * s + g >= K) {
+#pragma unroll
+          for (int fm = 0; fm < M; ++fm) a[fm] = 0.0;
+#pragma unroll
+          for (int fn = 0; fn < WN; ++fn) b[fn] = 0.0;
+        }
+        // a wave with its operands at hand goes ahead of those that address and wait (400 -> 375 us)
+        __builtin_amdgcn_s_setprio(1);
+        each([&](int fm, int fn) { acc[fm][fn] = mfma(a[fm], b[fn], acc[fm][fn]); });
+        __builtin_amdgcn_s_setprio(0);
+      }
+    };
+    auto chain = [&](int c0, int c1) {  // acc = the sum over the chunks [c0, c1)
+      each([&](int fm, int fn) { acc[fm][fn] = v4d{0, 0, 0, 0}; });
+      const int cf = min(c1, KF);
+      for (int c = c0; c < cf; ++c) {
+        wait(c);
+        issue(kDirect ? (bi == 0 ? kF64Buf - 1 : bi - 1) : (bi + 1 == kF64Buf ? 0 : bi + 1));
+        compute(c, false);
+        bi = bi + 1 == kF64Buf ? 0 : bi + 1;
+      }
+      if (cf < c1) {
+        wait(cf);
+        compute(cf, true);
+      }
+    };
+    auto row_of = [&](int fm, int r) { return m0 + mw + fm * 16 + g + 4 * r; };
+    auto col_of = [&](int fn) { return n0 + nw + fn * 16 + li; };
+    auto emit = [&](int64_t unit, v4d(&v)[M][WN]) {
+      double* __restrict__ out = part + unit * P * n;
+      each([&](int fm, int fn) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int64_t row = row_of(fm, r), col = col_of(fn);
+          if (row < P && col < n) out[row * n + col] = v[fm][fn][r];
+        }
+      });
+    };
+    if constexpr (kSplit == kByChain) {
+      for (int u = z * upz; c_of(u) < ce; ++u) {
+        chain(c_of(u), c_of(u + 1));
+        emit(u, acc);
+      }
+      return;
+    }
+    for (int c0 = cb; c0 < ce; c0 += sc) {
+      const int c1 = min(ce, c0 + sc);
+      each([&](int fm, int fn) { sum[fm][fn] = v4d{0, 0, 0, 0}; });
+      for (int c = c0; c < c1; c += cpc) {
+        chain(c, min(c1, c + cpc));
+        each([&](int fm, int fn) { sum[fm][fn] += acc[fm][fn]; });
+      }
+      if constexpr (kSplit == kWhole) each([&](int fm, int fn) { total[fm][fn] += sum[fm][fn]; });
+      else emit(z, sum);
+    }
+    if constexpr (kSplit != kWhole) return;
     each([&](int fm, int fn) {
+      const int64_t col = col_of(fn);
+      const double off = offset ? offset[min(col, n - 1)] : 0.0;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t row = row_of(fm, r), col = col_of(fn);
-        if (row < P && col < n && !(thin && fm)) out[row * n + col] = v[fm][fn][r];
+        const int64_t row = row_of(fm, r);
+        if (row < P && col < n) Y[row * ldy + col] = off + total[fm][fn][r];
       }
     });
   };
-  for (int64_t ks = kb; ks < ke; ks += kF64Slice) {
-    const int64_t kse = min(ke, ks + (int64_t)kF64Slice);
-    each([&](int fm, int fn) { sum[fm][fn] = v4d{0, 0, 0, 0}; });
-    for (int64_t kc = ks; kc < kse; kc += kFlushK) {
-      each([&](int fm, int fn) { acc[fm][fn] = v4d{0, 0, 0, 0}; });
-      chain(kc, min(kse, kc + (int64_t)kFlushK));
-      if constexpr (kSplit == kByChain) emit(kc / kFlushK, acc);
-      else each([&](int fm, int fn) { sum[fm][fn] += acc[fm][fn]; });
-    }
-    if constexpr (kSplit == kWhole) each([&](int fm, int fn) { total[fm][fn] += sum[fm][fn]; });
-    else if constexpr (kSplit == kBySlice) emit(ks / kF64Slice, sum);
+  if constexpr (WM == 2 && WN == 2) {
+    if (thin) return walk(std::true_type{});
   }
-  if constexpr (kSplit != kWhole) return;
-  each([&](int fm, int fn) {
-    const int64_t col = col_of(fn);
-    const double off = offset ? offset[min(col, n - 1)] : 0.0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t row = row_of(fm, r);
-      if (row < P && col < n && !(thin && fm)) Y[row * ldy + col] = off + total[fm][fn][r];
-    }
-  });
+  walk(std::false_type{});
 }
 
-// How contract_f64_kernel spreads k over workgroups (nz = 1: not at all, no workspace): when the
-// tiles alone are fewer than kF64SplitGroups, in units of a slice if that gives enough
-// workgroups (little workspace traffic: 5000 x 160 outputs, K 10 002, 480 -> 345-390 us), else in
-// units of a chain (500 x 64, K 9986: 472 us unsplit, 104 us by slices, 31 us by chains).
+// How contract_f64_kernel spreads the work: tiles of 64 or 32 points, and k not at all (nz = 1, no
+// workspace), a slice per workgroup, or upz chains each, whichever takes least by this estimate.
+// A CU holds three workgroups of the larger tile (four of the smaller, 16 % slower per point); alone
+// one reaches about half of the matrix cores' rate, two 0.8 of it.  So a CU that gets q workgroups
+// takes as long as q of them at the full rate, and more for the last one or two.  The partial
+// sums are written and read once, at about 4.5 TB/s, by a second launch.
+// 5000 x 160, K 10 002: 388 us with slices of 2048 dealt to equal numbers of workgroups, 315 us by
+// thirds; 8192 x 256, K 5000: 435 and 376 us; 2000 x 2000 of an evaluation with K 660: 272 us with
+// tiles of 64 points (1024 tiles, four per CU), 248 us of 32; 500 x 64, K 9986: 472 us unsplit, 104
+// us by slices, 31 us by chains.
 struct F64Plan {
-  int64_t nz = 1, kpz = 0, units = 0, bytes = 0;
-  int split = kWhole;
+  int64_t nz = 1, units = 0, per = 1, bytes = 0;
+  int split = kWhole, upz = 1, wm = 2;  // wm: 32 wm points per tile
 };
 inline int64_t f64_tile_n(int64_t n) { return n <= 32 ? 32 : 64; }
-F64Plan f64_plan(int64_t P, int64_t n, int64_t K) {
-  F64Plan pl;
-  if (P <= 0 || n <= 0) return pl;
-  const int64_t groups = ((P + kBlockM - 1) / kBlockM) * ((n + f64_tile_n(n) - 1) / f64_tile_n(n));
-  const int64_t want = (kF64SplitGroups + groups - 1) / groups;
-  const bool fine = want > (K + kF64Slice - 1) / kF64Slice;
-  const int64_t unit = fine ? kFlushK : kF64Slice;
-  const int64_t units = (K + unit - 1) / unit;
-  if (want < 2 || units < 2) return pl;
-  const int64_t upz = (units + want - 1) / want, nz = (units + upz - 1) / upz;
-  const int64_t bytes = units * P * n * 8;
-  if (nz < 2 || bytes > kSplitMaxBytes) return pl;
-  pl.nz = nz;
-  pl.kpz = upz * unit;
-  pl.units = units;
-  pl.bytes = bytes;
-  pl.split = fine ? kByChain : kBySlice;
-  return pl;
+F64Plan f64_plan(int64_t P, int64_t n, int64_t K, bool may_split = true) {
+  F64Plan best;
+  if (P <= 0 || n <= 0) return best;
+  const int64_t tn = f64_tile_n(n), tiles = (P + kBlockM - 1) / kBlockM * ((n + tn - 1) / tn);
+  const int64_t slice = f64_slice(K), slices = (K + slice - 1) / slice;
+  const int64_t per = (slice + kFlushK - 1) / kFlushK;
+  const int64_t chains = (slices - 1) * per + (K - (slices - 1) * slice + kFlushK - 1) / kFlushK;
+  // microseconds of `each` chains in every one of nz workgroups per tile, and of the partial sums
+  auto cost = [&](int64_t nz, double each, int64_t units) {
+    const double chain = 64.0 * tn * 2 * kFlushK / (72e6 / 256);
+    const int64_t q = (tiles * nz + 255) / 256, rest = q % 3;
+    const double rounds = (double)(q - rest) + (rest == 1 ? 2.0 : rest == 2 ? 2.5 : 0.0);
+    const double bytes = (double)units * P * n * 16;
+    return rounds * (each * chain + 2.0) + (units ? 6.0 + bytes / 4.5e6 : 0.0);
+  };
+  double least = cost(1, (double)K / kFlushK, 0);
+  {
+    const int64_t q = ((P + 31) / 32 * ((n + tn - 1) / tn) + 255) / 256, rest = q % 4;
+    const double half[4] = {0.0, 1.0, 1.25, 1.7};
+    const double chain = 64.0 * tn * 2 * kFlushK / (72e6 / 256);
+    const double c = (0.58 * (double)(q - rest) + half[rest]) * ((double)K / kFlushK * chain + 2.0);
+    if (c < least) {
+      least = c;
+      best.wm = 1;
+    }
+  }
+  if (K <= kFlushK || !may_split) return best;
+  auto consider = [&](int split, int64_t nz, double each, int64_t units, int64_t upz) {
+    if (nz < 2 || units * P * n * 8 > kSplitMaxBytes) return;
+    const double c = cost(nz, each, units);
+    if (c >= least) return;
+    least = c;
+    best.wm = 2;
+    best.split = split;
+    best.nz = nz;
+    best.units = units;
+    best.per = split == kByChain ? per : 1;
+    best.upz = (int)upz;
+    best.bytes = units * P * n * 8;
+  };
+  consider(kBySlice, slices, (double)slice / kFlushK, slices, 1);
+  for (int64_t upz = 1; upz <= std::min<int64_t>(chains, 64); ++upz)
+    consider(kByChain, (chains + upz - 1) / upz, (double)upz, chains, upz);
+  return best;
 }
 
 typedef void (*f64_kernel_t)(const double*, int64_t, const double*, int64_t, const double*, double*,
-                             int64_t, int64_t, int64_t, int64_t, int, int, int, int64_t, double*);
+                             int64_t, int64_t, int64_t, int64_t, int, int, int, int64_t, int, double*);
 template <int WN, bool kDirect>
 f64_kernel_t f64_kernel(int wm, int split) {
   if (split == kBySlice) return contract_f64_kernel<2, WN, kDirect, kBySlice>;
@@ -826,11 +888,12 @@ int contract_f64(const double* A, int64_t lda, const double* B, int64_t ldb, con
                  double* Y, int64_t ldy, int64_t P, int64_t n, int64_t K, bool padded, void* ws,
                  int64_t ws_bytes, hipStream_t st) {
   F64Plan pl = f64_plan(P, n, K);
-  if (!ws || ws_bytes < pl.bytes) pl = F64Plan{};
+  if (!ws || ws_bytes < pl.bytes) pl = f64_plan(P, n, K, false);
   const bool direct = K == 0 || (((uintptr_t)A | (uintptr_t)B) % 16 == 0 && lda % 2 == 0 &&
-                                 ldb % 2 == 0 && (padded || (P % 2 == 0 && n % 2 == 0)));
+                                 ldb % 2 == 0 && std::max(lda, ldb) < (1 << 24) &&  // 32-bit offsets
+                                 (padded || (P % 2 == 0 && n % 2 == 0)));
   const int64_t tn = f64_tile_n(n), ntn = (n + tn - 1) / tn;
-  const int wm = pl.nz == 1 && (P + 63) / 64 * ntn < 192 ? 1 : 2;
+  const int wm = pl.wm;
   const int64_t ntm = (P + 32 * wm - 1) / (32 * wm);
   const int64_t grid = ((ntm * pl.nz + 7) / 8) * 8 * ntn;
   if (grid > 0x7fffffff) {
@@ -842,13 +905,12 @@ int contract_f64(const double* A, int64_t lda, const double* B, int64_t ldb, con
                                        : (direct ? f64_kernel<2, true>(wm, pl.split)
                                                  : f64_kernel<2, false>(wm, pl.split));
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * kWaves), 0, st, A, lda, B, ldb, offset,
-                     Y, ldy, P, n, K, (int)ntm, (int)ntn, (int)pl.nz, pl.kpz, (double*)ws);
+                     Y, ldy, P, n, K, (int)ntm, (int)ntn, (int)pl.nz, f64_slice(K), pl.upz, (double*)ws);
   SBI_HIP_CHECK(hipGetLastError());
   if (pl.nz > 1) {
     const int64_t rg = std::min<int64_t>((P * n + 255) / 256, 4096);
-    const int64_t per = pl.split == kByChain ? kF64Slice / kFlushK : 1;
     hipLaunchKernelGGL((contract_reduce_kernel<double>), dim3((unsigned)rg), dim3(256), 0, st,
-                       (const double*)ws, pl.units, per, nullptr, offset, Y, ldy, P, n, K);
+                       (const double*)ws, pl.units, pl.per, nullptr, offset, Y, ldy, P, n, K);
     SBI_HIP_CHECK(hipGetLastError());
   }
   return SBI_OK;

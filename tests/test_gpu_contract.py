@@ -279,7 +279,7 @@ def test_contract_bf16_tile_shapes_same_bits(gpu):
 @pytest.mark.parametrize("P,n,K", [(1, 1, 1), (63, 33, 15), (65, 96, 257), (500, 64, 2049),
                                    (130, 7, 4096), (777, 40, 5003), (5000, 160, 4100)])
 def test_contract_f64_ws_same_bits_for_every_split_and_alignment(gpu, P, n, K):
-    """sbi_contract_f64_ws: k spread over workgroups (by 256-term chains or 2048-term slices, as the
+    """sbi_contract_f64_ws: k spread over workgroups (by 256-term chains or by thirds, as the
     shape asks) and 16-byte copies with a spare element per odd row, against sbi_contract (no
     workspace, 8-byte loads where a width is odd): the same bits; and against the FP64 product.
     Bound: (K + 8) * 2^-53 of sum |A| |B| per element (one rounding per term, any order)."""
@@ -300,3 +300,29 @@ def test_contract_f64_ws_same_bits_for_every_split_and_alignment(gpu, P, n, K):
     assert torch.equal(Y, contract(Ac, Bc, off))
     ref, scale = _ref(Ac, Bc, off)
     assert ((Y - ref).abs() <= (K + 8) * 2.0 ** -53 * (scale + off.abs())).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("P,n,K", [(16447, 50, 100), (2600, 700, 769), (5000, 160, 1601), (8191, 130, 2500)])
+def test_contract_f64_points_alone_and_in_a_batch(gpu, P, n, K):
+    """Tiles of 64 and of 32 points, k whole, by thirds and by chains (the batch and its first points
+    take different plans): the same bits for the first points."""
+    g = torch.Generator(device="cuda").manual_seed(P + n + K)
+    A = torch.randn((K, P + P % 2), dtype=torch.float64, device="cuda", generator=g)
+    B = torch.randn((K, n), dtype=torch.float64, device="cuda", generator=g)
+    off = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    Ys = []
+    for p in (P, 600, 70, 1):
+        nb = N.c_i64()
+        N.check(N.fn["sbi_contract_f64_workspace"](p, n, K, ctypes.byref(nb)), "workspace")
+        W = torch.full((max(nb.value, 8) // 8,), float("nan"), dtype=torch.float64, device="cuda")
+        Y = torch.full((p, n), float("nan"), dtype=torch.float64, device="cuda")
+        N.check(N.fn["sbi_contract_f64_ws"](A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0),
+                                            off.data_ptr(), Y.data_ptr(), n, p, n, K, W.data_ptr(),
+                                            nb.value, st), "contract")
+        Ys.append(Y)
+    ref, scale = _ref(A[:, :P].contiguous(), B, off)
+    assert ((Ys[0] - ref).abs() <= (K + 8) * 2.0 ** -53 * (scale + off.abs())).all()
+    for Y in Ys[1:]:
+        assert torch.equal(Y, Ys[0][: len(Y)])
