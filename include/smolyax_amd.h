@@ -430,6 +430,7 @@ int sbi_bary_basis_f32(const sbi_plan* plan, const double* x, int64_t P, int64_t
  * with A the basis matrix written by sbi_newton_basis / sbi_bary_basis_* (K x P, row stride lda)
  * and B the coefficients (K x n, row stride ldb), both of dtype 0 (FP64, FP64 MFMA) or 1 (FP32,
  * FP32 MFMA with the partial sums added into FP64 every 256 terms); Y is FP64 (row stride ldy).
+ * FP64: chains of 256 terms, added in the order of k.
  * Replaces the dense GEMM that follows the per-point weights in the reference's evaluation
  * (barycentric.py:69-123 contracts F with the weight tensors block by block).  Each row of Y
  * depends only on its own column of A, summed in a fixed order, so a point's result is the same
@@ -441,7 +442,8 @@ int sbi_contract(const void* A, int64_t lda, const void* B, int64_t ldb, const d
 
 /* sbi_contract with FP64 operands and a workspace: when the P x n tiles are too few to fill the GPU,
  * the k range is spread over extra workgroups that write their partial sums to `workspace`, and a
- * second kernel adds them in sbi_contract's order (the same bits).  sbi_contract_f64_workspace sets
+ * second kernel adds them: chains of 256 terms into thirds of K, then the thirds, in that order with
+ * and without a workspace (the same bits).  sbi_contract_f64_workspace sets
  * *bytes to what it needs for a shape (0: not used); with less (or NULL) nothing is spread.
  * The operands are copied 16 bytes at a time when both bases are 16-byte aligned, both row strides
  * even, and each is at least its width rounded up to two: every row, the last one included, must

@@ -575,7 +575,7 @@ int contract_split_launch(const SplitPlan& sp, const float* A, int64_t lda, cons
 // on one XCD (its L2 serves their A rows).
 //
 // LDS image of a chunk: rows of the tile's width; the 16-byte slot q of row r holds the elements
-// of slot q ^ (8 * (r & 1)), so the two rows that half a wave reads together lie in different
+// of slot q ^ (8 * ((r >> 2) & 1)) (step s multiplies rows s, 4 + s, 8 + s, 12 + s), so the two rows that half a wave reads together lie in different
 // halves of the banks.  kDirect = false: row strides, widths or bases that are not multiples of
 // 16 bytes go through registers (8-byte loads one chunk ahead); the same image, the same bits.
 //
@@ -584,6 +584,7 @@ int contract_split_launch(const SplitPlan& sp, const float* A, int64_t lda, cons
 // kFlushK) + 3 terms.  Grids that would leave CUs idle spread k over workgroups (f64_plan), a
 // slice or some chains each; they write the sums of these units to `part` and
 // contract_reduce_kernel adds them in the same order: the same bits for any P, alone or in a batch.
+// `ordered` (sbi_contract): one slice, the chains added in order, never spread.
 // ------------------------------------------------------------------------------------------
 constexpr int kF64Slices = 3;
 constexpr int kF64Buf = 3;
@@ -649,7 +650,7 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64
     const int T = isA ? TM : TN;
     const int pos = (isA ? c : c - nA) * 128 + lane * 2;
     const int64_t org = isA ? m0 : n0;
-    const int64_t at = org + (((pos % T) / 2) ^ (8 * (krow(i) & 1))) * 2, end = isA ? P : n;
+    const int64_t at = org + (((pos % T) / 2) ^ (8 * ((krow(i) >> 2) & 1))) * 2, end = isA ? P : n;
     if (!kDirect && at + 1 >= end) odd |= 1u << i;
     col[i] = (off_t)((min(at, kDirect ? (end - 1) & ~(int64_t)1 : end - 1) - org) * 8);
     voff[i] = col[i] + (off_t)krow(i) * (off_t)((isA ? lda : ldb) * 8);
@@ -728,19 +729,19 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64
     each([&](int fm, int fn) { total[fm][fn] = v4d{0, 0, 0, 0}; });
     uint32_t pa[M], pb[WN];  // byte offsets of this lane's elements in a buffer
 #pragma unroll
-    for (int fm = 0; fm < M; ++fm) pa[fm] = (uint32_t)(g * TM + ((mw + fm * 16 + li) ^ sw)) * 8;
+    for (int fm = 0; fm < M; ++fm) pa[fm] = (uint32_t)(4 * g * TM + ((mw + fm * 16 + li) ^ sw)) * 8;
 #pragma unroll
-    for (int fn = 0; fn < WN; ++fn) pb[fn] = (uint32_t)(kA + (g * TN + ((nw + fn * 16 + li) ^ sw)) * 8);
+    for (int fn = 0; fn < WN; ++fn) pb[fn] = (uint32_t)(kA + (4 * g * TN + ((nw + fn * 16 + li) ^ sw)) * 8);
     auto compute = [&](int c, bool tail) {
       const char* buf = smem + bi * kStep;
 #pragma unroll
       for (int s = 0; s < kChunk / 4; ++s) {
         double a[M], b[WN];
 #pragma unroll
-        for (int fm = 0; fm < M; ++fm) a[fm] = *(const double*)(buf + pa[fm] + s * 32 * TM);
+        for (int fm = 0; fm < M; ++fm) a[fm] = *(const double*)(buf + pa[fm] + s * 8 * TM);
 #pragma unroll
-        for (int fn = 0; fn < WN; ++fn) b[fn] = *(const double*)(buf + pb[fn] + s * 32 * TN);
-        if (tail && (int64_t)c * kChunk + 4 * s + g >= K) {
+        for (int fn = 0; fn < WN; ++fn) b[fn] = *(const double*)(buf + pb[fn] + s * 8 * TN);
+        if (tail && (int64_t)c * kChunk + 4 * g + s >= K) {
 #pragma unroll
           for (int fm = 0; fm < M; ++fm) a[fm] = 0.0;
 #pragma unroll
@@ -885,9 +886,9 @@ f64_kernel_t f64_kernel(int wm, int split) {
 
 // padded: every row of A (B) is readable up to P (n) rounded up to a multiple of two.
 int contract_f64(const double* A, int64_t lda, const double* B, int64_t ldb, const double* offset,
-                 double* Y, int64_t ldy, int64_t P, int64_t n, int64_t K, bool padded, void* ws,
-                 int64_t ws_bytes, hipStream_t st) {
-  F64Plan pl = f64_plan(P, n, K);
+                 double* Y, int64_t ldy, int64_t P, int64_t n, int64_t K, bool padded, bool ordered,
+                 void* ws, int64_t ws_bytes, hipStream_t st) {
+  F64Plan pl = f64_plan(P, n, K, !ordered);
   if (!ws || ws_bytes < pl.bytes) pl = f64_plan(P, n, K, false);
   const bool direct = K == 0 || (((uintptr_t)A | (uintptr_t)B) % 16 == 0 && lda % 2 == 0 &&
                                  ldb % 2 == 0 && std::max(lda, ldb) < (1 << 24) &&  // 32-bit offsets
@@ -905,7 +906,7 @@ int contract_f64(const double* A, int64_t lda, const double* B, int64_t ldb, con
                                        : (direct ? f64_kernel<2, true>(wm, pl.split)
                                                  : f64_kernel<2, false>(wm, pl.split));
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * kWaves), 0, st, A, lda, B, ldb, offset,
-                     Y, ldy, P, n, K, (int)ntm, (int)ntn, (int)pl.nz, f64_slice(K), pl.upz, (double*)ws);
+                     Y, ldy, P, n, K, (int)ntm, (int)ntn, (int)pl.nz, ordered ? std::max<int64_t>(K, 1) : f64_slice(K), pl.upz, (double*)ws);
   SBI_HIP_CHECK(hipGetLastError());
   if (pl.nz > 1) {
     const int64_t rg = std::min<int64_t>((P * n + 255) / 256, 4096);
@@ -1393,7 +1394,7 @@ extern "C" int sbi_contract(const void* A, int64_t lda, const void* B, int64_t l
   hipStream_t st = (hipStream_t)stream;
   if (dtype == 0)
     return contract_f64((const double*)A, lda, (const double*)B, ldb, offset, Y, ldy, P, n, K,
-                        false, nullptr, 0, st);
+                        false, true, nullptr, 0, st);
   if (dtype == 1)
     return contract_launch<false>((const float*)A, lda, (const float*)B, ldb, offset, Y, ldy, P,
                                   n, K, nullptr, 0, nullptr, 0, 0, st);
@@ -1422,7 +1423,7 @@ extern "C" int sbi_contract_f64_ws(const double* A, int64_t lda, const double* B
   }
   if (P == 0 || n == 0) return SBI_OK;
   const bool padded = lda >= P + (P & 1) && ldb >= n + (n & 1);
-  return contract_f64(A, lda, B, ldb, offset, Y, ldy, P, n, K, padded, workspace, ws_bytes,
+  return contract_f64(A, lda, B, ldb, offset, Y, ldy, P, n, K, padded, false, workspace, ws_bytes,
                       (hipStream_t)stream);
 }
 

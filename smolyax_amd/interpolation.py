@@ -190,7 +190,7 @@ class SmolyakBarycentricInterpolator:
         zero = np.array([g(0)[0] for g in nf.node_gen], dtype=np.float64)
         X = np.stack([nf.grid_point(nu, zero) for nu in nf.nus])
         keep = self._n_inputs
-        Y = self.evaluate(torch.as_tensor(X, device=self._device), precision="fp64")
+        Y = self._evaluate(torch.as_tensor(X, device=self._device), "fp64", ordered=True)
         self._n_inputs = keep
         self._set_surpluses(nf, Y)
         return nf
@@ -226,11 +226,11 @@ class SmolyakBarycentricInterpolator:
         # points from the nodes' measure only: far out, the polynomial's own size sets the scale
         X = torch.as_tensor(self._proxy_samples()[: PROXY_SAMPLES // 2], device=self._device)
         keep, warned = self._n_inputs, self._warned_mixed
-        ref = self.evaluate(X, precision="newton-fp64" if self._newton_fp64_ok else "fp64")
+        ref = self._evaluate(X, "newton-fp64" if self._newton_fp64_ok else "fp64", ordered=True)
         scale = float(ref.abs().max()) or 1.0
         NL = self._nlayout
         while True:
-            err = float((self.evaluate(X, precision="mixed") - ref).abs().max()) / scale
+            err = float((self._evaluate(X, "mixed") - ref).abs().max()) / scale
             self._mixed_err = err
             if err <= MIXED_TARGET or NL.n_head >= NL.basis_n:
                 break
@@ -268,9 +268,9 @@ class SmolyakBarycentricInterpolator:
         Gauss-Hermite ones; at degree ~30 it reaches ~1e-8)."""
         X = torch.as_tensor(self._proxy_samples(), device=self._device)
         keep = self._n_inputs
-        y64 = self.evaluate(X, precision="fp64")
+        y64 = self._evaluate(X, "fp64", ordered=True)
         self._newton_fp64_ok = True  # for this measurement only
-        yn = self.evaluate(X, precision="newton-fp64")
+        yn = self._evaluate(X, "newton-fp64", ordered=True)
         self._n_inputs = keep
         scale = float(y64.abs().max())
         err = float((yn - y64).abs().max()) / scale if scale > 0 else float((yn - y64).abs().max())
@@ -550,7 +550,12 @@ class SmolyakBarycentricInterpolator:
 
     def evaluate(self, x, precision: str = None) -> torch.Tensor:
         """Evaluate on a chosen path (see the constructor's `precision`)."""
-        precision = precision or self._precision
+        return self._evaluate(x, precision or self._precision)
+
+    def _evaluate(self, x, precision, ordered=False):
+        """`evaluate`; ordered: FP64 sums of several outputs block by block and in the order of k,
+        which fixes the bits of what set_f derives from them (a proxy's surpluses, which the FP32
+        rounding of "mixed" makes visible) whatever the fastest split of the sums is."""
         if precision not in PRECISIONS:
             raise ValueError(f"precision must be one of {PRECISIONS}")
         if precision == "mixed" and self._nplan is None:
@@ -558,7 +563,7 @@ class SmolyakBarycentricInterpolator:
                 warnings.warn(f"precision 'mixed': the Newton form is unavailable "
                               f"({self._newton_off}); evaluating with 'bary-fp32' (FP32 "
                               f"barycentric, about 1e-4 relative)", SmolyaxPrecisionWarning,
-                              stacklevel=2)
+                              stacklevel=3)
                 self._warned_mixed = True
             precision = "bary-fp32"
         # On nested nodes the Newton form is the same polynomial with 5 to 7 times fewer terms and
@@ -587,7 +592,7 @@ class SmolyakBarycentricInterpolator:
                 or (precision != "fp64" and self._d_out > 1))
         if not gemm:
             y = torch.empty((P, self._d_out), dtype=torch.float64, device=self._device)
-            if precision == "fp64" and self._desc.n_share:
+            if precision == "fp64" and self._desc.n_share and not ordered:
                 ws = N.fn["sbi_bary_eval_few_workspace"](self._plan, P)
                 W = torch.empty(ws, dtype=torch.uint8, device=self._device) if ws else None
                 N.check(N.fn["sbi_bary_eval_few_f64"](self._plan, x.data_ptr(), P, x.stride(0),
@@ -597,19 +602,19 @@ class SmolyakBarycentricInterpolator:
                 rc = N.fn["sbi_bary_eval_f64"](self._plan, x.data_ptr(), P, x.stride(0),
                                                y.data_ptr(), self._stream())
                 if rc == N.SBI_ERR_CAPACITY:  # prefix table too large for LDS: GEMM form
-                    return self._eval_bary_gemm(x)
+                    return self._eval_bary_gemm(x, ordered=ordered)
                 N.check(rc, "eval")
             else:
                 fn = "sbi_newton_eval_mixed" if precision == "mixed" else "sbi_newton_eval_f64"
                 rc = N.fn[fn](self._nplan, x.data_ptr(), P, x.stride(0), y.data_ptr(),
                               self._stream())
                 if rc == N.SBI_ERR_CAPACITY:  # internal-node table beyond LDS: GEMM form
-                    return self._eval_newton_gemm(x, precision)
+                    return self._eval_newton_gemm(x, precision, ordered)
                 N.check(rc, precision)
             return y
         if precision == "fp64":
-            return self._eval_bary_gemm(x)
-        return self._eval_newton_gemm(x, precision)
+            return self._eval_bary_gemm(x, ordered=ordered)
+        return self._eval_newton_gemm(x, precision, ordered)
 
     def _point_chunk(self, rows, itemsize, P):
         """Points per chunk so that the basis matrix stays within memory_limit GiB, and within
@@ -631,13 +636,14 @@ class SmolyakBarycentricInterpolator:
         ld = cols + (cols & 1) if dtype == torch.float64 else cols
         return torch.empty((rows, ld), dtype=dtype, device=device)[:, :cols]
 
-    def _contract(self, A, B, offset, y):
+    def _contract(self, A, B, offset, y, ordered=False):
         """y[P, n] = offset + A^T B on the matrix cores (sbi_contract_f64_ws; sbi_contract for FP32
-        operands with FP64 accumulation; rows independent of the batch)."""
+        operands with FP64 accumulation and, ordered, for FP64 sums in the order of k; rows
+        independent of the batch)."""
         ld = self._ld
         off = None if offset is None else offset.data_ptr()
         (P, n), K = y.shape, A.shape[0]
-        if A.dtype == torch.float64:
+        if A.dtype == torch.float64 and not ordered:
             nb = N.c_i64()
             N.check(N.fn["sbi_contract_f64_workspace"](P, n, K, ctypes.byref(nb)), "contract")
             ws = nb.value
@@ -648,9 +654,10 @@ class SmolyakBarycentricInterpolator:
                     "contract")
             return
         N.check(N.fn["sbi_contract"](A.data_ptr(), ld(A), B.data_ptr(), ld(B), off, y.data_ptr(),
-                                     ld(y), P, n, K, 1, self._stream()), "contract")
+                                     ld(y), P, n, K, int(A.dtype == torch.float32), self._stream()),
+                "contract")
 
-    def _eval_bary_gemm(self, x, fp32=False, out=None):
+    def _eval_bary_gemm(self, x, fp32=False, out=None, ordered=False):
         """y = offset + W F: barycentric entry weights (HIP kernel), then the contraction with the
         zeta-scaled values on the matrix cores (FP64, or FP32 operands with FP64 accumulation)."""
         P = x.shape[0]
@@ -672,7 +679,7 @@ class SmolyakBarycentricInterpolator:
             WT = self._rows_buffer(K, b - a, dt, self._device)
             N.check(N.fn[fn](self._plan, xc.data_ptr(), b - a, xc.stride(0), WT.data_ptr(),
                              WT.stride(0), self._stream()), "bary_basis")
-            self._contract(WT, F, self._dev["offset"], y[a:b])
+            self._contract(WT, F, self._dev["offset"], y[a:b], ordered)
         return y
 
     def _surpluses(self, kind, gemm=False):
@@ -725,7 +732,7 @@ class SmolyakBarycentricInterpolator:
             self._Sg["bf16k8"] = S
         return S
 
-    def _eval_newton_gemm(self, x, precision):
+    def _eval_newton_gemm(self, x, precision, ordered=False):
         """y = H S: Newton basis matrix (HIP kernel), then the contraction with the surpluses on
         the matrix cores: sbi_contract for FP64; for "mixed" (FP32) and "bf16" the heaviest rows
         in FP64 (sbi_newton_rows_f64, FP64 MFMA) and the rest in FP32 or BF16, k-interleaved
@@ -746,7 +753,7 @@ class SmolyakBarycentricInterpolator:
                 N.check(N.fn["sbi_newton_basis_rows"](self._nplan, xc.data_ptr(), b - a,
                                                       xc.stride(0), 0, Nn, HT.data_ptr(),
                                                       HT.stride(0), 0, st), "basis")
-                self._contract(HT, S, None, y[a:b])
+                self._contract(HT, S, None, y[a:b], ordered)
             return y
         if kind == "f32":  # one call per chunk: head rows, FP32 rows, contraction
             pc = self._point_chunk(self._ndesc.gemm_kq + 2 * self._ndesc.gemm_head, 4, P)

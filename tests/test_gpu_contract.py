@@ -280,8 +280,8 @@ def test_contract_bf16_tile_shapes_same_bits(gpu):
                                    (130, 7, 4096), (777, 40, 5003), (5000, 160, 4100)])
 def test_contract_f64_ws_same_bits_for_every_split_and_alignment(gpu, P, n, K):
     """sbi_contract_f64_ws: k spread over workgroups (by 256-term chains or by thirds, as the
-    shape asks) and 16-byte copies with a spare element per odd row, against sbi_contract (no
-    workspace, 8-byte loads where a width is odd): the same bits; and against the FP64 product.
+    shape asks) and 16-byte copies with a spare element per odd row, against a call
+    without (8-byte loads where a width is odd): the same bits; and against the FP64 product.
     Bound: (K + 8) * 2^-53 of sum |A| |B| per element (one rounding per term, any order)."""
     g = torch.Generator(device="cuda").manual_seed(P + 3 * n + 7 * K)
     A = torch.randn((K, P + P % 2), dtype=torch.float64, device="cuda", generator=g)
@@ -297,7 +297,10 @@ def test_contract_f64_ws_same_bits_for_every_split_and_alignment(gpu, P, n, K):
                                         off.data_ptr(), Y.data_ptr(), n, P, n, K, W.data_ptr(),
                                         nb.value, st), "contract")
     Ac, Bc = A[:, :P].contiguous(), B[:, :n].contiguous()
-    assert torch.equal(Y, contract(Ac, Bc, off))
+    Z = torch.full((P, n), float("nan"), dtype=torch.float64, device="cuda")
+    N.check(N.fn["sbi_contract_f64_ws"](Ac.data_ptr(), P, Bc.data_ptr(), n, off.data_ptr(),
+                                        Z.data_ptr(), n, P, n, K, None, 0, st), "contract")
+    assert torch.equal(Y, Z)
     ref, scale = _ref(Ac, Bc, off)
     assert ((Y - ref).abs() <= (K + 8) * 2.0 ** -53 * (scale + off.abs())).all()
 
