@@ -588,6 +588,7 @@ int contract_split_launch(const SplitPlan& sp, const float* A, int64_t lda, cons
 // ------------------------------------------------------------------------------------------
 constexpr int kF64Slices = 3;
 constexpr int kF64Buf = 3;
+constexpr int kPanel = 4;  // point tiles an XCD works on side by side (contract_k4_kernel)
 // k per slice (the last one may be shorter): whole chunks, one slice up to three chains
 inline int64_t f64_slice(int64_t K) {
   if (K <= kF64Slices * kFlushK) return std::max<int64_t>(K, 1);
@@ -917,6 +918,167 @@ int contract_f64(const double* A, int64_t lda, const double* B, int64_t ldb, con
   return SBI_OK;
 }
 
+// ------------------------------------------------------------------------------------------
+// FP32 contraction with k-interleaved operands, staged in LDS: contract_kernel<., true> with
+// other tiles and the same sums (the FP64 head first, chains of kFlushK terms from the FP32
+// MFMA added into FP64 in order), so the same bits.  Bound: v_mfma_f32_16x16x4, 32 cycles of a SIMD.
+// A workgroup of 4 waves (2 x 2) owns 32 WM points x 32 WN outputs; a chunk of 4 KQ k is copied into
+// one of three LDS buffers by direct 16-byte loads two chunks ahead (one barrier per chunk, as in
+// contract_f64_kernel), and one 16-byte LDS read gives a lane its operand of four steps.
+// The output tiles run over XCDs by point tile, four point tiles at a time, so that the chunks of A
+// and B that an XCD's workgroups read at about the same time fit its L2.
+// 4096 x 4096, K 9986: 3.24 ms with each wave loading its own fragments from L2, 2.78 ms with 4 x 4
+// fragments per wave (matrix cores busy 85 % of the time at 2.15 GHz), 2.95 with 4 x 2, 3.08 with 2 x
+// 2 and chunks of 32 k; 5000 x 256, K 5000 (316 tiles of 2 x 2): 232 -> 212 us.  No gain from four to
+// eight buffers or from reading the next chunk's fragments ahead of the MFMAs.
+// ------------------------------------------------------------------------------------------
+template <int WM, int WN, int KQ>
+__global__ __launch_bounds__(64 * kWaves, WM * WN > 8 ? 2 : 3) void contract_k4_kernel(
+    const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
+    const double* __restrict__ offset, double* __restrict__ Y, int64_t ldy, int64_t P, int64_t n,
+    int64_t K, const double* __restrict__ A64, int64_t lda64, const double* __restrict__ B64,
+    int64_t ldb64, int64_t K64, int ntm, int ntn) {
+  constexpr int TM = 32 * WM, TN = 32 * WN;
+  constexpr int kA = KQ * TM * 16, kStep = kA + KQ * TN * 16;  // bytes of a chunk: A, then B
+  constexpr int nA = kA / 1024, kPer = kStep / 4096;         // 1 KB copies: of A, per wave
+  static_assert(nA % 4 == 0 && kStep % 4096 == 0, "whole copies per wave");
+  __shared__ __attribute__((aligned(16))) char smem[kF64Buf * kStep];
+  // tile t of this XCD's: its point tiles in panels (the last one may be narrower), a panel's tiles
+  // output by output; no workgroup without a tile but at the end, so that none of the CUs, which
+  // take the workgroups in turn, is left with those
+  const int xcd = blockIdx.x & 7, t = blockIdx.x >> 3;
+  const int own = (ntm - xcd + 7) / 8;
+  if (t >= own * ntn) return;
+  const int first = t / (kPanel * ntn) * kPanel, width = min(kPanel, own - first);
+  const int in_panel = t - first * ntn;
+  const int tn = in_panel / width, tm = (first + in_panel % width) * 8 + xcd;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, g = lane >> 4;
+  const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
+  const int mw = (wave & 1) * (16 * WM), nw = (wave >> 1) * (16 * WN);
+
+  // copies: scalar base plus this lane's fixed offset (columns past the edge re-read the last one)
+  const char* baseA = (const char*)(A + m0 * 4);
+  const char* baseB = (const char*)(B + n0 * 4);
+  const int KR = (int)(K / 4), KC = (KR + KQ - 1) / KQ;  // rows of four k, chunks
+  uint64_t voff[kPer];
+  auto offsets = [&](int rows) {  // rows of the chunk (all but the last one: KQ)
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const bool isA = 4 * i < nA;
+      const int idx = (isA ? wave + 4 * i : wave + 4 * i - nA) * 64 + lane;
+      const int T = isA ? TM : TN;
+      const int64_t at = min((isA ? m0 : n0) + idx % T, (isA ? P : n) - 1) - (isA ? m0 : n0);
+      voff[i] = (uint64_t)(min(idx / T, rows - 1) * (isA ? lda : ldb) + at) * 16;
+    }
+  };
+  offsets(KQ);
+  int ci = 0;  // the next chunk to be copied
+  auto issue = [&](int b) {
+    if (ci >= KC) return;
+    if (KQ > 4 && (ci + 1) * KQ > KR) offsets(KR - ci * KQ);
+    char* dst = smem + b * kStep + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      __builtin_amdgcn_global_load_lds((const void*)((4 * i < nA ? baseA : baseB) + voff[i]),
+                                       (lds_void*)(dst + i * 4096), 16, 0, 0);
+    baseA += lda * (16 * KQ);
+    baseB += ldb * (16 * KQ);
+    ++ci;
+  };
+
+  issue(0);
+  issue(1);
+
+  v4d sum[WM][WN];
+#pragma unroll
+  for (int fm = 0; fm < WM; ++fm)
+#pragma unroll
+    for (int fn = 0; fn < WN; ++fn) sum[fm][fn] = v4d{0, 0, 0, 0};
+  if (K64 > 0) {
+    int64_t ph[WM], jcol[WN];
+#pragma unroll
+    for (int fm = 0; fm < WM; ++fm)
+      ph[fm] = min(m0 + mw + fm * 16 + 4 * (li & 3) + (li >> 2), P - 1);
+#pragma unroll
+    for (int fn = 0; fn < WN; ++fn) jcol[fn] = min(n0 + nw + fn * 16 + li, n - 1);
+    head_fp64<WM, WN>(A64, lda64, B64, ldb64, K64, g, ph, jcol, sum);
+  }
+
+  uint32_t pa[WM], pb[WN];  // byte offsets of this lane's operands in a buffer
+#pragma unroll
+  for (int fm = 0; fm < WM; ++fm) pa[fm] = (uint32_t)(g * TM + mw + fm * 16 + li) * 16;
+#pragma unroll
+  for (int fn = 0; fn < WN; ++fn) pb[fn] = (uint32_t)(kA + (g * TN + nw + fn * 16 + li) * 16);
+  v4f acc[WM][WN];
+  int bi = 0;
+  for (int c0 = 0; c0 < KC; c0 += kFlushK / (4 * KQ)) {
+    const int c1 = min(KC, c0 + kFlushK / (4 * KQ));
+#pragma unroll
+    for (int fm = 0; fm < WM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < WN; ++fn) acc[fm][fn] = v4f{0, 0, 0, 0};
+    for (int c = c0; c < c1; ++c) {
+      if (c + 1 < KC) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_barrier" ::: "memory");
+      issue(bi == 0 ? kF64Buf - 1 : bi - 1);
+#pragma unroll
+      for (int h = 0; h < KQ / 4; ++h) {  // 16 k
+        if (h && c * KQ + 4 * h >= KR) break;
+        const char* buf = smem + bi * kStep;
+        v4f a[WM], b[WN];
+#pragma unroll
+        for (int fm = 0; fm < WM; ++fm) a[fm] = *(const v4f*)(buf + pa[fm] + h * (64 * TM));
+#pragma unroll
+        for (int fn = 0; fn < WN; ++fn) b[fn] = *(const v4f*)(buf + pb[fn] + h * (64 * TN));
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int fm = 0; fm < WM; ++fm)
+#pragma unroll
+            for (int fn = 0; fn < WN; ++fn) acc[fm][fn] = mfma(a[fm][s], b[fn][s], acc[fm][fn]);
+        __builtin_amdgcn_s_setprio(0);
+      }
+      bi = bi + 1 == kF64Buf ? 0 : bi + 1;
+    }
+#pragma unroll
+    for (int fm = 0; fm < WM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < WN; ++fn)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[fm][fn][r] += (double)acc[fm][fn][r];
+  }
+#pragma unroll
+  for (int fn = 0; fn < WN; ++fn) {
+    const int64_t col = n0 + nw + fn * 16 + li;
+    if (col >= n) continue;
+    const double off = offset ? offset[col] : 0.0;
+#pragma unroll
+    for (int fm = 0; fm < WM; ++fm)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t row = m0 + mw + fm * 16 + 4 * g + r;
+        if (row < P) Y[row * ldy + col] = off + sum[fm][fn][r];
+      }
+  }
+}
+
+template <int WM, int WN, int KQ>
+void contract_k4_launch(const float* A, int64_t lda, const float* B, int64_t ldb,
+                        const double* offset, double* Y, int64_t ldy, int64_t P, int64_t n,
+                        int64_t K, const double* A64, int64_t lda64, const double* B64,
+                        int64_t ldb64, int64_t K64, hipStream_t st) {
+  const int64_t ntm = (P + 32 * WM - 1) / (32 * WM), ntn = (n + 32 * WN - 1) / (32 * WN);
+  const int64_t grid = (ntm + 7) / 8 * 8 * ntn;
+  hipLaunchKernelGGL((contract_k4_kernel<WM, WN, KQ>), dim3((unsigned)grid), dim3(64 * kWaves), 0, st, A,
+                     lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64, (int)ntm,
+                     (int)ntn);
+}
+
 template <bool kK4 = false>
 int contract_launch(const float* A, int64_t lda, const float* B, int64_t ldb, const double* offset,
                     double* Y, int64_t ldy, int64_t P, int64_t n, int64_t K, const double* A64,
@@ -927,11 +1089,31 @@ int contract_launch(const float* A, int64_t lda, const float* B, int64_t ldb, co
   if (tn == 32) {
     hipLaunchKernelGGL((contract_kernel<1, kK4>), dim3(gm, (unsigned)((n + 31) / 32)), block, 0, st,
                        A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64);
+  } else if constexpr (kK4) {
+    // the tile that takes least: workgroups per CU that run side by side at the full rate, fewer at
+    // the end at less (4 x 4 fragments: two per CU, one alone at 0.7; else three, two at 0.7, one at
+    // 0.6), the smaller tiles at 0.94 and 0.88 of the largest one's rate.  12 000 x 900, K 5000: 1.36
+    // ms with 4 x 4 fragments (752 workgroups, three per CU), 1.19 with 4 x 2 (whole evaluations).
+    auto cost = [&](int64_t tm, int64_t tn, double size, int slots, double one, double two) {
+      const int64_t q = ((P + tm - 1) / tm * ((n + tn - 1) / tn) + 255) / 256, rest = q % slots;
+      return size * ((double)(q - rest) + (rest == 1 ? one : rest == 2 ? two : 0.0));
+    };
+    const double c44 = cost(128, 128, 4.0, 2, 1.4, 0.0), c42 = cost(128, 64, 2.0 / 0.94, 3, 1.6, 2.8),
+                 c22 = cost(64, 64, 1.0 / 0.88, 3, 1.7, 2.8);
+    if (c44 <= std::min(c42, c22))
+      contract_k4_launch<4, 4, 4>(A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64,
+                                  K64, st);
+    else if (c42 <= c22)
+      contract_k4_launch<4, 2, 4>(A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64,
+                                  K64, st);
+    else
+      contract_k4_launch<2, 2, 8>(A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64,
+                                  K64, st);
   } else if (tn == 64) {
-    hipLaunchKernelGGL((contract_kernel<2, kK4>), dim3(gm, (unsigned)((n + 63) / 64)), block, 0, st,
-                       A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64);
+    hipLaunchKernelGGL((contract_kernel<2, false>), dim3(gm, (unsigned)((n + 63) / 64)), block, 0,
+                       st, A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64);
   } else {
-    hipLaunchKernelGGL((contract_kernel<4, kK4>), dim3(gm, (unsigned)((n + 127) / 128)), block, 0,
+    hipLaunchKernelGGL((contract_kernel<4, false>), dim3(gm, (unsigned)((n + 127) / 128)), block, 0,
                        st, A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64);
   }
   SBI_HIP_CHECK(hipGetLastError());

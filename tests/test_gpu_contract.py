@@ -329,3 +329,25 @@ def test_contract_f64_points_alone_and_in_a_batch(gpu, P, n, K):
     assert ((Ys[0] - ref).abs() <= (K + 8) * 2.0 ** -53 * (scale + off.abs())).all()
     for Y in Ys[1:]:
         assert torch.equal(Y, Ys[0][: len(Y)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("P,n,K64,K32", [(4095, 2047, 3, 272), (5999, 2041, 0, 80), (5001, 251, 64, 528),
+                                         (65, 33, 1, 16), (16001, 300, 5, 1040)])
+def test_contract_split_k4_tiles_equal_plain_layout(gpu, P, n, K64, K32):
+    """Every tile of the LDS-staged FP32 contraction (4 x 4, 4 x 2 and 2 x 2 fragments per wave) at
+    ragged edges, with half of the last chunk of 32 k: the same bits as the plain layout."""
+    g = torch.Generator(device="cuda").manual_seed(P + n + K32)
+    A64 = torch.randn((max(K64, 1), P), dtype=torch.float64, device="cuda", generator=g)[:K64]
+    B64 = torch.randn((max(K64, 1), n), dtype=torch.float64, device="cuda", generator=g)[:K64]
+    A32 = torch.randn((K32, P), dtype=torch.float32, device="cuda", generator=g)
+    B32 = torch.randn((K32, n), dtype=torch.float32, device="cuda", generator=g)
+    off = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
+    Y0 = contract_split(A64.contiguous(), B64.contiguous(), A32, B32, off)
+    A4, B4 = _k4(A32, K32), _k4(B32, K32)
+    Y1 = torch.full((P, n), float("nan"), dtype=torch.float64, device="cuda")
+    N.check(N.fn["sbi_contract_split_k4"](
+        A64.data_ptr() if K64 else None, P, B64.data_ptr() if K64 else None, n, K64, A4.data_ptr(),
+        P, B4.data_ptr(), n, K32, off.data_ptr(), Y1.data_ptr(), n, P, n,
+        torch.cuda.current_stream().cuda_stream), "k4")
+    assert torch.equal(Y0, Y1)
