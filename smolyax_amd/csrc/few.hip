@@ -247,7 +247,8 @@ __global__ __launch_bounds__(256) void bary_few_reduce_kernel(const double* __re
 // longer workgroups leave CUs idle at the end: 16 384 points, 14 shares, 40 inputs: 298 us one by
 // one, 351 us with all 14 in a workgroup (9000 points: 182 and 222 us).
 int shares_per_wg(const sbi_bary_desc& d, int64_t P) {
-  const bool alone = (P + kTile - 1) / kTile >= 2048 || d.n_share * P * d.d_out * 8 > (int64_t(256) << 20);
+  const bool alone = (P + kTile - 1) / kTile >= 2048 || d.n_share > 65535 ||  // (launch limit)
+                     d.n_share * P * d.d_out * 8 > (int64_t(256) << 20);
   return alone ? d.n_share : 1;
 }
 
