@@ -11,7 +11,8 @@
 // of A only, summed in a fixed order: a point's result does not depend on P, on its position in
 // the batch or on the batch's other points (bit for bit).
 //
-// FP64 operands: contract_f64_kernel (operands staged in LDS).  FP32: contract_kernel below.
+// FP64 operands: contract_f64_kernel; FP32 with k interleaved by four and more than 32 outputs:
+// contract_k4_kernel (both stage their operands in LDS).  Other FP32 calls: contract_kernel below.
 //
 // contract_kernel, work split: a workgroup of 4 waves owns a 64-point x (32*FN)-output tile of Y;
 // each wave a 32 x 16*FN sub-tile made of 2 x FN MFMA 16x16 fragments.
@@ -227,8 +228,7 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
     if constexpr (kK4) {
       // the chunks of one kFlushK run form an inner loop with the flush after it, so the MFMA
       // accumulators stay in the matrix-core registers across the run (a flush test inside the
-      // chunk loop made the compiler copy them to and from ordinary registers at every chunk:
-      // 4096 x 4096 outputs, K 10 016: 3.11 -> 2.90 ms).  The
+      // chunk loop made the compiler copy them to and from ordinary registers at every chunk).  The
       // plain FP32 layout keeps the flat loop (3.73 ms flat, 4.53 ms nested).  Same sums.
       for (int64_t kc = 0; kc < K16; kc += kFlushK) {
         const int64_t kce = min(K16, kc + (int64_t)kFlushK);
