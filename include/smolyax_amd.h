@@ -401,15 +401,18 @@ int sbi_newton_vjp(const sbi_newton_plan* plan, const double* x, int64_t P, int6
                    const void* GT, int64_t ldg, int32_t dtype, double* gx, void* workspace,
                    int64_t ws_bytes, void* stream);
 /* Bytes of device workspace sbi_newton_jacobian_f64 needs for P points and n outputs: the factor
- * table when it takes more than 40 KB per 64 points; for n <= 8 the partial sums of split dims;
- * for n > 8 the derivative basis D^T (adjoint entries x P). */
+ * table when it takes more than 40 KB per 64 points and the pass reads it from global memory; for
+ * n <= 8 the partial sums of split dims; for n > 8 the derivative basis D^T (adjoint entries x P
+ * rounded up to two), the partial sums of the jobs that share a group of dims (n_jac_slots x P x n x
+ * 8) and 8 bytes to align it.  The workspace is aligned for doubles. */
 int64_t sbi_newton_jacobian_workspace(const sbi_newton_plan* plan, int64_t P, int64_t n);
 /* Dense Jacobian of the Newton form, J[P, n, d_in] (FP64, contiguous), the reference's gradient
  * (interpolation.py:306-345, barycentric.py:126-229) of the same polynomial:
  *   J[p, o, j] = sum over nodes nu with a factor (j, k):  S[nu, o] h'_k(x_j) prod_{other (j',k')} h_k'(x_j')
  * S: surpluses [basis_n, lds], rows in the node order of the adjoint (the rows of G^T of
- * sbi_newton_vjp).  n <= 8: one pass over work units of at most 128 entries, sums in registers
- * (a dim split over several units adds their partial sums in unit order);
+ * sbi_newton_vjp); no element beyond column n - 1 of a row is read.  n <= 8: one pass over work units
+ * of at most 128 entries (jac_unit; 64 with the factor table in LDS, jt_unit), sums in registers (a dim
+ * split over several units adds their partial sums in unit order);
  * n > 8: D^T is written to the workspace and contracted on the FP64 matrix cores with the
  * entries' surplus rows, one group of rows per input dim, eight dims per workgroup.
  * J[p, :, j] = NaN where x_j is one of sing_x of dim j (the reference's result at a node
@@ -417,6 +420,12 @@ int64_t sbi_newton_jacobian_workspace(const sbi_newton_plan* plan, int64_t P, in
 int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double* x, int64_t P, int64_t ldx,
                             const double* S, int64_t lds, int64_t n, double* J, void* workspace,
                             int64_t ws_bytes, void* stream);
+/* The same (the same bits), for an S whose rows, the last one included, are readable up to n rounded
+ * up to two: for n > 8, with a 16-byte aligned S and an even lds > n, an odd number of outputs is then
+ * copied 16 bytes at a time too (the extra element is never used).  Other S: as above. */
+int sbi_newton_jacobian_f64_padded(const sbi_newton_plan* plan, const double* x, int64_t P,
+                                   int64_t ldx, const double* S, int64_t lds, int64_t n, double* J,
+                                   void* workspace, int64_t ws_bytes, void* stream);
 /* Barycentric entry weights W^T[k_raw, ldw] (FP64) at x[P, ldx]: y = offset + W F, the
  * reference's per-block contraction (barycentric.py:69-123) as one dense GEMM (large d_out). */
 int sbi_bary_basis_f64(const sbi_plan* plan, const double* x, int64_t P, int64_t ldx, double* WT,

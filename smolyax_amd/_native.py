@@ -116,6 +116,8 @@ SIGNATURES = {
     "sbi_newton_jacobian_workspace": (c_i64, [c_vp, c_i64, c_i64]),
     "sbi_newton_jacobian_f64": (c_i32, [c_vp, c_vp, c_i64, c_i64, c_vp, c_i64, c_i64, c_vp, c_vp,
                                         c_i64, c_vp]),
+    "sbi_newton_jacobian_f64_padded": (c_i32, [c_vp, c_vp, c_i64, c_i64, c_vp, c_i64, c_i64, c_vp, c_vp,
+                                        c_i64, c_vp]),
     "sbi_bary_basis_f64": (c_i32, [c_vp, c_vp, c_i64, c_i64, c_vp, c_i64, c_vp]),
     "sbi_bary_basis_f32": (c_i32, [c_vp, c_vp, c_i64, c_i64, c_vp, c_i64, c_vp]),
     "sbi_newton_mixed_staged": (c_i32, [c_vp]),

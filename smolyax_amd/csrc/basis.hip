@@ -1308,9 +1308,10 @@ extern "C" int64_t sbi_newton_jacobian_workspace(const sbi_newton_plan* plan, in
   const int64_t P64 = (P + kTile - 1) / kTile * kTile;
   if (jac_global_table(*dp) && !jac_tile_waves(*dp, n))
     bytes += (int64_t)dp->n_tab_rows * P64 * (int64_t)sizeof(double);
-  if (n > kJacDirectMax)  // D^T (row stride even), then the jobs' parts
+  if (n > kJacDirectMax)  // D^T (row stride even, on 16 bytes), then the jobs' parts
     bytes += (int64_t)dp->n_vjp_ent * jac_ld(P) * (int64_t)sizeof(double) +
-             (int64_t)dp->n_jac_slots * P * n * sbi::kJacGroup * (int64_t)sizeof(double);
+             (int64_t)dp->n_jac_slots * P * n * sbi::kJacGroup * (int64_t)sizeof(double) +
+             (int64_t)sizeof(double);
   else
     bytes += (int64_t)(jac_tile_waves(*dp, n) ? dp->n_jt_slots : dp->n_jac_partials) * P * n *
              (int64_t)sizeof(double);
@@ -1347,10 +1348,9 @@ static void jac_basis_launch(const sbi_newton_desc& d, const double* x, int64_t 
                      DT, jac_ld(P));
 }
 
-extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double* x, int64_t P,
-                                       int64_t ldx, const double* S, int64_t lds, int64_t n,
-                                       double* J, void* workspace, int64_t ws_bytes,
-                                       void* stream) {
+static int jacobian_launch(const sbi_newton_plan* plan, const double* x, int64_t P, int64_t ldx,
+                           const double* S, int64_t lds, bool padded, int64_t n, double* J,
+                           void* workspace, int64_t ws_bytes, void* stream) {
   const sbi_newton_desc* dp = nullptr;
   if (sbi_newton_plan_desc(plan, &dp) != SBI_OK || !x || !S || !J || P < 0 || n < 1 || lds < n ||
       ws_bytes < 0) {
@@ -1379,9 +1379,12 @@ extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double
   hipStream_t st = (hipStream_t)stream;
   const int waves = jac_tile_waves(d, n);
   const bool g = !waves && jac_global_table(d);
-  double* gtab = g ? (double*)workspace : nullptr;
+  // (D^T is copied 16 bytes at a time; the workspace only has to be aligned for doubles)
+  double* ws = (double*)(n > kJacDirectMax ? ((uintptr_t)workspace + 15) & ~(uintptr_t)15
+                                           : (uintptr_t)workspace);
+  double* gtab = g ? ws : nullptr;
   const int64_t P64 = (P + kTile - 1) / kTile * kTile;
-  double* DT = (double*)workspace + (g ? (int64_t)d.n_tab_rows * P64 : 0);
+  double* DT = ws + (g ? (int64_t)d.n_tab_rows * P64 : 0);
   if (g && d.n_tab_dims > 0) {
     const int64_t ny = std::min<int64_t>(d.n_tab_dims, 64);
     hipLaunchKernelGGL(newton_htab_kernel, dim3((unsigned)((P + 255) / 256), (unsigned)ny),
@@ -1432,7 +1435,7 @@ extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double
     // the rows of D^T by input dim (dims without entries get zeros)
     const sbi::JacRows rows{d.jac_row, d.jac_row_off, d.jac_row_end, d.jac_job, d.jac_group_red,
                             d.n_jac_jobs, d.n_jac_group_red};
-    const int rc = sbi::contract_jacobian_f64(DT, jac_ld(P), S, lds, rows, (int)d.d_in, J, P, n,
+    const int rc = sbi::contract_jacobian_f64(DT, jac_ld(P), S, lds, padded, rows, (int)d.d_in, J, P, n,
                                               DT + (int64_t)d.n_vjp_ent * jac_ld(P), st);
     if (rc != SBI_OK) return rc;
   }
@@ -1441,4 +1444,18 @@ extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double
                      d, x, P, ldx, n, J);
   SBI_HIP_CHECK(hipGetLastError());
   return SBI_OK;
+}
+
+extern "C" int sbi_newton_jacobian_f64(const sbi_newton_plan* plan, const double* x, int64_t P,
+                                       int64_t ldx, const double* S, int64_t lds, int64_t n,
+                                       double* J, void* workspace, int64_t ws_bytes,
+                                       void* stream) {
+  return jacobian_launch(plan, x, P, ldx, S, lds, false, n, J, workspace, ws_bytes, stream);
+}
+
+extern "C" int sbi_newton_jacobian_f64_padded(const sbi_newton_plan* plan, const double* x,
+                                              int64_t P, int64_t ldx, const double* S, int64_t lds,
+                                              int64_t n, double* J, void* workspace,
+                                              int64_t ws_bytes, void* stream) {
+  return jacobian_launch(plan, x, P, ldx, S, lds, true, n, J, workspace, ws_bytes, stream);
 }

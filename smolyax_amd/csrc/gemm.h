@@ -26,10 +26,10 @@ struct JacRows {
 // Jacobian contraction (gemm.hip), FP64 matrix cores: for each input dim z < nz, p < P, c < n,
 //   J[(p * n + c) * nz + z] = sum over the rows q of dim z of A[row[2 q] * lda + p] *
 //                                                            S[row[2 q + 1] * lds + c].
-// A dim with no rows gets zeros.  A is 16-byte aligned, lda even and at least P rounded up to two;
-// where S is 16-byte aligned and lds even and at least n rounded up to two, its rows are readable
-// up to that width.  part: P * n * kJacGroup doubles per slot.
-int contract_jacobian_f64(const double* A, int64_t lda, const double* S, int64_t lds,
+// A dim with no rows gets zeros.  A is 16-byte aligned, lda even and at least P rounded up to two.
+// padded: the caller promises that every row of S, the last one included, is readable up to n rounded
+// up to two.  part: P * n * kJacGroup doubles per slot.
+int contract_jacobian_f64(const double* A, int64_t lda, const double* S, int64_t lds, bool padded,
                           const JacRows& t, int nz, double* J, int64_t P, int64_t n, double* part,
                           hipStream_t st);
 

@@ -1323,7 +1323,8 @@ contract_bf16_wide_kernel(SBI_BF16_ARGS) {
 // global -> LDS loads (16-byte slots of odd rows rotated by 8, as in contract_f64_kernel); the row
 // table is copied the same way three chunks ahead of that, into each wave's own ring, and read
 // into registers a chunk before it is needed.  Every wave issues the same number of copies per
-// chunk, past the last one too (rows clamped), so the waits are counts.  kWide = false: S rows that do not start on 16 bytes are copied in 4-byte pieces.
+// chunk, past the last one too (rows clamped), so the waits are counts.  kWide = false: S rows that do not start on 16 bytes, or an odd number of outputs
+// without the promise of a spare element (jac_wide_rows), are copied in 4-byte pieces.
 //
 // The tile is written through LDS, one accumulator register of every dim at a time, so that eight
 // consecutive lanes write the kJacDims consecutive doubles of one (point, output): a lane writing
@@ -1537,7 +1538,7 @@ __global__ __launch_bounds__(256) void jac_group_reduce_kernel(const double* __r
 
 namespace sbi {
 
-int contract_jacobian_f64(const double* A, int64_t lda, const double* S, int64_t lds,
+int contract_jacobian_f64(const double* A, int64_t lda, const double* S, int64_t lds, bool padded,
                           const JacRows& t, int nz, double* J, int64_t P, int64_t n, double* part,
                           hipStream_t st) {
   if (P <= 0 || n <= 0 || nz <= 0) return SBI_OK;
@@ -1547,7 +1548,7 @@ int contract_jacobian_f64(const double* A, int64_t lda, const double* S, int64_t
     set_error("contract_jacobian_f64: launch too large");
     return SBI_ERR_INVALID;
   }
-  const bool wide = ((uintptr_t)S & 15) == 0 && lds % 2 == 0 && lds >= n + (n & 1);
+  const bool wide = jac_wide_rows(S, lds, n, padded);
   hipLaunchKernelGGL(wide ? jac_contract_kernel<true> : jac_contract_kernel<false>,
                      dim3((unsigned)grid), dim3(64 * kWaves), 0, st, A, (uint32_t)lda, S, lds, t, nz,
                      J, P, n, (int)ntp, (int)ntn, part);

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/smolyax_amd.h"
+#include "common.h"
 
 namespace {
 
@@ -156,6 +157,16 @@ void plan_paths() {
   expect(sbi_newton_plan_create(&n, &np) == SBI_ERR_INVALID, "newton plan with 4 waves");
 }
 
+// The 16-byte copies of a row of S read the element after an odd n: only with the caller's promise.
+void row_copies() {
+  alignas(16) static double s[64];
+  expect(sbi::jac_wide_rows(s, 10, 10, false), "even n, aligned rows");
+  expect(!sbi::jac_wide_rows(s, 10, 9, false), "odd n without the promise");
+  expect(sbi::jac_wide_rows(s, 10, 9, true), "odd n with the promise");
+  expect(!sbi::jac_wide_rows(s, 9, 9, true), "odd stride");
+  expect(!sbi::jac_wide_rows(s + 1, 10, 10, true), "rows off 16 bytes");
+}
+
 }  // namespace
 
 int main() {
@@ -165,6 +176,7 @@ int main() {
   index_case(30, 600);
   error_paths();
   plan_paths();
+  row_copies();
   if (failures) return 1;
   std::printf("ok\n");
   return 0;

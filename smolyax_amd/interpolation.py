@@ -916,10 +916,10 @@ class SmolyakBarycentricInterpolator:
             xc = x[p0:p1]
             nb = int(N.fn["sbi_newton_jacobian_workspace"](self._nplan, p1 - p0, n))
             ws = torch.empty(max(1, (nb + 7) // 8), dtype=torch.float64, device=self._device)
-            N.check(N.fn["sbi_newton_jacobian_f64"](self._nplan, xc.data_ptr(), p1 - p0,
-                                                    xc.stride(0), S.data_ptr(), S.stride(0), n,
-                                                    J[p0:p1].data_ptr(), ws.data_ptr(), nb,
-                                                    self._stream()), "jacobian")
+            # (S is a _rows_buffer: its rows have the spare element of an odd width)
+            N.check(N.fn["sbi_newton_jacobian_f64_padded"](
+                self._nplan, xc.data_ptr(), p1 - p0, xc.stride(0), S.data_ptr(), S.stride(0), n,
+                J[p0:p1].data_ptr(), ws.data_ptr(), nb, self._stream()), "jacobian")
 
     def integral(self) -> torch.Tensor:
         """interpolation.py:347-390: Q[d_out]; synchronises like the reference's block_until_ready."""
