@@ -13,6 +13,8 @@
 //
 // FP64 operands: contract_f64_kernel; FP32 with k interleaved by four and more than 32 outputs:
 // contract_k4_kernel (both stage their operands in LDS).  Other FP32 calls: contract_kernel below.
+// The staged loops' raw barriers wait for the wave's copies (vmcnt) and for its LDS reads (lgkmcnt): a
+// buffer that other waves copy into after the barrier has then been read.
 //
 // contract_kernel, work split: a workgroup of 4 waves owns a 64-point x (32*FN)-output tile of Y;
 // each wave a 32 x 16*FN sub-tile made of 2 x FN MFMA 16x16 fragments.
@@ -696,8 +698,8 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN < 4 ? 4 : 3) void contract_f64
   // chunk c has landed in every wave (the copies of the next one may be in flight)
   auto wait = [&](int c) {
     if constexpr (kDirect) {
-      if (c + 1 < ce) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (c + 1 < ce) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPer) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       asm volatile("s_barrier" ::: "memory");
     } else {
       __syncthreads();
@@ -1021,8 +1023,8 @@ __global__ __launch_bounds__(64 * kWaves, WM * WN > 8 ? 2 : 3) void contract_k4_
 #pragma unroll
       for (int fn = 0; fn < WN; ++fn) acc[fm][fn] = v4f{0, 0, 0, 0};
     for (int c = c0; c < c1; ++c) {
-      if (c + 1 < KC) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (c + 1 < KC) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPer) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       asm volatile("s_barrier" ::: "memory");
       issue(bi == 0 ? kF64Buf - 1 : bi - 1);
 #pragma unroll
@@ -1239,15 +1241,15 @@ __device__ __forceinline__ void contract_bf16_body(
         // this wave's copies of step s have landed once at most those of s + 1, s + 2 remain
         if (s + 2 < S) {
           issue(s + 2);
-          if constexpr (kPer == 4) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-          else if constexpr (kPer == 3) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-          else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+          if constexpr (kPer == 4) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+          else if constexpr (kPer == 3) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+          else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
         } else if (s + 1 < S) {
-          if constexpr (kPer == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-          else if constexpr (kPer == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-          else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+          if constexpr (kPer == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+          else if constexpr (kPer == 3) asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)" ::: "memory");
+          else asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
         } else {
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         }
         asm volatile("s_barrier" ::: "memory");  // every wave's copies of step s have landed
         const lds_v8bf* LA = (const lds_v8bf*)(smem + (s % kBfBuf) * kStep);
@@ -1441,7 +1443,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void jac_contract_kernel(
   const int endv = t.end[min(z0 + min(lane, kJacDims - 1), nz - 1)];
   int q = r0, c = 0, q0 = r0, b = 0;  // next row; its chunk, the chunk's first row and buffer
   auto begin = [&] {  // chunk c has landed in every wave (and row-table chunk c + 3); c + 2 is copied
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPer) : "memory");
     asm volatile("s_barrier" ::: "memory");
     copy(b == 0 ? 2 : b - 1);
     copy_rec(c + 5);
