@@ -334,7 +334,8 @@ typedef struct sbi_newton_desc {
   const int32_t* jt_unit;     /* [4 * 16 * n_jt_blocks] {dim | degree << 16, first step of the block,
                                  entries, slot or ~i (the unit is all of table dim i)} */
   const int32_t* jt_dim;      /* [4 * n_tab_dims] {dim, first row, largest degree | count << 16, first
-                                 singular coordinate (sing_x)} */
+                                 singular coordinate (sing_x)}; count 0 for the dims of jt_red, which
+                                 are marked while their units' sums are added */
   const int32_t* jt_red;      /* [3 * n_jt_red] {dim, first slot, slot count} */
 } sbi_newton_desc;
 

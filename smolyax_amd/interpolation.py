@@ -472,10 +472,11 @@ class SmolyakBarycentricInterpolator:
             raise RuntimeError("singular coordinates in a dim without factors")
         t["sing_off"], t["sing_x"] = _dev_tensor(sing_off, i32, dev), _dev_tensor(sing_x, f64, dev)
         if NL.n_jt_blocks:
+            # singular coordinates: only of the dims that one unit writes (degree 1: at most a few);
+            # dims of several units are marked while their sums are added
             nt = NL.n_tab_dims
             first, ns = sing_off[NL.tab_dim[:nt]], np.diff(sing_off)[NL.tab_dim[:nt]]
-            if int(ns.max()) > 0x7FFF:
-                raise RuntimeError("more singular coordinates in a dim than the plan's records hold")
+            ns = np.where(np.isin(NL.tab_dim[:nt], NL.jt_red[: 3 * NL.n_jt_red: 3]), 0, ns)
             jt_dim = np.stack([NL.tab_dim[:nt], NL.tab_row[:nt],
                                NL.tab_kmax[:nt].astype(np.int64) | ns.astype(np.int64) << 16,
                                np.where(ns > 0, first, 0)], axis=1)
