@@ -465,6 +465,19 @@ int sbi_contract_f64_ws(const double* A, int64_t lda, const double* B, int64_t l
                         const double* offset, double* Y, int64_t ldy, int64_t P, int64_t n,
                         int64_t K, void* workspace, int64_t ws_bytes, void* stream);
 
+/* FP64 evaluation of the Newton form for any number of outputs in one call: the basis matrix
+ * (sbi_newton_basis_rows, into the workspace), then y[P, d_out] = H S (sbi_contract_f64_ws): the same
+ * polynomial as interpolation.py:264-304.  S: surpluses [basis_n, lds] in basis-row order, rows as
+ * sbi_contract_f64_ws takes B.  workspace: 256-byte aligned, not shared with a concurrent call, at
+ * least *basis_bytes (the basis matrix); with all of sbi_newton_eval_f64_gemm_workspace's result (-1:
+ * invalid) a small batch is spread over more workgroups, with the same bits.  At most 65535 * 64
+ * points. */
+int64_t sbi_newton_eval_f64_gemm_workspace(const sbi_newton_plan* plan, int64_t P,
+                                           int64_t* basis_bytes);
+int sbi_newton_eval_f64_gemm(const sbi_newton_plan* plan, const double* x, int64_t P, int64_t ldx,
+                             const double* S, int64_t lds, double* y, int64_t ldy, void* workspace,
+                             int64_t ws_bytes, void* stream);
+
 /* Mixed contraction: Y = offset + A64^T B64 (K64 rows, FP64 MFMA) + A32^T B32 (K32 rows, FP32
  * MFMA, partial sums added into FP64 every 256 terms), with the same layouts as sbi_contract.
  * The few rows that carry most of the result (the constant and low-degree terms) go in the FP64

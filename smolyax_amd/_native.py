@@ -138,6 +138,9 @@ SIGNATURES = {
                                      c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp]),
     "sbi_contract_split": (c_i32, [c_vp, c_i64, c_vp, c_i64, c_i64, c_vp, c_i64, c_vp, c_i64, c_i64,
                                    c_vp, c_vp, c_i64, c_i64, c_i64, c_vp]),
+    "sbi_newton_eval_f64_gemm_workspace": (c_i64, [c_vp, c_i64, c_vp]),
+    "sbi_newton_eval_f64_gemm": (c_i32, [c_vp, c_vp, c_i64, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp,
+                                         c_i64, c_vp]),
     "sbi_contract": (c_i32, [c_vp, c_i64, c_vp, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_i64,
                              c_i32, c_vp]),
     "sbi_contract_f64_workspace": (c_i32, [c_i64, c_i64, c_i64, c_vp]),

@@ -1123,6 +1123,47 @@ extern "C" int sbi_newton_eval_mixed_gemm(const sbi_newton_plan* plan, const dou
                                   w + ht + h64, ws_bytes - ht - h64, stream);
 }
 
+static int64_t f64_basis_ld(int64_t P) { return P + (P & 1); }  // rows on 16 bytes
+
+extern "C" int64_t sbi_newton_eval_f64_gemm_workspace(const sbi_newton_plan* plan, int64_t P,
+                                                      int64_t* basis_bytes) {
+  const sbi_newton_desc* dp = nullptr;
+  if (sbi_newton_plan_desc(plan, &dp) != SBI_OK || P < 0 || dp->basis_n <= 0) {
+    sbi::set_error("sbi_newton_eval_f64_gemm_workspace: null plan, negative P or no basis rows");
+    return -1;
+  }
+  const int64_t basis = align256((int64_t)dp->basis_n * f64_basis_ld(P) * 8);
+  if (basis_bytes) *basis_bytes = basis;
+  int64_t part = 0;
+  if (sbi_contract_f64_workspace(P, dp->d_out, dp->basis_n, &part) != SBI_OK) return -1;
+  return basis + part;
+}
+
+extern "C" int sbi_newton_eval_f64_gemm(const sbi_newton_plan* plan, const double* x, int64_t P,
+                                        int64_t ldx, const double* S, int64_t lds, double* y,
+                                        int64_t ldy, void* workspace, int64_t ws_bytes,
+                                        void* stream) {
+  const sbi_newton_desc* dp = nullptr;
+  if (sbi_newton_plan_desc(plan, &dp) != SBI_OK || !x || !S || !y || P < 0 || ldx < dp->d_in ||
+      lds < dp->d_out || ldy < dp->d_out || dp->basis_n <= 0 || !workspace ||
+      ((uintptr_t)workspace & 255) || P > (int64_t)65535 * 64) {
+    sbi::set_error("sbi_newton_eval_f64_gemm: invalid argument (or the workspace is not 256-byte "
+                   "aligned)");
+    return SBI_ERR_INVALID;
+  }
+  if (P == 0) return SBI_OK;
+  const int64_t ldh = f64_basis_ld(P), basis = align256((int64_t)dp->basis_n * ldh * 8);
+  if (ws_bytes < basis) {
+    sbi::set_error("sbi_newton_eval_f64_gemm: workspace smaller than the basis matrix");
+    return SBI_ERR_INVALID;
+  }
+  double* HT = (double*)workspace;
+  const int rc = sbi_newton_basis_rows(plan, x, P, ldx, 0, dp->basis_n, HT, ldh, 0, stream);
+  if (rc != SBI_OK) return rc;
+  return sbi_contract_f64_ws(HT, ldh, S, lds, nullptr, y, ldy, P, dp->d_out, dp->basis_n,
+                             (char*)workspace + basis, ws_bytes - basis, stream);
+}
+
 static bool jac_global_table(const sbi_newton_desc& d);
 
 constexpr int kJacDirectMax = 8;  // outputs handled in one register pass

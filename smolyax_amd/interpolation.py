@@ -19,6 +19,7 @@ from .nodes import Generator, Leja1D
 
 PRECISIONS = ("fp64", "mixed", "newton-fp64", "bf16", "bary-fp32")
 GEMM_MIN_DOUT = 16  # from this d_out on, the d_out contraction is one dense GEMM
+CONTRACT_CHAIN = 256  # terms that the FP64 contraction sums in one workgroup in any case
 MAX_CALL_POINTS = 65535 * 64  # points per call of sbi_contract / _jacobian_f64 / sbi_newton_vjp
 # Newton form of a non-nested interpolant on a nested proxy grid (see _newton_proxy): its largest
 # relative distance from the FP64 barycentric path on sample points decides what it may serve.
@@ -411,8 +412,10 @@ class SmolyakBarycentricInterpolator:
             setattr(d, name, ten.data_ptr())
         d.n_split = packing.N_WAVES
         d.n_seg = int(L.seg_off[-1])
+        self._n_share = 0
         if sh is not None:
             d.n_share, d.share_rows = sh.n, sh.rows
+            self._n_share = sh.n
         if prog is not None:
             d.n_pseg = int(prog.seg_off[-1])
             d.ones_row = prog.ones_row
@@ -587,7 +590,7 @@ class SmolyakBarycentricInterpolator:
     # ------------------------------------------------------------------------------ evaluation
     def __call__(self, x) -> torch.Tensor:
         """interpolation.py:264-304: y[P, d_out] (float64 tensor) on the default precision path."""
-        return self.evaluate(x, precision=self._precision)
+        return self._evaluate(x, self._precision)
 
     def evaluate(self, x, precision: str = None) -> torch.Tensor:
         """Evaluate on a chosen path (see the constructor's `precision`)."""
@@ -633,7 +636,7 @@ class SmolyakBarycentricInterpolator:
                 or (precision != "fp64" and self._d_out > 1))
         if not gemm:
             y = torch.empty((P, self._d_out), dtype=torch.float64, device=self._device)
-            if precision == "fp64" and self._desc.n_share and not (ordered and self._desc.n_share > 1):
+            if precision == "fp64" and self._n_share and not (ordered and self._n_share > 1):
                 ws = N.fn["sbi_bary_eval_few_workspace"](self._plan, P)
                 W = torch.empty(ws, dtype=torch.uint8, device=self._device) if ws else None
                 N.check(N.fn["sbi_bary_eval_few_f64"](self._plan, x.data_ptr(), P, x.stride(0),
@@ -674,8 +677,9 @@ class SmolyakBarycentricInterpolator:
     def _rows_buffer(rows, cols, dtype, device):
         """An uninitialised (rows, cols) matrix; FP64 rows start on 16 bytes (an odd width gets one
         spare element), which the FP64 contraction's wide copies need."""
-        ld = cols + (cols & 1) if dtype == torch.float64 else cols
-        return torch.empty((rows, ld), dtype=dtype, device=device)[:, :cols]
+        if dtype != torch.float64 or cols % 2 == 0:
+            return torch.empty((rows, cols), dtype=dtype, device=device)
+        return torch.empty((rows, cols + 1), dtype=dtype, device=device)[:, :cols]
 
     def _contract(self, A, B, offset, y, ordered=False):
         """y[P, n] = offset + A^T B on the matrix cores (sbi_contract_f64_ws; sbi_contract for FP32
@@ -685,9 +689,11 @@ class SmolyakBarycentricInterpolator:
         off = None if offset is None else offset.data_ptr()
         (P, n), K = y.shape, A.shape[0]
         if A.dtype == torch.float64 and not ordered:
-            nb = N.c_i64()
-            N.check(N.fn["sbi_contract_f64_workspace"](P, n, K, ctypes.byref(nb)), "contract")
-            ws = nb.value
+            ws = 0
+            if K > CONTRACT_CHAIN:  # (shorter sums are never spread)
+                nb = N.c_i64()
+                N.check(N.fn["sbi_contract_f64_workspace"](P, n, K, ctypes.byref(nb)), "contract")
+                ws = nb.value
             W = torch.empty(ws, dtype=torch.uint8, device=y.device) if ws else None
             N.check(N.fn["sbi_contract_f64_ws"](A.data_ptr(), ld(A), B.data_ptr(), ld(B), off,
                                                 y.data_ptr(), ld(y), P, n, K,
@@ -784,6 +790,20 @@ class SmolyakBarycentricInterpolator:
         kind = {"newton-fp64": "f64", "mixed": "f32", "bf16": "bf16"}[precision]
         st = self._stream()
         y = torch.empty((P, self._d_out), dtype=torch.float64, device=self._device)
+        if kind == "f64" and not ordered:  # one call per chunk: basis matrix and contraction
+            S = self._surpluses("f64", gemm=True)
+            pc = self._point_chunk(Nn, 8, P)
+            for a in range(0, P, pc):
+                xc, yc = (x, y) if pc >= P else (x[a:a + pc], y[a:a + pc])
+                n = yc.shape[0]
+                nb = N.c_i64()
+                ws = N.fn["sbi_newton_eval_f64_gemm_workspace"](self._nplan, n, ctypes.byref(nb))
+                W = torch.empty(ws, dtype=torch.uint8, device=self._device)
+                N.check(N.fn["sbi_newton_eval_f64_gemm"](self._nplan, xc.data_ptr(), n,
+                                                         xc.stride(0), S.data_ptr(), self._ld(S),
+                                                         yc.data_ptr(), self._ld(yc), W.data_ptr(),
+                                                         ws, st), "newton-fp64")
+            return y
         if kind == "f64":
             S = self._surpluses("f64", gemm=True)
             pc = self._point_chunk(Nn, 8, P)
@@ -794,7 +814,7 @@ class SmolyakBarycentricInterpolator:
                 N.check(N.fn["sbi_newton_basis_rows"](self._nplan, xc.data_ptr(), b - a,
                                                       xc.stride(0), 0, Nn, HT.data_ptr(),
                                                       HT.stride(0), 0, st), "basis")
-                self._contract(HT, S, None, y[a:b], ordered)
+                self._contract(HT, S, None, y[a:b], ordered=True)
             return y
         if kind == "f32":  # one call per chunk: head rows, FP32 rows, contraction
             pc = self._point_chunk(self._ndesc.gemm_kq + 2 * self._ndesc.gemm_head, 4, P)
