@@ -893,8 +893,12 @@ class SmolyakBarycentricInterpolator:
             xc = x[p0:p1]
             # G^T[nu, p] = sum_m S[nu, m] v[p, m] on the matrix cores (A = S^T and B = v^T; FP64,
             # or FP32 operands with FP64 accumulation)
-            VT = self._rows_buffer(self._d_out, p1 - p0, dt, self._device)
-            VT.copy_(v[p0:p1].detach().t())
+            # (one point or one output: v^T is v's own memory; else one copy, odd rows padded)
+            VT = v[p0:p1].detach().t()
+            if (p1 - p0) % 2 and p1 - p0 > 1 and self._d_out > 1 and dt == torch.float64:
+                VT = self._rows_buffer(self._d_out, p1 - p0, dt, self._device).copy_(VT)
+            else:
+                VT = VT.to(dt).contiguous()
             GT = torch.empty((n_nodes, p1 - p0), dtype=torch.float64, device=self._device)
             self._contract(ST, VT, None, GT)
             nb = int(N.fn["sbi_newton_vjp_workspace"](self._nplan, p1 - p0))
