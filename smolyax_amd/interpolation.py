@@ -19,6 +19,15 @@ from .nodes import Generator, Leja1D
 
 PRECISIONS = ("fp64", "mixed", "newton-fp64", "bf16", "bary-fp32")
 GEMM_MIN_DOUT = 16  # from this d_out on, the d_out contraction is one dense GEMM
+# The smallest plans (entries x outputs, at least 2 of them) keep the walk over blocks in "fp64": one
+# launch, where the Newton form of 2 to 15 outputs takes two and that of one output a longer chain on
+# chip.  300 points, us a call in a row and alone: 10 indices x 2 inputs, 24 entries: 12 and 24 against
+# 19 and 27 (8 outputs), 12 and 22 against 12 and 24 (one); 220 entries x 2 outputs: 15 and 30 against
+# 19 and 34; 300 x 4: 19 and 33 on both.  With many outputs and points the walk falls behind beyond the
+# line: 16 384 points, 72 entries x 15: 38 against 30.  Blocks of a high degree are long serial runs: 40
+# entries of one dim 17 and 32 against 14 and 29.
+SMALL_PLAN = 500
+SMALL_PLAN_DEGREE = 16  # largest degree + 1
 CONTRACT_CHAIN = 256  # terms that the FP64 contraction sums in one workgroup in any case
 MAX_CALL_POINTS = 65535 * 64  # points per call of sbi_contract / _jacobian_f64 / sbi_newton_vjp
 # Newton form of a non-nested interpolant on a nested proxy grid (see _newton_proxy): its largest
@@ -107,6 +116,7 @@ class SmolyakBarycentricInterpolator:
         self._proxy_err = None      # non-nested: proxy Newton form vs the FP64 barycentric path
         self._newton_fp64_ok = False
         self._fp64_newton = False   # "fp64" is served by the Newton form (see evaluate)
+        self._small_plan = False    # ... except on plans where the walk over blocks is faster
         self._warned_mixed = False
         self._mixed_err = None      # mixed GEMM path vs the FP64 path on sample points (d_out > 1)
         self._maxdeg = None         # per dim: highest degree in Lambda (sample points)
@@ -154,6 +164,8 @@ class SmolyakBarycentricInterpolator:
             self._newton_off = str(e)
         self._fp64_newton = (self._is_nested and self._nplan is not None and self._finite_s
                              and self._newton_is_accurate(values))
+        self._small_plan = (self._d_out < GEMM_MIN_DOUT and L.dmax1 <= SMALL_PLAN_DEGREE
+                            and L.k_raw * max(2, self._d_out) <= SMALL_PLAN)
         if self._is_nested and not self._fp64_newton and 2 <= self._d_out <= packing.SHARE_MAX_OUT:
             self._upload(shares=True)
         self._values = None
@@ -617,7 +629,7 @@ class SmolyakBarycentricInterpolator:
         # below 1e-14 up to degree 300.  16 384 points x 1000 inputs: 54 us against 132 us;
         # 5000 points x 160 outputs: 0.45 ms against 3.7 ms.  (Values that are not finite spread to
         # other nodes' surpluses: such an interpolant keeps the reference's sums.)
-        if precision == "fp64" and self._fp64_newton:
+        if precision == "fp64" and self._fp64_newton and not self._small_plan:
             precision = "newton-fp64"
         if precision == "newton-fp64" and self._nplan is not None and not self._newton_fp64_ok:
             raise ValueError(f"precision 'newton-fp64': the proxy Newton form of this non-nested "
