@@ -902,23 +902,21 @@ class SmolyakBarycentricInterpolator:
         chunk = self._point_chunk(n_nodes * 8 + max(0, ws1) // 64 + 1, 1, P)
         for p0 in range(0, P, chunk):
             p1 = min(P, p0 + chunk)
-            xc = x[p0:p1]
+            xc, vc, gc = (x, v, gx) if chunk >= P else (x[p0:p1], v[p0:p1], gx[p0:p1])
             # G^T[nu, p] = sum_m S[nu, m] v[p, m] on the matrix cores (A = S^T and B = v^T; FP64,
             # or FP32 operands with FP64 accumulation)
             # (one point or one output: v^T is v's own memory; else one copy, odd rows padded)
-            VT = v[p0:p1].detach().t()
             if (p1 - p0) % 2 and p1 - p0 > 1 and self._d_out > 1 and dt == torch.float64:
-                VT = self._rows_buffer(self._d_out, p1 - p0, dt, self._device).copy_(VT)
+                VT = self._rows_buffer(self._d_out, p1 - p0, dt, self._device).copy_(vc.detach().t())
             else:
-                VT = VT.to(dt).contiguous()
+                VT = vc.t().to(dt).contiguous()
             GT = torch.empty((n_nodes, p1 - p0), dtype=torch.float64, device=self._device)
             self._contract(ST, VT, None, GT)
             nb = int(N.fn["sbi_newton_vjp_workspace"](self._nplan, p1 - p0))
             ws = torch.empty(max(1, (nb + 7) // 8), dtype=torch.float64, device=self._device)
             N.check(N.fn["sbi_newton_vjp"](self._nplan, xc.data_ptr(), p1 - p0, xc.stride(0),
-                                           GT.data_ptr(), GT.stride(0), 0,
-                                           gx[p0:p1].data_ptr(), ws.data_ptr(), nb,
-                                           self._stream()), "vjp")
+                                           GT.data_ptr(), GT.stride(0), 0, gc.data_ptr(),
+                                           ws.data_ptr(), nb, self._stream()), "vjp")
         return gx
 
     def differentiable(self, x: torch.Tensor, precision: str = None) -> torch.Tensor:
