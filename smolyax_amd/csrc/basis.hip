@@ -1174,8 +1174,16 @@ constexpr int kJacDirectMax = 8;  // outputs handled in one register pass
 // card's 288 GB.  5..8 outputs take 240 registers, so that small tables gain nothing from LDS:
 // 4096 points x 200 inputs x 8 outputs (249 rows) 179 us against 153 us by the other pass, 1000
 // inputs (1058 rows) 409 us against 573 us; 4 outputs: 98 against 104 us, 198 against 284 us.
+// Small plans in which no dim is split over the other pass's units of 128 entries need no launch for the
+// sums there, but one here, where a unit is one degree of a dim: 5 inputs x 60 indices (110 entries),
+// 64 points, in a row and alone: 17 and 29 us by the other pass, 20 and 33 here; 360 entries and one
+// output 19.5 and 38 against 22 and 40, four outputs 33 and 52 against 25 and 44.
+constexpr int64_t kJacSmall = 800;  // entries x (outputs + 1)
 static int jac_tile_waves(const sbi_newton_desc& d, int64_t n) {
-  if (!d.jt_unit || d.n_jt_blocks <= 0 || d.basis_n < 16 || n > kJacDirectMax) return 0;
+  if (!d.jt_unit || !d.jt_ent || !d.jt_dim || (d.n_jt_red > 0 && !d.jt_red) || d.n_jt_blocks <= 0 ||
+      d.basis_n < 16 || n > kJacDirectMax)
+    return 0;
+  if (d.n_jac_red == 0 && (int64_t)d.n_vjp_ent * (n + 1) <= kJacSmall && !jac_global_table(d)) return 0;
   for (int waves : {4, 8, 16})
     if (jac_tile_lds(d) <= (size_t)kMaxLds * waves / 16) return n > 4 && waves < 16 ? 0 : waves;
   return 0;
