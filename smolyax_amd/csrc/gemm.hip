@@ -1489,12 +1489,23 @@ __global__ __launch_bounds__(64 * kWaves, 2) void jac_contract_kernel(
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies past the last chunk
   __syncthreads();
 
-  // FP64 16x16x4 result: row (point) g + 4r in register r, column (output) = lane % 16
+  // FP64 16x16x4 result: row (point) g + 4r in register r, column (output) = lane % 16.  Register r of
+  // all dims goes through LDS; lanes l = 8 i + (lane >> 3) of it are written in step i, so a step has
+  // one point and 8 outputs, the points follow each other, and the address is a scalar that advances
+  // plus the lane's own fixed offset (with an address per element a call on one job of a few rows took
+  // 1.5 us more, and 999 points x 256 outputs x 200 dims 351 instead of 346 us).
   double* __restrict__ tr = (double*)smem + wave * kJacDims * kJacT;
-  const int jj = lane & 7;
+  const int jj = lane & 7, sub = lane >> 3;
+  const double* __restrict__ from = tr + jj * kJacT + sub;
+  const int64_t row0 = m0 + mw, col0 = n0 + nw;
+  const int rows = (int)min(P - row0, (int64_t)32);
+  const int64_t ldo = slot >= 0 ? kJacDims : nz;
+  const uint32_t own = (uint32_t)sub * (uint32_t)ldo + jj;
+  const bool in0 = col0 + sub < n, in1 = col0 + 8 + sub < n;
   for (;; z0 += kJacDims) {  // (groups without rows follow the job of the group before them)
-    double* __restrict__ out = slot >= 0 ? part + (int64_t)slot * P * n * kJacDims + jj : J + z0 + jj;
-    const int64_t ldo = slot >= 0 ? kJacDims : nz;
+    typedef __attribute__((address_space(1))) double gdouble;
+    gdouble* out = (gdouble*)(slot >= 0 ? part + (int64_t)slot * P * n * kJacDims : J + z0) +
+                   (row0 * n + col0) * ldo;
     const bool mine = slot >= 0 || z0 + jj < nz;
 #pragma unroll
     for (int fm = 0; fm < 2; ++fm)
@@ -1502,12 +1513,17 @@ __global__ __launch_bounds__(64 * kWaves, 2) void jac_contract_kernel(
       for (int r = 0; r < 4; ++r) {
 #pragma unroll
         for (int u = 0; u < kJacDims; ++u) tr[u * kJacT + lane] = acc[u][fm][r];
+        double v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {  // the elements of lanes 8 i .. 8 i + 7
-          const int l = 8 * i + (lane >> 3);
-          const int64_t row = m0 + mw + fm * 16 + (l >> 4) + 4 * r, col = n0 + nw + (l & 15);
-          const double v = tr[jj * kJacT + l];
-          if (row < P && col < n && mine) out[(row * n + col) * ldo] = v;
+        for (int i = 0; i < 8; ++i) v[i] = from[8 * i];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          if (fm * 16 + 4 * r + h < rows) {
+            if (mine && in0) out[own] = v[2 * h];
+            if (mine && in1) (out + 8 * ldo)[own] = v[2 * h + 1];
+          }
+          out += n * ldo;
+          asm volatile("" : "+s"(out));  // (or the 32 addresses are computed and kept ahead of the loop)
         }
       }
     if (slot >= 0 || z0 + kJacDims >= nz ||
