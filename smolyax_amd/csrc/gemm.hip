@@ -275,7 +275,7 @@ __global__ __launch_bounds__(64 * kWaves) void contract_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         // result layout: row 4g + r in register r of lane group g, column lane % 16
-        const int64_t row = m_base + fm * 16 + 4 * g + r;
+        const int64_t row = m_base + fm * 16 + (4 * g + r);
         const double v = acc64(fm, fn, r);
         if (row < P) Y[row * ldy + col] = off + v;
       }
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
   for (int fn = 0; fn < FN; ++fn) jcol[fn] = min(n_base + fn * 16 + li, n - 1);
   // element (fm, fn, r) of this lane: row and column of Y
   auto out_at = [&](int fm, int fn, int r, int64_t& row, int64_t& col) {
-    row = m_base + fm * 16 + 4 * g + r;
+    row = m_base + fm * 16 + (4 * g + r);
     col = n_base + fn * 16 + li;
   };
 
@@ -463,7 +463,8 @@ __global__ __launch_bounds__(64 * kWaves) void contract_split_kernel(
 
 // Y[p, j] = offset[j] + (((head + part_0) + part_1) + ...) (+ 0.0 when K is a multiple of
 // kFlushK: contract_kernel's final flush then adds an empty partial tile), head = 0 without one.
-template <typename E>
+// kGrouped (FP64 chains): the sums of `per` chains first, then theirs.
+template <typename E, bool kGrouped>
 __global__ __launch_bounds__(256) void contract_reduce_kernel(const E* __restrict__ part,
                                                               int64_t nch, int64_t per,
                                                               const double* __restrict__ head,
@@ -475,10 +476,16 @@ __global__ __launch_bounds__(256) void contract_reduce_kernel(const E* __restric
        i += (int64_t)gridDim.x * 256) {
     const int64_t row = i / n, col = i - row * n;
     double v = head ? head[i] : 0.0;
-    if (per == 1) {
-#pragma unroll 4
-      for (int64_t c = 0; c < nch; ++c) v += (double)part[c * Pn + i];
-    } else {  // FP64 chains: slice sums of `per` chains first
+    if constexpr (!kGrouped) {
+      for (int64_t c = 0; c < nch; c += 4) {  // four loads in flight, also where fewer are left
+        E q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = part[min(c + u, nch - 1) * Pn + i];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (c + u < nch) v += (double)q[u];
+      }
+    } else {
       for (int64_t c = 0; c < nch; c += per) {
         double s = 0.0;
 #pragma unroll 8
@@ -552,7 +559,7 @@ int contract_split_launch(const SplitPlan& sp, const float* A, int64_t lda, cons
   const int64_t Pn = P * n;
   int64_t rg = (Pn + 255) / 256;
   if (rg > 4096) rg = 4096;
-  hipLaunchKernelGGL((contract_reduce_kernel<float>), dim3((unsigned)rg), dim3(256), 0, st, part,
+  hipLaunchKernelGGL((contract_reduce_kernel<float, false>), dim3((unsigned)rg), dim3(256), 0, st, part,
                      sp.nch, int64_t(1), head, offset, Y, ldy, P, n, K);
   SBI_HIP_CHECK(hipGetLastError());
   return SBI_OK;
@@ -913,8 +920,10 @@ int contract_f64(const double* A, int64_t lda, const double* B, int64_t ldb, con
   SBI_HIP_CHECK(hipGetLastError());
   if (pl.nz > 1) {
     const int64_t rg = std::min<int64_t>((P * n + 255) / 256, 4096);
-    hipLaunchKernelGGL((contract_reduce_kernel<double>), dim3((unsigned)rg), dim3(256), 0, st,
-                       (const double*)ws, pl.units, pl.per, nullptr, offset, Y, ldy, P, n, K);
+    const auto reduce = pl.per > 1 ? contract_reduce_kernel<double, true>
+                                   : contract_reduce_kernel<double, false>;
+    hipLaunchKernelGGL(reduce, dim3((unsigned)rg), dim3(256), 0, st, (const double*)ws, pl.units,
+                       pl.per, nullptr, offset, Y, ldy, P, n, K);
     SBI_HIP_CHECK(hipGetLastError());
   }
   return SBI_OK;
@@ -1279,7 +1288,7 @@ __device__ __forceinline__ void contract_bf16_body(
     for (int fm = 0; fm < kBfWM; ++fm)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t row = m_base + fm * 16 + 4 * g + r;
+        const int64_t row = m_base + fm * 16 + (4 * g + r);
         if (row < P) Y[row * ldy + col] = off + acc64[fm][fn][r];
       }
   }
