@@ -608,10 +608,12 @@ class SmolyakBarycentricInterpolator:
         """Evaluate on a chosen path (see the constructor's `precision`)."""
         return self._evaluate(x, precision or self._precision)
 
-    def _evaluate(self, x, precision, ordered=False):
+    def _evaluate(self, x, precision, ordered=False, scratch=True):
         """`evaluate`; ordered: FP64 sums of several outputs block by block (few outputs, unless one
-        share holds all blocks) and in the order of k, which fixes the bits of what set_f derives from them (a proxy's surpluses, which the FP32
-        rounding of "mixed" makes visible) whatever the fastest split of the sums is."""
+        share holds all blocks) and in the order of k, which fixes the bits of what set_f derives from
+        them (a proxy's surpluses, which the FP32 rounding of "mixed" makes visible) whatever the
+        fastest split of the sums is.  scratch: small batches may take the workspaces that spread their
+        FP64 sums over more workgroups (scratch_bytes; the same bits without)."""
         if precision not in PRECISIONS:
             raise ValueError(f"precision must be one of {PRECISIONS}")
         if precision == "mixed" and self._nplan is None:
@@ -649,7 +651,8 @@ class SmolyakBarycentricInterpolator:
         if not gemm:
             y = torch.empty((P, self._d_out), dtype=torch.float64, device=self._device)
             if precision == "fp64" and self._n_share and not (ordered and self._n_share > 1):
-                ws = N.fn["sbi_bary_eval_few_workspace"](self._plan, P)
+                ws = N.fn["sbi_bary_eval_few_workspace"](self._plan, P) if scratch else 0
+                ws = self._within_limit(ws)
                 W = torch.empty(ws, dtype=torch.uint8, device=self._device) if ws else None
                 N.check(N.fn["sbi_bary_eval_few_f64"](self._plan, x.data_ptr(), P, x.stride(0),
                                                       y.data_ptr(), W.data_ptr() if ws else None,
@@ -658,19 +661,44 @@ class SmolyakBarycentricInterpolator:
                 rc = N.fn["sbi_bary_eval_f64"](self._plan, x.data_ptr(), P, x.stride(0),
                                                y.data_ptr(), self._stream())
                 if rc == N.SBI_ERR_CAPACITY:  # prefix table too large for LDS: GEMM form
-                    return self._eval_bary_gemm(x, ordered=ordered)
+                    return self._eval_bary_gemm(x, ordered=ordered, scratch=scratch)
                 N.check(rc, "eval")
             else:
                 fn = "sbi_newton_eval_mixed" if precision == "mixed" else "sbi_newton_eval_f64"
                 rc = N.fn[fn](self._nplan, x.data_ptr(), P, x.stride(0), y.data_ptr(),
                               self._stream())
                 if rc == N.SBI_ERR_CAPACITY:  # internal-node table beyond LDS: GEMM form
-                    return self._eval_newton_gemm(x, precision, ordered)
+                    return self._eval_newton_gemm(x, precision, ordered, scratch)
                 N.check(rc, precision)
             return y
         if precision == "fp64":
-            return self._eval_bary_gemm(x, ordered=ordered)
-        return self._eval_newton_gemm(x, precision, ordered)
+            return self._eval_bary_gemm(x, ordered=ordered, scratch=scratch)
+        return self._eval_newton_gemm(x, precision, ordered, scratch)
+
+    def _within_limit(self, ws, held=0):
+        """ws, the bytes of a workspace that a call can do without, or 0 where memory_limit has no
+        room for it beside `held` bytes."""
+        return ws if held + ws <= self._memory_limit * 1024**3 else 0
+
+    def scratch_bytes(self, precision: str, n_points: int) -> int:
+        """Bytes of workspace that an FP64 evaluation of n_points takes beside its basis matrix, input
+        and output, to spread a small batch over more workgroups: at most 256 MB, nothing beyond
+        memory_limit; 0 on the other paths."""
+        P = int(n_points)
+        if precision == "fp64" and self._fp64_newton and not self._small_plan:
+            precision = "newton-fp64"
+        if P <= 0 or precision not in ("fp64", "newton-fp64"):
+            return 0
+        if precision == "fp64" and self._d_out < GEMM_MIN_DOUT:
+            ws = N.fn["sbi_bary_eval_few_workspace"](self._plan, P) if self._n_share else 0
+            return self._within_limit(ws)
+        if self._d_out == 1 or (precision == "newton-fp64" and self._nplan is None):
+            return 0
+        K = self._layout.k_raw if precision == "fp64" else self._nlayout.basis_n
+        P = min(P, self._point_chunk(K, 8, P))
+        nb = N.c_i64()
+        N.check(N.fn["sbi_contract_f64_workspace"](P, self._d_out, K, ctypes.byref(nb)), "contract")
+        return self._within_limit(nb.value, K * (P + P % 2) * 8)
 
     def _point_chunk(self, rows, itemsize, P):
         """Points per chunk so that the basis matrix stays within memory_limit GiB, and within
@@ -693,7 +721,7 @@ class SmolyakBarycentricInterpolator:
             return torch.empty((rows, cols), dtype=dtype, device=device)
         return torch.empty((rows, cols + 1), dtype=dtype, device=device)[:, :cols]
 
-    def _contract(self, A, B, offset, y, ordered=False):
+    def _contract(self, A, B, offset, y, ordered=False, scratch=True):
         """y[P, n] = offset + A^T B on the matrix cores (sbi_contract_f64_ws; sbi_contract for FP32
         operands with FP64 accumulation and, ordered, for FP64 sums in the order of k; rows
         independent of the batch)."""
@@ -702,10 +730,10 @@ class SmolyakBarycentricInterpolator:
         (P, n), K = y.shape, A.shape[0]
         if A.dtype == torch.float64 and not ordered:
             ws = 0
-            if K > CONTRACT_CHAIN:  # (shorter sums are never spread)
+            if scratch and K > CONTRACT_CHAIN:  # (shorter sums are never spread)
                 nb = N.c_i64()
                 N.check(N.fn["sbi_contract_f64_workspace"](P, n, K, ctypes.byref(nb)), "contract")
-                ws = nb.value
+                ws = self._within_limit(nb.value, max(A.numel(), y.numel()) * 8)
             W = torch.empty(ws, dtype=torch.uint8, device=y.device) if ws else None
             N.check(N.fn["sbi_contract_f64_ws"](A.data_ptr(), ld(A), B.data_ptr(), ld(B), off,
                                                 y.data_ptr(), ld(y), P, n, K,
@@ -716,7 +744,7 @@ class SmolyakBarycentricInterpolator:
                                      ld(y), P, n, K, int(A.dtype == torch.float32), self._stream()),
                 "contract")
 
-    def _eval_bary_gemm(self, x, fp32=False, out=None, ordered=False):
+    def _eval_bary_gemm(self, x, fp32=False, out=None, ordered=False, scratch=True):
         """y = offset + W F: barycentric entry weights (HIP kernel), then the contraction with the
         zeta-scaled values on the matrix cores (FP64, or FP32 operands with FP64 accumulation)."""
         P = x.shape[0]
@@ -738,7 +766,7 @@ class SmolyakBarycentricInterpolator:
             WT = self._rows_buffer(K, b - a, dt, self._device)
             N.check(N.fn[fn](self._plan, xc.data_ptr(), b - a, xc.stride(0), WT.data_ptr(),
                              WT.stride(0), self._stream()), "bary_basis")
-            self._contract(WT, F, self._dev["offset"], y[a:b], ordered)
+            self._contract(WT, F, self._dev["offset"], y[a:b], ordered, scratch)
         return y
 
     def _surpluses(self, kind, gemm=False):
@@ -791,7 +819,7 @@ class SmolyakBarycentricInterpolator:
             self._Sg["bf16k8"] = S
         return S
 
-    def _eval_newton_gemm(self, x, precision, ordered=False):
+    def _eval_newton_gemm(self, x, precision, ordered=False, scratch=True):
         """y = H S: Newton basis matrix (HIP kernel), then the contraction with the surpluses on
         the matrix cores: sbi_contract for FP64; for "mixed" (FP32) and "bf16" the heaviest rows
         in FP64 (sbi_newton_rows_f64, FP64 MFMA) and the rest in FP32 or BF16, k-interleaved
@@ -810,6 +838,8 @@ class SmolyakBarycentricInterpolator:
                 n = yc.shape[0]
                 nb = N.c_i64()
                 ws = N.fn["sbi_newton_eval_f64_gemm_workspace"](self._nplan, n, ctypes.byref(nb))
+                if ws > nb.value and not (scratch and self._within_limit(ws)):
+                    ws = nb.value  # the basis matrix alone
                 W = torch.empty(ws, dtype=torch.uint8, device=self._device)
                 N.check(N.fn["sbi_newton_eval_f64_gemm"](self._nplan, xc.data_ptr(), n,
                                                          xc.stride(0), S.data_ptr(), self._ld(S),

@@ -163,7 +163,8 @@ class Server:
         torch.cuda.synchronize()
 
     def footprint(self, name, n_points):
-        """Device bytes a batch needs while in flight: basis matrix + output + input copy."""
+        """Device bytes a batch needs while in flight: basis matrix + output + input copy.  (FP64
+        evaluations of small batches take more where the budget has room: ip.scratch_bytes.)"""
         ip = self.ips[name]
         rows = ip.layout.k_raw if ip._nlayout is None or self.precision == "bary-fp32" else \
             ip._nlayout.basis_n
@@ -248,9 +249,13 @@ class Server:
                     self.n_pending -= 1
             if not pieces:
                 break  # wait for memory to free up
-            need = bpp * pts
-            self.reserved += need
             ip = self.ips[head.name]
+            need = bpp * pts
+            ws = ip.scratch_bytes(self.precision, pts)
+            scratch = self.reserved + need + ws <= self.budget
+            if scratch:
+                need += ws
+            self.reserved += need
             use_graph = self.graphs and (self.graph_mode is True or
                                          self.n_pending >= len(self.slots))
             for r, _, _ in pieces:  # the points are read on this stream once their producer is done
@@ -273,7 +278,7 @@ class Server:
                     xs = x_st
                 else:
                     xs = torch.cat(xin) if len(xin) > 1 else xin[0]
-                    y = ip.evaluate(xs, precision=self.precision)
+                    y = ip._evaluate(xs, self.precision, scratch=scratch)
                 a = 0
                 for r, a0, n in pieces:
                     if a0 == 0 and n == r.x.shape[0]:
