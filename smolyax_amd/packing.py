@@ -38,14 +38,15 @@ PROG_GROUP = 4           # segments per group of the eval kernel (kXGroup in bar
 PROG_MAX_GEN = 255       # per-block (generic) blocks per program segment
 PROG_MAX_COUNT = 65535   # records of one type per program segment
 PROG_MAX_ROWS = 320      # prefix table rows + 2 rows of ones, 64 points x 8 B each, in 160 KiB
-# Shares of the kernel for 2 to 16 outputs (few.hip): entries per share (about 10 us of a CU's matrix
+# Shares of the kernel for few outputs (few.hip; it takes up to 16, evaluate() gives it 2 to 15: from 16
+# on the outputs are one dense contraction): entries per share (about 10 us of a CU's matrix
 # work; 64 shares of 96 000 entries), basis rows per share (64 points x 8 B each in 160 KiB, with the
 # row of ones), factors per entry, header size in int32
 SHARE_ENTRIES = 1536
 SHARE_ROWS = 318
 SHARE_MAX_K = 8
 SHARE_HDR = 16
-SHARE_MAX_OUT = 16
+SHARE_MAX_OUT = 15
 PROG_SGPR = 48           # SGPRs per record chunk (kProgSgpr in bary.hip)
 # Wave split of the program: per-wave cost in cycles as measured on MI355X at d_in = 1000 (one
 # scalar memory round trip per record chunk): a full chunk, a partial chunk, a segment start
