@@ -33,6 +33,17 @@ def pair(d, m, d_out, kind="leja", kscale=1.0, f=None):
     return ref, SmolyakBarycentricInterpolator(d_out=d_out, node_gen=sng, k=k, t=t, f=f), ong
 
 
+def walk(ip, plan, x):
+    """sbi_bary_eval_f64."""
+    from smolyax_amd import _native as N
+
+    xt = torch.as_tensor(x, device="cuda")
+    y = torch.full((len(x), ip.d_out), float("nan"), dtype=torch.float64, device="cuda")
+    N.check(N.fn["sbi_bary_eval_f64"](plan, xt.data_ptr(), len(x), xt.stride(0), y.data_ptr(),
+                                      ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "eval")
+    return y.cpu().numpy()
+
+
 def few(ip, x, ws=True):
     """sbi_bary_eval_few_f64."""
     from smolyax_amd import _native as N
@@ -62,6 +73,41 @@ def points(d, n, seed, ong):
     return x
 
 
+@pytest.mark.parametrize("d,m,kscale", [(8, 3000, 0.3), (2, 40, 1.0), (12, 600, 0.2), (6, 200, 1.0)])
+def test_record_program_on_nested_layouts(gpu, d, m, kscale):
+    from smolyax_amd import _native as N
+
+    ref, ip, ong = pair(d, m, 1, kscale=kscale)
+    assert ip._prog is not None and ip._desc.n_pseg > 0
+    x = points(d, 131, m, ong)
+    print(f"d={d} m={m}: {ip._prog.n_records} records", flush=True)
+    y = walk(ip, ip._plan, x)
+    near_exact(y, ref, x)
+    q = N.BaryDesc()  # the per-block kernel: the same tables without the program
+    ctypes.pointer(q)[0] = ip._desc
+    q.pseg = None
+    plan = ctypes.c_void_p()
+    N.check(N.fn["sbi_bary_plan_create"](ctypes.byref(q), ctypes.byref(plan)), "plan")
+    try:
+        near_exact(walk(ip, plan, x), ref, x)
+    finally:
+        N.fn["sbi_plan_destroy"](plan)
+    assert np.array_equal(walk(ip, ip._plan, x[70:71])[0], y[70])
+
+
+@pytest.mark.parametrize("d,m,d_out", [(4, 60, 5), (8, 500, 16), (6, 300, 33), (20, 900, 40)])
+def test_barycentric_gemm_on_nested_layouts(gpu, d, m, d_out):
+    ref, ip, ong = pair(d, m, d_out)
+    x = points(d, 150, m, ong)
+    xt = torch.as_tensor(x, device="cuda")
+    y = ip._eval_bary_gemm(xt)
+    near_exact(y[:40].cpu().numpy(), ref, x[:40])
+    ip._memory_limit = 64 * 8 * ip.layout.k_raw / 1024**3  # chunks of 64 points
+    assert ip._point_chunk(ip.layout.k_raw, 8, 150) == 64
+    assert torch.equal(ip._eval_bary_gemm(xt), y)
+    assert torch.equal(ip._eval_bary_gemm(xt[149:150])[0], y[149])
+
+
 @pytest.mark.parametrize("d,m,P", [(5, 300, 65), (40, 2000, 130)])
 def test_share_kernel_takes_16_outputs(gpu, monkeypatch, d, m, P):
     """evaluate() sends 16 outputs to the dense contraction, so set_f builds no shares for them; the
@@ -77,3 +123,22 @@ def test_share_kernel_takes_16_outputs(gpu, monkeypatch, d, m, P):
     near_exact(y[:32], ref, x[:32])
     assert np.array_equal(few(ip, x, ws=False), y)
     assert np.array_equal(few(ip, x[P - 1:])[0], y[P - 1])
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_values_that_are_not_finite_in_one_of_three_outputs(gpu, value):
+    """A nested plan with such a value keeps the technique, and gets its shares for it: output 1 is
+    what the walk over blocks gives, the others are finite and near it (1e-12 of max |y|: a sum of at
+    most 1000 entries, each rounded a few times)."""
+    d = 4
+    f = lambda x: np.array([np.sum(x), value if np.asarray(x)[1] == 1.0 else 1.0 + x[0], np.cos(x[2])])
+    _, ip, ong = pair(d, 60, 3, f=f)
+    assert not ip._fp64_newton and ip._desc.n_share > 0
+    x = points(d, 70, 3, ong)
+    y = ip.evaluate(x, "fp64").cpu().numpy()
+    yw = walk(ip, ip._plan, x)
+    assert np.array_equal(y, few(ip, x), equal_nan=True)
+    assert np.array_equal(np.isnan(y), np.isnan(yw)) and np.array_equal(np.isinf(y), np.isinf(yw))
+    assert np.isfinite(y[:, [0, 2]]).all()
+    ok = np.isfinite(yw)
+    assert np.max(np.abs(y[ok] - yw[ok])) <= 1e-12 * np.max(np.abs(yw[ok]))
