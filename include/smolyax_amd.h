@@ -317,8 +317,8 @@ typedef struct sbi_newton_desc {
   const int32_t* jac_row_off; /* [d_in + 1] first row of each input dim */
   const int32_t* jac_row_end; /* [d_in] one past its last row that is not padding */
   const int32_t* jac_job;     /* [4 * n_jac_jobs] {first row, end row, first dim, partial slot}: the
-                                 rows of whole groups of 8 dims (slot -1), or a part of one group's
-                                 rows (slot 0 .. n_jac_slots - 1) */
+                                 rows of a whole group of 8 dims (slot -1; none if the group has
+                                 none), or a part of its rows (slot 0 .. n_jac_slots - 1) */
   const int32_t* jac_group_red; /* [3 * n_jac_group_red] {first dim, first slot, slots} of the
                                  groups in several parts */
   /* register pass of the Jacobian (d_out <= 8) and the adjoint with the factor table in LDS

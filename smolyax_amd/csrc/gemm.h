@@ -10,9 +10,9 @@ namespace sbi {
 // Row and job tables of the Jacobian contraction (device arrays).  Rows of dim z: off[z] .. end[z] - 1;
 // off[z + 1] is end[z] rounded up to a multiple of four (the records in between are valid and
 // unused).  Jobs cover the dims in groups of kJacGroup: either all rows of the group that starts at
-// dim job[2] (rows job[0] .. job[1] - 1, slot job[3] = -1) and the groups without rows after it, or a
-// part of a group's rows with its own slot of partial sums; groups of several parts are listed in
-// `red`.  Parts start at multiples of four rows after the group's first.
+// dim job[2] (rows job[0] .. job[1] - 1, none for a group without rows, whose J is zero; slot job[3] =
+// -1), or a part of a group's rows with its own slot of partial sums; groups of several parts are listed
+// in `red`.  Parts start at multiples of four rows after the group's first.
 constexpr int kJacGroup = 8;
 struct JacRows {
   const int32_t* row;  // [2 * off[nz]] {row of A, row of S}

@@ -1433,7 +1433,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void jac_contract_kernel(
   };
 
   v4d acc[kJacDims][2];
-  int z0 = job[2];
+  const int z0 = job[2];
   if (r0 < r1) {
     copy_rec(0);
     copy_rec(1);
@@ -1511,36 +1511,29 @@ __global__ __launch_bounds__(64 * kWaves, 2) void jac_contract_kernel(
   const int64_t ldo = slot >= 0 ? kJacDims : nz;
   const uint32_t own = (uint32_t)sub * (uint32_t)ldo + jj;
   const bool in0 = col0 + sub < n, in1 = col0 + 8 + sub < n;
-  for (;; z0 += kJacDims) {  // (groups without rows follow the job of the group before them)
-    typedef __attribute__((address_space(1))) double gdouble;
-    gdouble* out = (gdouble*)(slot >= 0 ? part + (int64_t)slot * P * n * kJacDims : J + z0) +
-                   (row0 * n + col0) * ldo;
-    const bool mine = slot >= 0 || z0 + jj < nz;
+  typedef __attribute__((address_space(1))) double gdouble;
+  gdouble* out = (gdouble*)(slot >= 0 ? part + (int64_t)slot * P * n * kJacDims : J + z0) +
+                 (row0 * n + col0) * ldo;
+  const bool mine = slot >= 0 || z0 + jj < nz;
 #pragma unroll
-    for (int fm = 0; fm < 2; ++fm)
+  for (int fm = 0; fm < 2; ++fm)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < 4; ++r) {
 #pragma unroll
-        for (int u = 0; u < kJacDims; ++u) tr[u * kJacT + lane] = acc[u][fm][r];
-        double v[8];
+      for (int u = 0; u < kJacDims; ++u) tr[u * kJacT + lane] = acc[u][fm][r];
+      double v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = from[8 * i];
+      for (int i = 0; i < 8; ++i) v[i] = from[8 * i];
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          if (fm * 16 + 4 * r + h < rows) {
-            if (mine && in0) out[own] = v[2 * h];
-            if (mine && in1) (out + 8 * ldo)[own] = v[2 * h + 1];
-          }
-          out += n * ldo;
-          asm volatile("" : "+s"(out));  // (or the 32 addresses are computed and kept ahead of the loop)
+      for (int h = 0; h < 4; ++h) {
+        if (fm * 16 + 4 * r + h < rows) {
+          if (mine && in0) out[own] = v[2 * h];
+          if (mine && in1) (out + 8 * ldo)[own] = v[2 * h + 1];
         }
+        out += n * ldo;
+        asm volatile("" : "+s"(out));  // (or the 32 addresses are computed and kept first)
       }
-    if (slot >= 0 || z0 + kJacDims >= nz ||
-        t.off[min(z0 + 2 * kJacDims, nz)] > t.off[z0 + kJacDims])
-      return;
-#pragma unroll
-    for (int u = 0; u < kJacDims; ++u) acc[u][0] = acc[u][1] = v4d{0, 0, 0, 0};
-  }
+    }
 }
 
 // J of the dim groups that several jobs share: the sum of their parts in order (blockIdx.y: the

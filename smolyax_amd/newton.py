@@ -679,8 +679,8 @@ def build_jacobian_units(L: NewtonLayout, tab_dims, row0, per_row) -> None:
 def build_jacobian_rows(L: NewtonLayout, node, d_out: int) -> None:
     """Rows and jobs of the Jacobian's contraction (d_out > 8): the adjoint entries dim by dim, each
     dim padded to a multiple of four rows by repeats of its last entry.  Jobs by groups of 8 dims:
-    a group of more than 8 d_out rows (at least 256, whole chunks of 16) is cut into parts of that
-    many, whose sums are added afterwards; groups without rows go with the job before them.  (At
+    a group of more than 8 d_out rows (at least 256, a multiple of 16) is cut into parts of that
+    many, whose sums are added afterwards; a group without rows is a job of its own.  (At
     256 outputs a part is 20 us of one SIMD's matrix work.)  The cuts depend on the plan alone: a
     point's sums are the same in every batch."""
     d_in = len(L.vjp_dim_off) - 1
@@ -703,8 +703,6 @@ def build_jacobian_rows(L: NewtonLayout, node, d_out: int) -> None:
             for c0, c1 in zip(cuts[:-1], cuts[1:]):
                 jobs.append((c0, c1, z0, slots))
                 slots += 1
-        elif jobs and jobs[-1][3] < 0 and a == b:
-            continue
         else:
             jobs.append((a, b, z0, -1))
     L.n_jac_jobs, L.n_jac_slots, L.n_jac_group_red = len(jobs), slots, len(red)

@@ -40,3 +40,28 @@ def test_any_number_of_singular_coordinates(monkeypatch):
             assert deg >> 16 == 0
         else:
             assert (deg >> 16, first) == (count[j], off[j])
+
+
+def test_every_group_of_dims_has_its_own_jobs():
+    """Jobs of the Jacobian contraction (d_out > 8): every group of 8 dims, with rows or without, is one
+    job or several parts; no job writes the groups of others one after another."""
+    from smolyax_amd import newton as NW
+    from smolyax_amd import nodes as SN
+
+    d, d_out = 203, 9
+    k = np.log((2 + np.arange(d)) / np.log(2))
+    t = OI.find_approximate_threshold(k, 300, True)
+    nf = NW.NewtonForm(k, t, SN.Leja(dim=d), d_out)
+    nf.set_values(np.ones((len(nf.nus), d_out)))
+    L = NW.build_newton_layout(nf)
+    off = L.jac_row_off
+    groups = {}
+    for a, b, z0, slot in L.jac_job.reshape(-1, 4).tolist():
+        assert z0 % 8 == 0 and off[z0] <= a <= b <= off[min(z0 + 8, d)]
+        groups.setdefault(z0, []).append((a, b, slot))
+    assert sorted(groups) == list(range(0, d, 8))
+    assert any(off[z] == off[min(z + 8, d)] for z in groups)  # (groups without rows are there)
+    for z0, jobs in groups.items():
+        assert jobs[0][0] == off[z0] and jobs[-1][1] == off[min(z0 + 8, d)]
+        assert all(p[1] == q[0] for p, q in zip(jobs[:-1], jobs[1:]))
+        assert (len(jobs) == 1) == (jobs[0][2] < 0)
