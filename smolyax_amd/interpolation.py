@@ -19,15 +19,6 @@ from .nodes import Generator, Leja1D
 
 PRECISIONS = ("fp64", "mixed", "newton-fp64", "bf16", "bary-fp32")
 GEMM_MIN_DOUT = 16  # from this d_out on, the d_out contraction is one dense GEMM
-# The smallest plans (entries x outputs, at least 2 of them) keep the walk over blocks in "fp64": one
-# launch, where the Newton form of 2 to 15 outputs takes two and that of one output a longer chain on
-# chip.  300 points, us a call in a row and alone: 10 indices x 2 inputs, 24 entries: 12 and 24 against
-# 19 and 27 (8 outputs), 12 and 22 against 12 and 24 (one); 220 entries x 2 outputs: 15 and 30 against
-# 19 and 34; 300 x 4: 19 and 33 on both.  With many outputs and points the walk falls behind beyond the
-# line: 16 384 points, 72 entries x 15: 38 against 30.  Blocks of a high degree are long serial runs: 40
-# entries of one dim 17 and 32 against 14 and 29.
-SMALL_PLAN = 500
-SMALL_PLAN_DEGREE = 16  # largest degree + 1
 CONTRACT_CHAIN = 256  # terms that the FP64 contraction sums in one workgroup in any case
 MAX_CALL_POINTS = 65535 * 64  # points per call of sbi_contract / _jacobian_f64 / sbi_newton_vjp
 # Newton form of a non-nested interpolant on a nested proxy grid (see _newton_proxy): its largest
@@ -39,6 +30,21 @@ NEWTON_FLOOR = 1e-14  # a Newton form with less rounding than this serves "fp64"
 # "mixed" on the GEMM path (d_out > 1): while sample points are further than this from the FP64
 # path (relative to max |y|), 4x more of the heaviest Newton basis rows move into the FP64 head
 MIXED_TARGET = 2e-7
+# The smallest nested plans keep the walk over blocks in "fp64": one launch, where the Newton form of 2
+# to 15 outputs takes two and that of one output a longer chain on chip.  The walk takes four outputs at
+# a time.  Entries of the plan up to which it does, by outputs: 1: 1000, 2 to 4: 450, more: 500 in all.
+# us a call in a row and alone, the walk against the Newton form: 24 entries x 8 outputs, 300 points: 12
+# and 24 against 19 and 27; 805 x 1: 12 and 25 against 12 and 27; 260 x 2, 16 384 points: 20 and 34
+# against 26 and 42; 400 x 3: 24 and 38 against 26 and 43; beyond the line 805 x 2, 300 points: 23 and
+# 39 against 20 and 38; 206 x 5, 16 384 points: 23 and 39 against 20 and 30; 72 x 15: 38 and 54 against
+# 20 and 28.  Blocks of a high degree are long serial runs: 40 entries of one dim 17 and 32 against 14
+# and 29.
+SMALL_PLAN_DEGREE = 16  # largest degree + 1
+
+
+def _small_plan(k_raw, d_out, dmax1):
+    most = 1000 if d_out == 1 else 450 if d_out <= 4 else 500 // d_out
+    return d_out < GEMM_MIN_DOUT and k_raw <= most and dmax1 <= SMALL_PLAN_DEGREE
 
 
 class SmolyaxPrecisionWarning(UserWarning):
@@ -164,8 +170,7 @@ class SmolyakBarycentricInterpolator:
             self._newton_off = str(e)
         self._fp64_newton = (self._is_nested and self._nplan is not None and self._finite_s
                              and self._newton_is_accurate(values))
-        self._small_plan = (self._d_out < GEMM_MIN_DOUT and L.dmax1 <= SMALL_PLAN_DEGREE
-                            and L.k_raw * max(2, self._d_out) <= SMALL_PLAN)
+        self._small_plan = _small_plan(L.k_raw, self._d_out, L.dmax1)
         if self._is_nested and not self._fp64_newton and 2 <= self._d_out <= packing.SHARE_MAX_OUT:
             self._upload(shares=True)
         self._values = None

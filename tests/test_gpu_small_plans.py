@@ -14,9 +14,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("d,m,d_out,small", [(1, 1, 2, True), (1, 15, 3, True), (1, 40, 1, False),
-                                             (2, 10, 15, True), (2, 40, 2, True), (3, 45, 2, False),
+                                             (2, 10, 15, True), (2, 40, 2, True), (3, 45, 2, True),
                                              (5, 20, 8, True), (40, 80, 1, True), (40, 80, 5, False),
-                                             (2, 10, 16, False)])
+                                             (2, 10, 16, False), (10, 160, 1, True),
+                                             (10, 160, 2, False), (5, 160, 1, False)])
 def test_route_of_small_plans(gpu, d, m, d_out, small):
     from smolyax_amd import nodes as SN
     from smolyax_amd.interpolation import SmolyakBarycentricInterpolator
