@@ -1111,7 +1111,15 @@ int contract_launch(const float* A, int64_t lda, const float* B, int64_t ldb, co
     };
     const double c44 = cost(128, 128, 4.0, 2, 1.4, 0.0), c42 = cost(128, 64, 2.0 / 0.94, 3, 1.6, 2.8),
                  c22 = cost(64, 64, 1.0 / 0.88, 3, 1.7, 2.8);
-    if (c44 <= std::min(c42, c22))
+    // a short K is over before the staged tiles' pipeline pays: where two 64 x 128 tiles per CU cover
+    // the whole result, contract_kernel's direct loads reach 0.79 of that rate (16 384 x 200, K 336 and
+    // 64 head rows: 78 us, a whole evaluation, against 82 to 84 with 2 x 2 fragments and 4 tiles per
+    // CU; K 640: 104 and 106; 9000 x 200, K 336: 72 and 67)
+    const int64_t direct = (int64_t)gm * ((n + 127) / 128);
+    if (K <= 512 && direct > 480 && direct <= 512 && 4.0 / 0.79 < std::min(c44, std::min(c42, c22)))
+      hipLaunchKernelGGL((contract_kernel<4, true>), dim3(gm, (unsigned)((n + 127) / 128)), block, 0, st,
+                         A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64, K64);
+    else if (c44 <= std::min(c42, c22))
       contract_k4_launch<4, 4, 4>(A, lda, B, ldb, offset, Y, ldy, P, n, K, A64, lda64, B64, ldb64,
                                   K64, st);
     else if (c42 <= c22)
