@@ -470,8 +470,9 @@ int sbi_contract_f64_ws(const double* A, int64_t lda, const double* B, int64_t l
  * polynomial as interpolation.py:264-304.  S: surpluses [basis_n, lds] in basis-row order, rows as
  * sbi_contract_f64_ws takes B.  workspace: 256-byte aligned, not shared with a concurrent call, at
  * least *basis_bytes (the basis matrix); with all of sbi_newton_eval_f64_gemm_workspace's result (-1:
- * invalid) a small batch is spread over more workgroups, with the same bits.  At most 65535 * 64
- * points. */
+ * invalid) a small batch is spread over more workgroups, and a plan whose factor table (64 points x
+ * n_tab_rows) exceeds LDS has it written to the workspace once instead of making every factor where it is
+ * needed: the same bits.  At most 65535 * 64 points. */
 int64_t sbi_newton_eval_f64_gemm_workspace(const sbi_newton_plan* plan, int64_t P,
                                            int64_t* basis_bytes);
 int sbi_newton_eval_f64_gemm(const sbi_newton_plan* plan, const double* x, int64_t P, int64_t ldx,

@@ -350,24 +350,104 @@ struct HTab {
   }
 };
 
+// A workgroup makes the rows of 32 dims for 64 points.  The coordinates come through LDS, 32 neighbouring
+// dims of a point per half wave: read by a lane per point they are a line apart (16 384 points x 348 of
+// 1000 dims: 33 us so, 18 here; 131 072 points, x in HBM: 141 us here, and a whole evaluation of 2
+// outputs 731 us instead of 1440).
+constexpr int kHtabDims = 32;
 __global__ __launch_bounds__(256) void newton_htab_kernel(sbi_newton_desc d,
                                                          const double* __restrict__ x, int64_t P,
                                                          int64_t ldx, double* __restrict__ tab,
                                                          int64_t ldt) {
-  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= P) return;
+  __shared__ double xs[kHtabDims][kTile + 1];
+  const int64_t p0 = (int64_t)blockIdx.x * kTile;
+  const int i0 = blockIdx.y * kHtabDims, nd = min(kHtabDims, d.n_tab_dims - i0);
+  const int mine = threadIdx.x & (kHtabDims - 1), q0 = threadIdx.x / kHtabDims;
+  if (mine < nd) {
+    const double* __restrict__ xj = x + d.tab_dim[i0 + mine];
+#pragma unroll
+    for (int q = 0; q < kTile; q += 256 / kHtabDims)
+      xs[mine][q0 + q] = xj[min(p0 + q0 + q, P - 1) * ldx];
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (p0 + lane >= P) return;
   cptr<int32_t> tdim = C(d.tab_dim), trow = C(d.tab_row), tk = C(d.tab_kmax);
   cptr<double> dim_xi = C(d.dim_xi), dim_c = C(d.dim_c);
-  for (int i = blockIdx.y; i < d.n_tab_dims; i += gridDim.y) {
-    const int j = tdim[i], row = trow[i], km = tk[i];
-    const double xj = x[p * ldx + j];
+  double* __restrict__ out = tab + (int64_t)blockIdx.x * ldt * kTile + lane;
+  for (int i = wave; i < nd; i += 4) {
+    const int j = tdim[i0 + i], row = trow[i0 + i], km = tk[i0 + i];
+    const double xj = xs[i][lane];
     cptr<double> xi = dim_xi + (int64_t)j * d.kmax1;
     cptr<double> c = dim_c + (int64_t)j * d.kmax1;
     double pr = 1.0;
     for (int k = 1; k <= km; ++k) {
       pr *= (xj - xi[k - 1]);
-      tab[((p / kTile) * ldt + row + k - 1) * kTile + (p % kTile)] = pr * c[k];
+      out[(int64_t)(row + k - 1) * kTile] = pr * c[k];
     }
+  }
+}
+
+static void htab_launch(const sbi_newton_desc& d, const double* x, int64_t P, int64_t ldx, double* tab,
+                        hipStream_t st) {
+  hipLaunchKernelGGL(newton_htab_kernel,
+                     dim3((unsigned)((P + kTile - 1) / kTile),
+                          (unsigned)((d.n_tab_dims + kHtabDims - 1) / kHtabDims)),
+                     dim3(256), 0, st, d, x, P, ldx, tab, (int64_t)d.n_tab_rows);
+}
+
+// H^T in FP64 like newton_basis_kernel when the tile's factor table does not fit in LDS, from the
+// global table of newton_htab_kernel (the same values and products as newton_basis_direct_kernel,
+// which makes a factor's value again for every node that has it, from coordinates a line apart).
+// A wave takes 64 nodes; the loads of 8 nodes' factors go out together.  The workgroups of a tile of
+// points run one after another on one XCD, whose L2 then holds the tile's table.  Bound by the writes
+// of H^T and the reads of two to three factors per node: 16 384 points x 8982 nodes (1000 inputs) 1110 us
+// factor by factor, 417 here; x 4997 nodes (300 inputs) 480 and 195; 4000 points 302 and 80, 181 and 42.
+constexpr int kBTWaves = 4;
+constexpr int kBTBatch = 8;
+__global__ __launch_bounds__(kTile* kBTWaves) void newton_basis_table_kernel(
+    sbi_newton_desc d, const double* __restrict__ tab, int64_t P, double* __restrict__ HT, int64_t ldh,
+    int tiles, int chunks) {
+  const int idx = blockIdx.x >> 3;
+  const int tile = (idx / chunks) * 8 + (int)(blockIdx.x & 7);
+  if (tile >= tiles) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int base = ((idx % chunks) * kBTWaves + wave) * 64;
+  if (base >= d.basis_n) return;
+  const int cnt = min(64, d.basis_n - base);
+  const int64_t p = (int64_t)tile * kTile + lane;
+  const double* __restrict__ t = tab + (int64_t)tile * d.n_tab_rows * kTile + lane;
+  const uint4 none = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
+  const uint4 dv = lane < cnt ? reinterpret_cast<const uint4*>(d.basis_desc)[base + lane] : none;
+  const uint32_t w[4] = {dv.x, dv.y, dv.z, dv.w};
+  double* __restrict__ out = HT + (int64_t)base * ldh + p;
+  for (int i = 0; i < cnt; i += kBTBatch) {
+    double v[kBTBatch];
+#pragma unroll
+    for (int u = 0; u < kBTBatch; ++u) v[u] = 1.0;
+#pragma unroll
+    for (int f = 0; f < 8; ++f) {  // (rows are packed first: 0xffff after a node's last)
+      double h[kBTBatch];
+      bool any = false;
+#pragma unroll
+      for (int u = 0; u < kBTBatch; ++u) {
+        const uint32_t r =
+            ((uint32_t)__builtin_amdgcn_readlane((int)w[f >> 1], i + u) >> ((f & 1) * 16)) & 0xffff;
+        h[u] = 1.0;
+        if (r != 0xffff) {
+          h[u] = t[(int64_t)r * kTile];
+          any = true;
+        }
+      }
+      if (!any) break;
+#pragma unroll
+      for (int u = 0; u < kBTBatch; ++u) v[u] *= h[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kBTBatch; ++u)
+      if (i + u < cnt && p < P) out[(int64_t)(i + u) * ldh] = v[u];
   }
 }
 
@@ -1124,6 +1204,11 @@ extern "C" int sbi_newton_eval_mixed_gemm(const sbi_newton_plan* plan, const dou
 }
 
 static int64_t f64_basis_ld(int64_t P) { return P + (P & 1); }  // rows on 16 bytes
+// Bytes of the global factor table of newton_basis_table_kernel (0: the tile's table fits LDS)
+static int64_t f64_basis_table(const sbi_newton_desc& d, int64_t P) {
+  if ((size_t)d.n_tab_rows * kTile * sizeof(double) <= (size_t)kMaxLds) return 0;
+  return align256((int64_t)d.n_tab_rows * ((P + kTile - 1) / kTile * kTile) * 8);
+}
 
 extern "C" int64_t sbi_newton_eval_f64_gemm_workspace(const sbi_newton_plan* plan, int64_t P,
                                                       int64_t* basis_bytes) {
@@ -1136,7 +1221,7 @@ extern "C" int64_t sbi_newton_eval_f64_gemm_workspace(const sbi_newton_plan* pla
   if (basis_bytes) *basis_bytes = basis;
   int64_t part = 0;
   if (sbi_contract_f64_workspace(P, dp->d_out, dp->basis_n, &part) != SBI_OK) return -1;
-  return basis + part;
+  return basis + f64_basis_table(*dp, P) + part;
 }
 
 extern "C" int sbi_newton_eval_f64_gemm(const sbi_newton_plan* plan, const double* x, int64_t P,
@@ -1158,10 +1243,30 @@ extern "C" int sbi_newton_eval_f64_gemm(const sbi_newton_plan* plan, const doubl
     return SBI_ERR_INVALID;
   }
   double* HT = (double*)workspace;
-  const int rc = sbi_newton_basis_rows(plan, x, P, ldx, 0, dp->basis_n, HT, ldh, 0, stream);
-  if (rc != SBI_OK) return rc;
+  const int64_t table = f64_basis_table(*dp, P);
+  int64_t used = basis;
+  if (table > 0 && ws_bytes >= basis + table) {
+    const sbi_newton_desc& d = *dp;
+    if (!d.basis_desc || !d.tab_dim) {
+      sbi::set_error("sbi_newton_eval_f64_gemm: plan has no basis tables");
+      return SBI_ERR_INVALID;
+    }
+    hipStream_t st = (hipStream_t)stream;
+    double* tab = (double*)((char*)workspace + basis);
+    htab_launch(d, x, P, ldx, tab, st);
+    SBI_HIP_CHECK(hipGetLastError());
+    const int tiles = (int)((P + kTile - 1) / kTile);
+    const int chunks = (d.basis_n + kTile * kBTWaves - 1) / (kTile * kBTWaves);
+    hipLaunchKernelGGL(newton_basis_table_kernel, dim3((unsigned)((tiles + 7) / 8 * 8 * chunks)),
+                       dim3(kTile * kBTWaves), 0, st, d, tab, P, HT, ldh, tiles, chunks);
+    SBI_HIP_CHECK(hipGetLastError());
+    used += table;
+  } else {
+    const int rc = sbi_newton_basis_rows(plan, x, P, ldx, 0, dp->basis_n, HT, ldh, 0, stream);
+    if (rc != SBI_OK) return rc;
+  }
   return sbi_contract_f64_ws(HT, ldh, S, lds, nullptr, y, ldy, P, dp->d_out, dp->basis_n,
-                             (char*)workspace + basis, ws_bytes - basis, stream);
+                             (char*)workspace + used, ws_bytes - used, stream);
 }
 
 static bool jac_global_table(const sbi_newton_desc& d);
@@ -1230,9 +1335,7 @@ static int vjp_launch(const sbi_newton_desc& d, const double* x, int64_t P, int6
   double* gtab = g ? (double*)workspace : nullptr;
   double* part = (double*)workspace + (g ? (int64_t)d.n_tab_rows * P64 : 0);
   if (g && d.n_tab_dims > 0) {
-    const int64_t ny = std::min<int64_t>(d.n_tab_dims, 64);
-    hipLaunchKernelGGL(newton_htab_kernel, dim3((unsigned)((P + 255) / 256), (unsigned)ny),
-                       dim3(256), 0, st, d, x, P, ldx, gtab, (int64_t)d.n_tab_rows);
+    htab_launch(d, x, P, ldx, gtab, st);
     SBI_HIP_CHECK(hipGetLastError());
   }
   if (d.n_tab_dims < d.d_in) {  // dims without a factor keep 0
@@ -1438,9 +1541,7 @@ static int jacobian_launch(const sbi_newton_plan* plan, const double* x, int64_t
   const int64_t P64 = (P + kTile - 1) / kTile * kTile;
   double* DT = ws + (g ? (int64_t)d.n_tab_rows * P64 : 0);
   if (g && d.n_tab_dims > 0) {
-    const int64_t ny = std::min<int64_t>(d.n_tab_dims, 64);
-    hipLaunchKernelGGL(newton_htab_kernel, dim3((unsigned)((P + 255) / 256), (unsigned)ny),
-                       dim3(256), 0, st, d, x, P, ldx, gtab, (int64_t)d.n_tab_rows);
+    htab_launch(d, x, P, ldx, gtab, st);
     SBI_HIP_CHECK(hipGetLastError());
   }
   if (n <= kJacDirectMax) {

@@ -19,6 +19,7 @@ from .nodes import Generator, Leja1D
 
 PRECISIONS = ("fp64", "mixed", "newton-fp64", "bf16", "bary-fp32")
 GEMM_MIN_DOUT = 16  # from this d_out on, the d_out contraction is one dense GEMM
+LDS_BYTES = 160 * 1024
 CONTRACT_CHAIN = 256  # terms that the FP64 contraction sums in one workgroup in any case
 MAX_CALL_POINTS = 65535 * 64  # points per call of sbi_contract / _jacobian_f64 / sbi_newton_vjp
 # Newton form of a non-nested interpolant on a nested proxy grid (see _newton_proxy): its largest
@@ -687,8 +688,9 @@ class SmolyakBarycentricInterpolator:
 
     def scratch_bytes(self, precision: str, n_points: int) -> int:
         """Bytes of workspace that an FP64 evaluation of n_points takes beside its basis matrix, input
-        and output, to spread a small batch over more workgroups: at most 256 MB, nothing beyond
-        memory_limit; 0 on the other paths."""
+        and output and can do without: to spread a small batch over more workgroups (at most 256 MB),
+        and the global factor table of wide plans; nothing beyond memory_limit, 0 on the other
+        paths."""
         P = int(n_points)
         if precision == "fp64" and self._fp64_newton and not self._small_plan:
             precision = "newton-fp64"
@@ -699,11 +701,30 @@ class SmolyakBarycentricInterpolator:
             return self._within_limit(ws)
         if self._d_out == 1 or (precision == "newton-fp64" and self._nplan is None):
             return 0
-        K = self._layout.k_raw if precision == "fp64" else self._nlayout.basis_n
+        if precision == "newton-fp64":
+            P = min(P, self._point_chunk(self._nlayout.basis_n + self._table_rows(), 8, P))
+            return self._gemm_workspace(P, True)[1]
+        K, nb = self._layout.k_raw, N.c_i64()
         P = min(P, self._point_chunk(K, 8, P))
-        nb = N.c_i64()
         N.check(N.fn["sbi_contract_f64_workspace"](P, self._d_out, K, ctypes.byref(nb)), "contract")
         return self._within_limit(nb.value, K * (P + P % 2) * 8)
+
+    def _gemm_workspace(self, n, scratch):
+        """Bytes of sbi_newton_eval_f64_gemm's workspace for n points: the basis matrix, and what it
+        can do without (scratch, and within memory_limit: all of it, or the factor table alone)."""
+        nb = N.c_i64()
+        ws = N.fn["sbi_newton_eval_f64_gemm_workspace"](self._nplan, n, ctypes.byref(nb))
+        more = ws - nb.value
+        if more and not (scratch and self._within_limit(ws)):
+            table = self._nlayout.n_tab_rows * (-(-n // 64) * 64) * 8 if self._table_rows() else 0
+            more = self._within_limit(-(-table // 256) * 256, nb.value) if scratch else 0
+        return nb.value, more
+
+    def _table_rows(self):
+        """Rows of the global factor table that the FP64 basis matrix is made from where a tile's table
+        (64 points) does not fit LDS; else 0."""
+        rows = self._nlayout.n_tab_rows
+        return rows + 1 if rows * 64 * 8 > LDS_BYTES else 0  # (one more for rounding to 256 bytes)
 
     def _point_chunk(self, rows, itemsize, P):
         """Points per chunk so that the basis matrix stays within memory_limit GiB, and within
@@ -837,14 +858,11 @@ class SmolyakBarycentricInterpolator:
         y = torch.empty((P, self._d_out), dtype=torch.float64, device=self._device)
         if kind == "f64" and not ordered:  # one call per chunk: basis matrix and contraction
             S = self._surpluses("f64", gemm=True)
-            pc = self._point_chunk(Nn, 8, P)
+            pc = self._point_chunk(Nn + self._table_rows(), 8, P)
             for a in range(0, P, pc):
                 xc, yc = (x, y) if pc >= P else (x[a:a + pc], y[a:a + pc])
                 n = yc.shape[0]
-                nb = N.c_i64()
-                ws = N.fn["sbi_newton_eval_f64_gemm_workspace"](self._nplan, n, ctypes.byref(nb))
-                if ws > nb.value and not (scratch and self._within_limit(ws)):
-                    ws = nb.value  # the basis matrix alone
+                ws = sum(self._gemm_workspace(n, scratch))
                 W = torch.empty(ws, dtype=torch.uint8, device=self._device)
                 N.check(N.fn["sbi_newton_eval_f64_gemm"](self._nplan, xc.data_ptr(), n,
                                                          xc.stride(0), S.data_ptr(), self._ld(S),

@@ -26,7 +26,8 @@ def build(d, d_out, m, **kw):
 
 
 @pytest.mark.parametrize("d,d_out,m,P", [(2, 2, 12, 1), (3, 9, 200, 63), (6, 33, 250, 64),
-                                         (10, 15, 900, 130), (40, 16, 1500, 65), (12, 3, 4000, 7)])
+                                         (10, 15, 900, 130), (40, 16, 1500, 65), (12, 3, 4000, 7),
+                                         (400, 2, 1500, 131), (330, 3, 1030, 1), (1000, 17, 2000, 64)])
 def test_one_call_has_the_bits_of_its_parts(gpu, d, d_out, m, P):
     from smolyax_amd import _native as N
 
@@ -55,6 +56,8 @@ def test_one_call_has_the_bits_of_its_parts(gpu, d, d_out, m, P):
         assert torch.equal(y[:, :d_out], want) and torch.isnan(y[:, d_out]).all()
     assert torch.equal(ip.evaluate(x, "newton-fp64"), want)
     assert torch.equal(ip.evaluate(x[P // 2], "newton-fp64")[0], want[P // 2])
+    assert (ip._table_rows() > 0) == (d > 300)  # (wide plans: basis from a table in global memory, or,
+    # with the basis matrix alone and in the chunks below, factor by factor)
     ip._memory_limit = 64 * 8 * n / 1024**3  # chunks of 64 points
     assert torch.equal(ip.evaluate(x, "newton-fp64"), want)
     assert N.fn["sbi_newton_eval_f64_gemm"](ip._nplan, x.data_ptr(), P, ldx, S.data_ptr(), ld,
