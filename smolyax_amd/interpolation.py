@@ -213,7 +213,7 @@ class SmolyakBarycentricInterpolator:
         zero = np.array([g(0)[0] for g in nf.node_gen], dtype=np.float64)
         X = np.stack([nf.grid_point(nu, zero) for nu in nf.nus])
         keep = self._n_inputs
-        Y = self._evaluate(torch.as_tensor(X, device=self._device), "fp64", ordered=True)
+        Y = self.evaluate(torch.as_tensor(X, device=self._device), "fp64", _ordered=True)
         self._n_inputs = keep
         self._set_surpluses(nf, Y)
         return nf
@@ -249,11 +249,11 @@ class SmolyakBarycentricInterpolator:
         # points from the nodes' measure only: far out, the polynomial's own size sets the scale
         X = torch.as_tensor(self._proxy_samples()[: PROXY_SAMPLES // 2], device=self._device)
         keep, warned = self._n_inputs, self._warned_mixed
-        ref = self._evaluate(X, "newton-fp64" if self._newton_fp64_ok else "fp64", ordered=True)
+        ref = self.evaluate(X, "newton-fp64" if self._newton_fp64_ok else "fp64", _ordered=True)
         scale = float(ref.abs().max()) or 1.0
         NL = self._nlayout
         while True:
-            err = float((self._evaluate(X, "mixed") - ref).abs().max()) / scale
+            err = float((self.evaluate(X, "mixed") - ref).abs().max()) / scale
             self._mixed_err = err
             if err <= MIXED_TARGET or NL.n_head >= NL.basis_n:
                 break
@@ -287,7 +287,7 @@ class SmolyakBarycentricInterpolator:
         keep = self._n_inputs
         xt = torch.as_tensor(X, device=self._device)
         scale = np.abs(exact).max(axis=0)
-        err = [float((np.abs(self._evaluate(xt, p).cpu().numpy()[:, cols] - exact).max(axis=0)
+        err = [float((np.abs(self.evaluate(xt, p).cpu().numpy()[:, cols] - exact).max(axis=0)
                       / np.where(scale > 0, scale, 1.0)).max()) for p in ("newton-fp64", "fp64")]
         self._n_inputs = keep
         return err[0] <= max(err[1], NEWTON_FLOOR)
@@ -322,9 +322,9 @@ class SmolyakBarycentricInterpolator:
         Gauss-Hermite ones; at degree ~30 it reaches ~1e-8)."""
         X = torch.as_tensor(self._proxy_samples(), device=self._device)
         keep = self._n_inputs
-        y64 = self._evaluate(X, "fp64", ordered=True)
+        y64 = self.evaluate(X, "fp64", _ordered=True)
         self._newton_fp64_ok = True  # for this measurement only
-        yn = self._evaluate(X, "newton-fp64", ordered=True)
+        yn = self.evaluate(X, "newton-fp64", _ordered=True)
         self._n_inputs = keep
         scale = float(y64.abs().max())
         err = float((yn - y64).abs().max()) / scale if scale > 0 else float((yn - y64).abs().max())
@@ -608,18 +608,17 @@ class SmolyakBarycentricInterpolator:
     # ------------------------------------------------------------------------------ evaluation
     def __call__(self, x) -> torch.Tensor:
         """interpolation.py:264-304: y[P, d_out] (float64 tensor) on the default precision path."""
-        return self._evaluate(x, self._precision)
+        return self.evaluate(x, self._precision)
 
-    def evaluate(self, x, precision: str = None) -> torch.Tensor:
-        """Evaluate on a chosen path (see the constructor's `precision`)."""
-        return self._evaluate(x, precision or self._precision)
+    def evaluate(self, x, precision: str = None, *, _ordered=False, _scratch=True) -> torch.Tensor:
+        """Evaluate on a chosen path (see the constructor's `precision`).
 
-    def _evaluate(self, x, precision, ordered=False, scratch=True):
-        """`evaluate`; ordered: FP64 sums of several outputs block by block (few outputs, unless one
-        share holds all blocks) and in the order of k, which fixes the bits of what set_f derives from
-        them (a proxy's surpluses, which the FP32 rounding of "mixed" makes visible) whatever the
-        fastest split of the sums is.  scratch: small batches may take the workspaces that spread their
-        FP64 sums over more workgroups (scratch_bytes; the same bits without)."""
+        _ordered: FP64 sums of several outputs block by block (few outputs, unless one share holds all
+        blocks) and in the order of k, which fixes the bits of what set_f derives from them (a proxy's
+        surpluses, which the FP32 rounding of "mixed" makes visible) whatever the fastest split of the
+        sums is.  _scratch: small batches may take the workspaces that spread their FP64 sums over more
+        workgroups (scratch_bytes; the same bits without)."""
+        precision = precision or self._precision
         if precision not in PRECISIONS:
             raise ValueError(f"precision must be one of {PRECISIONS}")
         if precision == "mixed" and self._nplan is None:
@@ -627,16 +626,17 @@ class SmolyakBarycentricInterpolator:
                 warnings.warn(f"precision 'mixed': the Newton form is unavailable "
                               f"({self._newton_off}); evaluating with 'bary-fp32' (FP32 "
                               f"barycentric, about 1e-4 relative)", SmolyaxPrecisionWarning,
-                              stacklevel=3)
+                              stacklevel=2)
                 self._warned_mixed = True
             precision = "bary-fp32"
         # On nested nodes the Newton form is the same polynomial with 5 to 7 times fewer terms and
         # without the combination technique's cancellation: from the exact interpolant, max error
         # over max |y|, 3.9e-15 against 1.1e-12 at 1000 inputs x 9999 nodes, 3.3e-14 against 5.7e-12
-        # at 100 inputs x 9986 nodes x 4096 outputs; in one dim, where nothing cancels, both stay
-        # below 1e-14 up to degree 300.  16 384 points x 1000 inputs: 54 us against 132 us;
-        # 5000 points x 160 outputs: 0.45 ms against 3.7 ms.  (Values that are not finite spread to
-        # other nodes' surpluses: such an interpolant keeps the reference's sums.)
+        # at 100 inputs x 9986 nodes x 4096 outputs; in one dim, where nothing cancels, both are near
+        # 1e-15 (_newton_is_accurate: on Leja sequences).  16 384 points x 1000 inputs: 63 us a call
+        # against 143; 5000 points x 160 outputs: 0.37 ms against 4.2.  (Values that are not finite
+        # spread to other nodes' surpluses: such an interpolant keeps the reference's sums; so do the
+        # smallest plans, for speed.)
         if precision == "fp64" and self._fp64_newton and not self._small_plan:
             precision = "newton-fp64"
         if precision == "newton-fp64" and self._nplan is not None and not self._newton_fp64_ok:
@@ -656,9 +656,10 @@ class SmolyakBarycentricInterpolator:
                 or (precision != "fp64" and self._d_out > 1))
         if not gemm:
             y = torch.empty((P, self._d_out), dtype=torch.float64, device=self._device)
-            if precision == "fp64" and self._n_share and not (ordered and self._n_share > 1):
-                ws = N.fn["sbi_bary_eval_few_workspace"](self._plan, P) if scratch else 0
-                ws = self._within_limit(ws)
+            if precision == "fp64" and self._n_share and not (_ordered and self._n_share > 1):
+                ws = 0
+                if _scratch and self._n_share > 1:
+                    ws = self._within_limit(N.fn["sbi_bary_eval_few_workspace"](self._plan, P))
                 W = torch.empty(ws, dtype=torch.uint8, device=self._device) if ws else None
                 N.check(N.fn["sbi_bary_eval_few_f64"](self._plan, x.data_ptr(), P, x.stride(0),
                                                       y.data_ptr(), W.data_ptr() if ws else None,
@@ -667,19 +668,19 @@ class SmolyakBarycentricInterpolator:
                 rc = N.fn["sbi_bary_eval_f64"](self._plan, x.data_ptr(), P, x.stride(0),
                                                y.data_ptr(), self._stream())
                 if rc == N.SBI_ERR_CAPACITY:  # prefix table too large for LDS: GEMM form
-                    return self._eval_bary_gemm(x, ordered=ordered, scratch=scratch)
+                    return self._eval_bary_gemm(x, ordered=_ordered, scratch=_scratch)
                 N.check(rc, "eval")
             else:
                 fn = "sbi_newton_eval_mixed" if precision == "mixed" else "sbi_newton_eval_f64"
                 rc = N.fn[fn](self._nplan, x.data_ptr(), P, x.stride(0), y.data_ptr(),
                               self._stream())
                 if rc == N.SBI_ERR_CAPACITY:  # internal-node table beyond LDS: GEMM form
-                    return self._eval_newton_gemm(x, precision, ordered, scratch)
+                    return self._eval_newton_gemm(x, precision, _ordered, _scratch)
                 N.check(rc, precision)
             return y
         if precision == "fp64":
-            return self._eval_bary_gemm(x, ordered=ordered, scratch=scratch)
-        return self._eval_newton_gemm(x, precision, ordered, scratch)
+            return self._eval_bary_gemm(x, ordered=_ordered, scratch=_scratch)
+        return self._eval_newton_gemm(x, precision, _ordered, _scratch)
 
     def _within_limit(self, ws, held=0):
         """ws, the bytes of a workspace that a call can do without, or 0 where memory_limit has no

@@ -278,7 +278,7 @@ class Server:
                     xs = x_st
                 else:
                     xs = torch.cat(xin) if len(xin) > 1 else xin[0]
-                    y = ip._evaluate(xs, self.precision, scratch=scratch)
+                    y = ip.evaluate(xs, self.precision, _scratch=scratch)
                 a = 0
                 for r, a0, n in pieces:
                     if a0 == 0 and n == r.x.shape[0]:
