@@ -863,7 +863,14 @@ __global__ __launch_bounds__(256) void jac_reduce_kernel(sbi_newton_desc d,
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc += v[i];
     }
-    for (; u < ns; ++u) acc += part[((int64_t)(s0 + u) * P + p) * n + o];
+    for (; u < ns; u += 4) {  // the rest four by four
+      double v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = part[((int64_t)(s0 + min(u + i, ns - 1)) * P + p) * n + o];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (u + i < ns) acc += v[i];
+    }
     J[(p * n + o) * d.d_in + j] = nan_here ? NAN : acc;
   }
 }
