@@ -321,9 +321,10 @@ typedef struct sbi_newton_desc {
                                  none), or a part of its rows (slot 0 .. n_jac_slots - 1) */
   const int32_t* jac_group_red; /* [3 * n_jac_group_red] {first dim, first slot, slots} of the
                                  groups in several parts */
-  /* register pass of the Jacobian (d_out <= 8) and the adjoint with the factor table in LDS
-   * (optional: n_jt_blocks = 0 selects the pass over jac_unit).  A unit is a run of at most 64
-   * entries of one factor row; 16 units of about one length, the longest first, are a block, whose
+  /* register pass of the Jacobian (n <= 8) with the factor table in LDS (optional: n_jt_blocks = 0
+   * leaves it to the pass over jac_unit, which also takes n > 4 with a table of at most half of LDS,
+   * small plans without split dims, and the adjoint).  A unit is a run of at most 64 entries of one
+   * factor row; 16 units of about one length, the longest first, are a block, whose
    * records lie step by step; a dim of several units adds their sums in slot order */
   int32_t n_jt_blocks;
   int32_t n_jt_slots;

@@ -3,8 +3,7 @@
 // Newton form (nested nodes): y[p, :] = sum_nu H[p, nu] S[nu, :] with
 //   H[p, nu] = prod_{(j,k) in nu} h^{(j)}_k(x_{p,j})     (H[p, root] = 1).
 // newton_basis_kernel writes H^T (nodes x points, points contiguous) so that the d_out
-// contraction Y = H S is one dense GEMM (done by the caller's BLAS on MFMA in FP64, FP32 or
-// BF16 with FP32 accumulation).
+// contraction Y = H S is one dense product on the matrix cores (gemm.hip; FP64, FP32 or BF16).
 //
 // Adjoint (vector-Jacobian product) of the same form: with G = V S^T (a GEMM, V = dL/dy),
 //   dL/dx_{p,j} = sum_k h'^{(j)}_k(x_{p,j}) A[p, (j,k)],
@@ -15,7 +14,7 @@
 //
 // Barycentric form (the reference's algorithm): bary_basis_kernel writes the per-entry weights
 // W^T[e, p] = prod_i Lhat_i(x_{p, s_i})[mu_i] of every block entry e (K_raw rows) so that
-// y = offset + W F (zeta folded into F) is a dense FP64 GEMM.
+// y = offset + W F (zeta folded into F) is a dense product (gemm.hip).
 //
 // Tile = 64 points, one per lane; the 1D factors h_k(x_j) of the tile live in an LDS table.
 
@@ -628,8 +627,8 @@ __global__ __launch_bounds__(kTile* kBWaves) void newton_jac_kernel(
 // factor from L2.  Records lie step by step (one 256-byte read per step, no address arithmetic); a
 // step's coefficients are requested one step (of U entries) ahead, its records two.  Bound by LDS
 // reads and VALU issue.
-// 4096 points x 1000 inputs, 22 097 entries: 66 us and 7 us for the reduction, against 118 + 26 us
-// for the factor table in global memory and 9.5 us.  (8 lanes per unit: 103 us; units one after
+// 4096 points x 1000 inputs, 22 097 entries: 72 us a call, one after another (73 us and 7 for the
+// reduction in a kernel trace), against 118 + 26 us for the factor table in global memory and 9.5 us.  (8 lanes per unit: 103 us; units one after
 // another, 8 lanes by entry: 251 us, a chain of loads per unit.)  The adjoint keeps the pass above:
 // its 2.3 reads of G per node bound it (220 us here against 199 + 16 us; 8192 points x 200 inputs).
 // ------------------------------------------------------------------------------------------

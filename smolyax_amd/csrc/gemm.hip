@@ -1333,9 +1333,9 @@ contract_bf16_wide_kernel(SBI_BF16_ARGS) {
 // rows: the first dims of an index set hold most of them (the first 8 of 200: 5594 of 11 506), so
 // the host cuts such a group into parts, which jac_group_reduce_kernel adds in order.  Bound: the
 // FP64 matrix cores (75 us at 999 points x 256 outputs x 200 dims) and, for the many short groups,
-// the latency of a job's start; measured there 277 us + 28 us for the parts (466 us with masked
-// chunks across dims, each wave loading from L2 and every lane writing its own 64 bytes; without
-// the writes of J 223 us).  (Groups with few rows joined into longer jobs were slower, 542 us: a wave's stores of a finished group hold
+// the latency of a job's start; measured there 268 us + 27 us for the parts (466 us with masked
+// chunks across dims, each wave loading from L2 and every lane writing its own 64 bytes).  (Groups
+// with few rows joined into longer jobs were slower, 542 us: a wave's stores of a finished group hold
 // up its next loads, which complete in order behind them.)
 //
 // Operands are staged in LDS in chunks of 32 rows, three buffers, copied two chunks ahead by direct
